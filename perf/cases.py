@@ -279,6 +279,113 @@ def run(state):
 
 
 # ------------------------------------------------------------------------------------------------
+# The same in 64 bits
+# ------------------------------------------------------------------------------------------------
+def _product64(rowptr, col, value, rows, onto=None):
+    """sum of value[e] * rows(col[e]) over every row's edges, in slabs of rows that hold about 2 GB of products;
+    ``rows`` gives the dense operand's rows of an index vector in float64."""
+    counts = rowptr[1:] - rowptr[:-1]
+    ends, n = rowptr.cpu(), counts.numel()
+    F = rows(col[:1].to(torch.int64)).shape[1]
+    out = torch.zeros(n, F, dtype=torch.float64, device=col.device) if onto is None else onto.double()
+    first = 0
+    while first < n:
+        last = int(torch.searchsorted(ends, ends[first] + 256_000_000 // F, right=True)) - 1
+        last = min(n, max(last, first + 1))
+        a, b = int(ends[first]), int(ends[last])
+        terms = rows(col[a:b].to(torch.int64)).mul_(value[a:b].double()[:, None])
+        out[first:last] += torch.segment_reduce(terms, "sum", lengths=counts[first:last], unsafe=True)
+        first = last
+    return out
+
+
+def _transposed(rowptr, col, value, columns):
+    row = torch.repeat_interleave(torch.arange(rowptr.numel() - 1, device=col.device), rowptr[1:] - rowptr[:-1])
+    order = torch.argsort(col, stable=True)
+    ends = torch.zeros(columns + 1, dtype=torch.int64, device=col.device)
+    ends[1:] = torch.bincount(col.to(torch.int64), minlength=columns).cumsum(0)
+    return ends, row[order], value[order]
+
+
+def _decoded(state, bits, wanted):
+    """Rows ``wanted`` of the packed block: code * scale + zero_point."""
+    per_byte = 8 // bits
+    ends = state["work_range"].to(torch.int64)
+    sizes = ends[1:] - ends[:-1]
+    packed = torch.zeros_like(ends)
+    packed[1:] = ((sizes + per_byte - 1) // per_byte).cumsum(0)
+    ends, packed = ends.to(wanted.device), packed.to(wanted.device)
+    segment = torch.searchsorted(ends, wanted, right=True) - 1
+    inside = wanted - ends[segment]
+    shift = (per_byte - 1 - inside % per_byte) * bits
+    code = (state["data"][packed[segment] + inside // per_byte].to(torch.int64) >> shift[:, None]) & (2 ** bits - 1)
+    params = state["params"].double()[wanted]
+    return code.double() * params[:, 1:] + params[:, :1]
+
+
+def _train64(case, seed):
+    """The step with fp32 exchange: mean aggregation, two products, dropout, LayerNorm, rectifier."""
+    rowptr, col, _ = _graph(case, seed)
+    ones = torch.ones(col.numel(), device=DEVICE)
+    there, back = (rowptr, col, ones), _transposed(rowptr, col, ones, case["nodes"])
+    degree = (rowptr[1:] - rowptr[:-1]).clamp(min=1).double()[:, None]
+    state = _prepare_train(case, seed)
+    model, x = state["model"].double(), state["x"].double()
+    torch.manual_seed(seed)
+
+    class Aggregate(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, v):
+            return _product64(*there, lambda i: v[i])
+
+        @staticmethod
+        def backward(ctx, g):
+            return _product64(*back, lambda i: g[i])
+
+    for i, conv in enumerate(model.convs):
+        x = (Aggregate.apply(x) / degree) @ conv.lin_neigh.weight.t() + x @ conv.lin_self.weight.t() + conv.bias
+        if i + 1 < len(model.convs):
+            x = x * torch.nn.functional.dropout(torch.ones(x.shape, device=DEVICE), p=model.dropout)
+            x = torch.relu(model.norms[i](x))
+    out = torch.log_softmax(x, 1)
+    loss = -out.gather(1, state["labels"]).mean()
+    loss.backward()
+    return {"log_probabilities": out.detach(), "loss": loss.detach(), "gradients": [p.grad for p in model.parameters()]}
+
+
+def exact(case, seed):
+    op, seed = case["op"], int(seed)
+    if op == "spmm":
+        rowptr, col, value = _graph(case, seed)
+        if case["backward"]:
+            rowptr, col, value = _transposed(rowptr, col, value, case["nodes"])
+        x = torch.randn(case["nodes"], case["F"], generator=_generator(seed + 1), device=DEVICE)
+        return _product64(rowptr, col, value, lambda i: x[i].double())   # out is zero before the first pass
+    if op == "quantize":   # the packed codes are whole numbers
+        state = _prepare_quantize(case, seed)
+        x = state["x"] if state["row_index"] is None else state["x"][state["row_index"]]
+        low = x.amin(1).double()
+        scale = (x.amax(1).double() - low) / (2 ** case["bits"] - 1)
+        return None, torch.stack([low, torch.where(scale == 0, 1.0, scale)], 1)
+    if op == "dequantize":
+        state = _prepare_dequantize(case, seed)
+        return _decoded(state, case["bits"], torch.arange(case["rows"], device=DEVICE))
+    if op == "fused":
+        state = _prepare_fused(case, seed)
+        rowptr, col, value = state["matrix"].csr()
+        return _product64(rowptr, col, value, lambda i: _decoded(state, case["bits"], i), onto=state["out"])
+    if case["bits"] != 32:   # codes that follow from computed rows: a step of one is far more than any rounding
+        return None
+    if op == "train":
+        return _train64(case, seed)
+    rowptr, col, value = _graph(case, seed)
+    state = _prepare_aggregate(case, seed)
+    x, grad = state["x"].detach(), state["grad"]
+    return (_product64(rowptr, col, value, lambda i: x[i].double()),
+            _product64(*_transposed(rowptr, col, value, case["nodes"]), lambda i: grad[i].double()))
+
+
+# ------------------------------------------------------------------------------------------------
 # Bounds
 # ------------------------------------------------------------------------------------------------
 def _edges(case):
