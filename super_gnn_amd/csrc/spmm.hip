@@ -198,17 +198,32 @@ __device__ __forceinline__ uint32_t group_ballot(bool pred) {
 // Rows per chunk: each of the first nr+1 lanes of the group holds one rowptr entry.
 __host__ __device__ constexpr int chunk_row_limit(int G) { return (G < 32 ? G : 32) - 1; }
 
+// Gathers in flight per lane group of the short-row kernel.  Deep: the whole grid is resident at once and its time is the
+// longest chunk's chain of gathers, one memory latency per U of them.  Otherwise many rounds of waves follow each other, and
+// what counts is the bytes a CU has in flight: lines on their way occupy the XCD's 4 MB L2, and beyond about 64 KB per CU
+// they push out rows that others are about to use (uniform columns, F = 128: 30 k rows x 61 edges U = 1 / 2 / 4 / 8 52 / 55 /
+// 88 / 89 us, 100 k rows x 41 edges 245 / 270 / 280 / 281).  So about 2 KB per wave of 64 lanes.  Packed rows are 4 ... 16
+// times smaller.
+__host__ __device__ constexpr int short_unroll(int G, int NV, int bits, bool deep) {
+    if (NV > 1) return unroll_of(NV);
+    if (bits != 0) return G == 64 ? 8 : 4;
+    if (deep) return 8;
+    return G == 8 ? 8 : G == 16 ? 3 : G == 32 ? 2 : 6;
+}
+// Rows of 512 ... 1024 bytes keep every gather under its lane predicate: each then sits in an exec-mask region of its own
+// with a wait before it, i.e. one row in flight per wave, which is as much as the L2 bears (U = 1 without the predicate: 30 k
+// rows x 61 edges of F = 256 141 -> 152 us, 100 k x 41 535 -> 550).
+__host__ __device__ constexpr bool short_fenced(int G, int NV, int bits, bool deep) { return G == 64 && NV == 1 && bits == 0 && !deep; }
+
 // One lane group walks one chunk of consecutive rows for the feature columns [f_lo, f_hi) (both multiples
 // of VEC).  RP is the row-pointer type: the caller's int64 array, or the 32-bit per-band row pointers of a
 // band schedule.
-template <int VEC, int G, int NV, int BITS, typename RP, int UF = 0>
+template <int VEC, int G, int NV, int BITS, typename RP, int U, bool FENCED>
 __device__ __forceinline__ void short_chunk_body(
     const RP *__restrict__ rowptr, const int32_t *__restrict__ col, const float *__restrict__ val,
     const DenseSrc &dense, float *__restrict__ out, int4 ch, int f_lo, int f_hi,
     int64_t ldo, int accumulate, const float *__restrict__ row_div, int lig) {
     constexpr int TILE = G * VEC * NV;
-    // gathers in flight per lane group: 6 keeps the kernel at 75 VGPRs (6 waves per SIMD); 8 costs 83 (5 waves)
-    constexpr int U = UF > 0 ? UF : NV == 1 ? 6 : unroll_of(NV);
     const int F = f_hi;
     if constexpr (G == 64) {
         ch.x = __builtin_amdgcn_readfirstlane(ch.x);
@@ -238,13 +253,18 @@ __device__ __forceinline__ void short_chunk_body(
     const float mydiv = (row_div && lig < nr) ? row_div[rb + lig] : 1.0f;
 
     for (int f0 = f_lo; f0 < F; f0 += TILE) {
-        int off[NV];
-        bool act[NV];
+        // Lanes past the end of the row load the tile's first vector again (a cache hit) and never store: a gather under
+        // a lane predicate sits in an exec-mask region of its own with a wait for everything before it, which left ONE
+        // gather in flight (FENCED; 200 k power-law nodes, 4 M edges, F = 100: 148 -> 98 us).
+        int off[NV], off_ld[NV];
+        bool act[NV], act_ld[NV];
         float acc[NV][VEC], nxt_old[NV][VEC];
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             off[v] = f0 + (v * G + lig) * VEC;
             act[v] = off[v] < F;
+            off_ld[v] = act[v] ? off[v] : f0;
+            act_ld[v] = FENCED ? act[v] : true;
         }
         int cur = __builtin_ctz(mask);
         int cur_end = group_bcast_i<G>(rel, cur + 1);
@@ -289,7 +309,7 @@ __device__ __forceinline__ void short_chunk_body(
                     const int src = j + u < cnt ? j + u : cnt - 1;
                     int es = -1;
                     if constexpr ((BITS & kEdgeSlots) != 0) es = group_bcast_i<G>(mys, src);
-                    fetch_row<VEC, NV, BITS>(xv[u], dense, group_bcast_i<G>(myc, src), es, off, act);
+                    fetch_row<VEC, NV, BITS>(xv[u], dense, group_bcast_i<G>(myc, src), es, off_ld, act_ld);
                 }
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
@@ -336,7 +356,7 @@ __device__ __forceinline__ void short_chunk_body(
     }
 }
 
-template <int VEC, int G, int NV, int BITS>
+template <int VEC, int G, int NV, int BITS, bool DEEP>
 __global__ __launch_bounds__(kBlock) void spmm_short_kernel(
     const int64_t *__restrict__ rowptr, const int32_t *__restrict__ col, const float *__restrict__ val,
     const DenseSrc dense, float *__restrict__ out, const int4 *__restrict__ chunks, int n_chunks, int F,
@@ -348,7 +368,8 @@ __global__ __launch_bounds__(kBlock) void spmm_short_kernel(
     if (ci >= n_chunks) return;
     // A chunk record is (first row, row count, first edge, edge count): the column/weight loads
     // depend on it alone and are issued before the row pointers come back.
-    short_chunk_body<VEC, G, NV, BITS, int64_t>(rowptr, col, val, dense, out, chunks[ci], 0, F, ldo, accumulate, row_div, lig);
+    short_chunk_body<VEC, G, NV, BITS, int64_t, short_unroll(G, NV, BITS, DEEP), short_fenced(G, NV, BITS, DEEP)>(
+        rowptr, col, val, dense, out, chunks[ci], 0, F, ldo, accumulate, row_div, lig);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1090,6 +1111,7 @@ struct ShortArgs {
     const int4 *chunks; int n_chunks; const int32_t *empty_rows; int n_empty;
     int F; int64_t ldo; int accumulate; const float *row_div;
     bool prof;   // false: no profiling events (the non-allocating entry point creates nothing)
+    int64_t x_bytes;  // the dense operand
 };
 struct PieceArgs {
     const int32_t *col_long; const int32_t *eperm; const float *val; float *partial;
@@ -1100,6 +1122,17 @@ struct FinalArgs {
     const int32_t *long_rows; const int32_t *long_pbeg; const float *partial; float *out; int n_long;
     int F; int64_t ldo; int accumulate; const float *row_div;
 };
+
+// Chunks that the chip holds at once, about: up to here the short-row kernel keeps the larger number of gathers in flight.
+constexpr int kDeepChunks = kChunkGroupsWanted;
+
+// Unused LDS that a workgroup of the short-row kernel asks for so that four of them fit a CU: a dense operand beyond the
+// 256 MB Infinity Cache is gathered from HBM, and there 32 KB in flight per CU are enough; more only lowers the L2's hit rate
+// (62 M-edge power-law graph, F = 128, U = 2: 3.37 -> 3.09 ms; 1 M uniform columns x 17 edges 1.30 -> 1.24 ms, F = 64 0.69 ->
+// 0.66; 80 MB operand: 0.20 -> 0.24 ms, so not there).
+static uint32_t short_spare_lds(int bits, int G, int NV, int64_t x_bytes) {
+    return bits == 0 && NV == 1 && (G == 16 || G == 32) && x_bytes > (256ll << 20) ? 40000 : 0;
+}
 
 template <int VEC, int G, int NV, int BITS>
 static void launch_all(const ShortArgs &a, const PieceArgs &s, const FinalArgs &f, hipStream_t st) {
@@ -1133,8 +1166,13 @@ static void launch_all(const ShortArgs &a, const PieceArgs &s, const FinalArgs &
     if (a.n_chunks > 0) {
         const uint32_t nb = (uint32_t)((a.n_chunks + GPB - 1) / GPB);
         ProfScope prof(BITS == 0 ? K_SPMM_SHORT : K_FUSED_SHORT, st, a.prof);
-        hipLaunchKernelGGL((spmm_short_kernel<VEC, G, NV, BITS>), dim3(nb), dim3(kBlock), 0, st, a.rowptr, a.col, a.val,
-                           a.dense, a.out, a.chunks, a.n_chunks, a.F, a.ldo, a.accumulate, a.row_div, nb);
+        constexpr bool kHasDeep = short_unroll(G, NV, BITS, true) != short_unroll(G, NV, BITS, false);
+        if (kHasDeep && a.n_chunks <= kDeepChunks)
+            hipLaunchKernelGGL((spmm_short_kernel<VEC, G, NV, BITS, kHasDeep>), dim3(nb), dim3(kBlock), 0, st, a.rowptr, a.col,
+                               a.val, a.dense, a.out, a.chunks, a.n_chunks, a.F, a.ldo, a.accumulate, a.row_div, nb);
+        else
+            hipLaunchKernelGGL((spmm_short_kernel<VEC, G, NV, BITS, false>), dim3(nb), dim3(kBlock), short_spare_lds(BITS, G, NV, a.x_bytes),
+                               st, a.rowptr, a.col, a.val, a.dense, a.out, a.chunks, a.n_chunks, a.F, a.ldo, a.accumulate, a.row_div, nb);
     }
     if (a.n_empty > 0 && (!a.accumulate || a.row_div)) {
         const uint32_t nb = (uint32_t)((a.n_empty + GPB * kEmptyRowsPerGroup - 1) / (GPB * kEmptyRowsPerGroup));
@@ -2185,7 +2223,8 @@ static int spmm_run(sgnn_spmm_plan *p, const float *val, const DenseSrc &dense, 
     const int which = gw == 8 ? 0 : gw == 16 ? 1 : 2;
     SGNN_REQUIRE(p->n_chunks[which] >= 0, "plan has no chunk list for this feature width (plan creation failed?)");
     ShortArgs a{p->rowptr, p->col, val, dense, out, p->chunks[which], (int)p->n_chunks[which], p->empty_rows,
-                (int)p->n_empty, (int)F, ldo, accumulate, row_div, scratch == nullptr};
+                (int)p->n_empty, (int)F, ldo, accumulate, row_div, scratch == nullptr,
+                bits == 0 ? p->K * F * 4 : p->K * F * bits / 8};
     PieceArgs s{p->col_long, p->eperm, val, partial, p->cls_work, p->max_cls_items, (int)F};
     if (val != nullptr && val == p->bound_val && p->val_long != nullptr) {
         s.eperm = nullptr;   // values already sit in regrouped order: contiguous reads, no indirection
