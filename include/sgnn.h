@@ -73,6 +73,14 @@ int sgnn_spmm_plan_create(const int64_t *rowptr, const void *col, int col_is_i64
 
 int sgnn_spmm_plan_destroy(sgnn_spmm_plan *plan);
 
+/* One plan for the block-diagonal matrix of n_parts plans: rows, columns and edges of the parts one after the
+ * other, so that P small products become one call.  The parts' index arrays are copied (the parts may be
+ * destroyed).  A row gets the sum, bit for bit, that its own plan's row-class schedule gives it; the stacked plan
+ * never takes the band schedule.  Edge values are those of the parts, concatenated.  Refused (SGNN_ERR_ARG): parts
+ * that are held as row blocks, or themselves stacked, or whose edges together do not fit one plan.
+ * Synchronises the stream. */
+int sgnn_spmm_plan_stack(sgnn_spmm_plan *const *parts, int n_parts, sgnn_stream_t stream, sgnn_spmm_plan **plan_out);
+
 /* info[0]=M, [1]=K, [2]=nnz, [3]=#long rows, [4]=#pieces, [5]=edges in long rows,
  * [6]=long_row_threshold, [7]=piece_edges, [8]=1 if the long rows were regrouped by column class,
  * [9]=share of all edges that point at the 16384 most popular columns, in parts per million (0 when

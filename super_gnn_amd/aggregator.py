@@ -27,6 +27,7 @@ Because the partitions share one process, every partition's buffers are slices o
 buffer kind, and the exchange is ONE row-permuting copy per buffer (send rows of all ranks -> recv
 rows of all ranks).  The send-side chain and the local SpMMs are issued on two streams.
 """
+import os
 from typing import List, Sequence
 
 import torch
@@ -34,6 +35,7 @@ import torch
 from .ops.spmm_kernel import (SPMM_backward, SPMM_backward_quantized, SPMM_forward, SPMM_forward_quantized)
 from .quantizer import Quantizer_for_all_procs
 from .sparse import SparseTensor
+from .supergnn_ops import SpmmPlan, dequantize_tensor_for_all_procs, quant_segments, quantize_tensor_for_all_procs
 
 
 def _cumulative(splits):
@@ -260,6 +262,174 @@ def _world_backward(world, grads, bits, out_all=None):
     return outs
 
 
+# Up to this many edges (local, send and receive side) the partitions' matrices are also kept stacked as one, which
+# costs a second plan (about 12 bytes per edge and direction).  Beyond it a partition fills the chip by itself.
+_STACKED_EDGES = 1 << 25
+_BAND_SWITCHES = ("SGNN_SPMM_BAND", "SGNN_SPMM_BAND_COLS", "SGNN_SPMM_BAND_KB", "SGNN_SPMM_BAND_SLICES", "SGNN_SPMM_BAND_WINDOW")
+
+
+class _Product(object):
+    """The block-diagonal matrix of the partitions' matrices (or of their transposes): its plan and its edge values."""
+
+    def __init__(self, mats, transposed):
+        self.plans = [m.spmm_plan_T() if transposed else m.spmm_plan() for m in mats]
+        self.plan = SpmmPlan.stack(self.plans)
+        self.value = torch.cat([m.storage.value_T() if transposed else m.csr()[2] for m in mats])
+        self._bands = {}
+
+    def takes_bands(self, F):
+        """Whether one of the partitions' own fp32 products would take the band schedule."""
+        key = (F,) + tuple(os.environ.get(k) for k in _BAND_SWITCHES)
+        if key not in self._bands:
+            if len(self._bands) > 16:
+                self._bands.clear()
+            self._bands[key] = any(p.schedule(F)["band"] for p in self.plans)
+        return self._bands[key]
+
+    def run(self, x, out, accumulate):
+        self.plan.run(self.value, x, out, accumulate=accumulate)
+
+    def run_quantized(self, data, params, segs, bits, out):
+        self.plan.run_quantized(self.value, data, params, segs, bits, out)
+
+
+class _Stacked(object):
+    """The partitions of a world as ONE block-diagonal matrix per role, over the node features stacked in partition order
+    and the arenas' rows.  A partition of a graph of this size is 10 ... 40 us of work per product, most of it the latency of
+    the longest row and of the launches, P times in a row; stacked, the P products are one launch sequence that fills the
+    chip (eight partitions of 25 k nodes, int2, forward and backward: 2.02 -> 0.75 ms; two of 100 k: 1.18 -> 1.01).  The rows
+    get the sums that the partitions' own products give them."""
+
+    def __init__(self, world, signature):
+        self.world, self.signature, self.products = world, signature, {}
+        graphs = world.graphs
+        self.index = None
+        if not world.is_pre_delay:
+            self.index = torch.cat([g.idx_nodes_send_to_others + n0 for g, n0 in zip(graphs, world.node_offsets)])
+        # The partitions' segments one after the other: the packed rows then lie where the partitions' own calls put them.
+        self.send_range = torch.tensor(_cumulative([k for g in graphs for k in g.comm_splits.send_splits]), dtype=torch.int32)
+        self.recv_range = torch.tensor(_cumulative([k for g in graphs for k in g.comm_splits.recv_splits]), dtype=torch.int32)
+        self.segments = len(graphs) ** 2
+
+    def product(self, role, transposed=False):
+        p = self.products.get((role, transposed))
+        if p is None:
+            graphs, pre = self.world.graphs, self.world.is_pre_delay
+            if role == "local":
+                mats = [g.local_adj_t for g in graphs]
+            elif role == "remote":
+                mats = [g.adj_t_pre_post_aggr_from if pre else g.remote_adj_t for g in graphs]
+            else:
+                mats = [g.adj_t_pre_post_aggr_to if pre else _scatter_matrix(g, g.local_adj_t.sparse_size(0)) for g in graphs]
+            p = self.products[(role, transposed)] = _Product(mats, transposed)
+        return p
+
+    def same_schedule(self, F, fused, backward):
+        """False where a partition's own product would run as column bands, which a stacked plan does not have."""
+        roles = [("local", backward)]
+        if self.index is None or backward:
+            if not (backward and fused):
+                roles.append(("to", backward and self.index is None))
+        if backward or not fused:
+            roles.append(("remote", backward))
+        return not any(self.product(*r).takes_bands(F) for r in roles)
+
+    @staticmethod
+    def of(world, x, bits, backward=False):
+        """The world's stacked matrices, or None where the partitions run one by one.  They are rebuilt when a partition's
+        matrices, or the tensors in them, are replaced or edited in place."""
+        graphs, pre = world.graphs, world.is_pre_delay
+        if len(graphs) == 1 or not x.is_cuda:
+            return None
+        if x.shape[-1] > 256 and not (bits in (2, 4, 8) and x.shape[-1] % 2 == 0):
+            return None   # spmm() decides matrix by matrix whether such a width overwrites (reference_overwrites)
+        parts, used = [], []
+        for g in graphs:
+            mats = (g.local_adj_t, g.adj_t_pre_post_aggr_from, g.adj_t_pre_post_aggr_to) if pre else (g.local_adj_t, g.remote_adj_t)
+            for m in mats:
+                parts.extend(m.csr())
+                used.append(m)
+            if not pre:
+                parts.append(g.idx_nodes_send_to_others)
+        if any(t is None or t.device != x.device for t in parts):
+            return None
+        signature = [(t, t._version) for t in parts]
+        have = world._stacked
+        if have is None or len(have.signature) != len(signature) or any(
+                a[0] is not b[0] or a[1] != b[1] for a, b in zip(have.signature, signature)):
+            edges = sum(t.numel() for t in parts if t.dtype == torch.float32)
+            fits = edges <= _STACKED_EDGES and all(t.dtype in (torch.int64, torch.int32, torch.float32) for t in parts)
+            have = world._stacked = _Stacked(world, signature) if fits and "SGNN_SPMM_PART_EDGES" not in os.environ else None
+        fused = bits in (2, 4, 8) and x.shape[-1] % 2 == 0
+        if have is not None and not have.same_schedule(x.shape[-1], fused, backward):
+            return None
+        if have is not None:
+            for m in used:
+                m.note_use(x.shape[-1], backward)
+        return have
+
+
+def _stacked_forward(world, stacked, x, bits, out):
+    quantized = bits in (2, 4, 8)
+    arena = world.arena(x.shape[-1], x.device, bits)
+    fused = quantized and x.shape[-1] % 2 == 0
+    if quantized:
+        Quantizer_for_all_procs(len(world.graphs), bits)   # the process-wide instance the partitions' own calls would leave
+    rows = arena.send.shape[0]
+    main = torch.cuda.current_stream()
+    side = world.side_stream(x.device)
+    side.wait_stream(main)
+    with torch.cuda.stream(side):
+        if rows:
+            if stacked.index is None:
+                stacked.product("to").run(x, arena.send, False)
+            elif not quantized:
+                torch.index_select(x, 0, stacked.index, out=arena.send)
+            if quantized:
+                quantize_tensor_for_all_procs(x if stacked.index is not None else arena.send, arena.send_q, arena.send_params,
+                                              stacked.send_range, stacked.segments, bits, row_index=stacked.index)
+            arena.exchange("forward", quantized)
+    stacked.product("local").run(x, out, False)
+    main.wait_stream(side)
+    if not rows:
+        return
+    if fused:
+        stacked.product("remote").run_quantized(arena.recv_q, arena.recv_params, quant_segments(stacked.recv_range, bits), bits, out)
+    else:
+        if quantized:
+            dequantize_tensor_for_all_procs(arena.recv_q, arena.recv, arena.recv_params, stacked.recv_range, stacked.segments, bits)
+        stacked.product("remote").run(arena.recv, out, True)
+
+
+def _stacked_backward(world, stacked, grad, bits, out):
+    quantized = bits in (2, 4, 8)
+    arena = world.arena(grad.shape[-1], grad.device, bits)
+    fused = quantized and grad.shape[-1] % 2 == 0
+    if quantized:
+        Quantizer_for_all_procs(len(world.graphs), bits)
+    rows = arena.recv.shape[0]
+    main = torch.cuda.current_stream()
+    side = world.side_stream(grad.device)
+    side.wait_stream(main)
+    with torch.cuda.stream(side):
+        if rows:
+            stacked.product("remote", True).run(grad, arena.recv, False)
+            if quantized:
+                quantize_tensor_for_all_procs(arena.recv, arena.recv_q, arena.recv_params, stacked.recv_range, stacked.segments, bits)
+            arena.exchange("backward", quantized)
+    stacked.product("local", True).run(grad, out, False)
+    main.wait_stream(side)
+    if not rows:
+        return
+    if quantized and not fused:
+        dequantize_tensor_for_all_procs(arena.send_q, arena.send, arena.send_params, stacked.send_range, stacked.segments, bits)
+    back = stacked.product("to", stacked.index is None)
+    if fused:
+        back.run_quantized(arena.send_q, arena.send_params, quant_segments(stacked.send_range, bits), bits, out)
+    else:
+        back.run(arena.send, out, True)
+
+
 class LoopbackAggregator(torch.autograd.Function):
     """``outs = LoopbackAggregator.apply(world, *feats)`` with ``world = LoopbackWorld(...)``;
     ``feats[p]`` are partition p's node features [n_p, F] on the GPU, ``outs[p]`` its aggregated rows."""
@@ -267,11 +437,25 @@ class LoopbackAggregator(torch.autograd.Function):
     @staticmethod
     def forward(ctx, world, *feats):
         ctx.world = world
-        return tuple(_world_forward(world, feats, world.num_bits))
+        return _per_partition(world, feats, _stacked_forward, _world_forward)
 
     @staticmethod
     def backward(ctx, *grads):
-        return (None,) + tuple(_world_backward(ctx.world, grads, ctx.world.num_bits))
+        return (None,) + _per_partition(ctx.world, grads, _stacked_backward, _world_backward)
+
+
+def _per_partition(world, rows, together, one_by_one):
+    """One direction over a list of tensors, one per partition, each result a tensor of its own."""
+    sizes = world.partition_sizes
+    if len(rows) == len(sizes) and all(r.dim() == 2 and r.is_cuda and r.dtype == torch.float32 and r.shape[1] == rows[0].shape[1]
+                                       and r.shape[0] == n and r.device == rows[0].device for r, n in zip(rows, sizes)):
+        stacked = _Stacked.of(world, rows[0], world.num_bits, backward=together is _stacked_backward)
+        if stacked is not None:
+            x = torch.cat(rows)
+            out = torch.empty_like(x)
+            together(world, stacked, x, world.num_bits, out)
+            return tuple(o.clone() for o in torch.split(out, sizes))
+    return tuple(one_by_one(world, rows, world.num_bits))
 
 
 class Aggregator(torch.autograd.Function):
@@ -298,7 +482,12 @@ class Aggregator(torch.autograd.Function):
         x = local_nodes_feat.contiguous()
         feats = torch.split(x, world.partition_sizes) if len(world.graphs) > 1 else (x,)
         out = torch.empty((world.node_offsets[-1], x.shape[-1]), dtype=torch.float32, device=x.device)
-        _world_forward(world, feats, int(num_bits) if is_training else 32, out_all=out)
+        bits = int(num_bits) if is_training else 32
+        stacked = _Stacked.of(world, x, bits)
+        if stacked is not None:
+            _stacked_forward(world, stacked, x, bits, out)
+        else:
+            _world_forward(world, feats, bits, out_all=out)
         return out
 
     @staticmethod
@@ -307,7 +496,11 @@ class Aggregator(torch.autograd.Function):
         g = local_out_grad.contiguous()
         grads = torch.split(g, world.partition_sizes) if len(world.graphs) > 1 else (g,)
         out = torch.empty((world.node_offsets[-1], g.shape[-1]), dtype=torch.float32, device=g.device)
-        _world_backward(world, grads, ctx.num_bits, out_all=out)
+        stacked = _Stacked.of(world, g, ctx.num_bits, backward=True)
+        if stacked is not None:
+            _stacked_backward(world, stacked, g, ctx.num_bits, out)
+        else:
+            _world_backward(world, grads, ctx.num_bits, out_all=out)
         return None, out, None, None, None, None
 
 
@@ -356,6 +549,7 @@ class LoopbackWorld(object):
         self._current = None
         self._side = None
         self._in_degrees = None
+        self._stacked = None
 
     def arena(self, F, device, bits=None):
         """Buffers are kept per feature width and exchange format; the partitions' buffer attributes are

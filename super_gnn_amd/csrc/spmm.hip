@@ -1035,6 +1035,13 @@ __global__ __launch_bounds__(kBlock) void translate_columns_kernel(const int32_t
     if (i < n) dst[i] = table[__builtin_nontemporal_load(idx + i)];
 }
 
+// dst[i] = (src ? src[i] : i) + add: index arrays of a plan carried over into a stacked plan.
+__global__ __launch_bounds__(kBlock) void shift_indices_kernel(const int32_t *__restrict__ src, int32_t *__restrict__ dst, int64_t n,
+                                                               int32_t add) {
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) dst[i] = (src ? src[i] : (int32_t)i) + add;
+}
+
 __global__ __launch_bounds__(kBlock) void permute_values_kernel(const float *__restrict__ val, const int32_t *__restrict__ eperm,
                                                                 float *__restrict__ dst, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
@@ -1333,6 +1340,7 @@ struct sgnn_spmm_plan {
     // edges than that (the kernels' edge offsets are 32-bit); every call on the whole runs the blocks in turn.
     std::vector<sgnn_spmm_plan *> parts;
     std::vector<int64_t> part_row0, part_edge0;
+    bool stacked = false;              // made of other plans (sgnn_spmm_plan_stack): row-class schedule only
     sgnn_spmm_plan *whole = nullptr;   // a row block: the plan it belongs to, which owns the restaged-operand workspace
     uint64_t call_serial = 0;          // products run on this (whole) plan so far
     uint64_t xs_serial = 0;            // the product whose dense operand band_xs holds ...
@@ -1656,6 +1664,129 @@ extern "C" int sgnn_spmm_plan_create(const int64_t *rowptr, const void *col, int
     return SGNN_OK;
 }
 
+static int shift_indices(const int32_t *src, int32_t *dst, int64_t n, int64_t add, hipStream_t st) {
+    if (n == 0) return SGNN_OK;
+    hipLaunchKernelGGL(shift_indices_kernel, dim3((uint32_t)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, src, dst, n, (int32_t)add);
+    SGNN_HIP_CHECK(hipGetLastError());
+    return SGNN_OK;
+}
+
+template <typename T>
+static int download(std::vector<T> &dst, const T *src, size_t n, hipStream_t st) {
+    dst.resize(n);
+    if (n == 0) return SGNN_OK;
+    SGNN_HIP_CHECK(hipMemcpyAsync(dst.data(), src, sizeof(T) * n, hipMemcpyDeviceToHost, st));
+    SGNN_HIP_CHECK(hipStreamSynchronize(st));
+    return SGNN_OK;
+}
+
+// The long rows' pieces are taken over as they are, so a row's partial sums are the same, and are added in the same order, as
+// in its own plan's product; the chunks of short rows are cut anew (a row's sum does not depend on them).
+static int plan_stack_impl(sgnn_spmm_plan *p, sgnn_spmm_plan *const *parts, int n_parts, hipStream_t st) {
+    SGNN_HIP_CHECK(hipGetDevice(&p->device));
+    bool any = false;
+    int64_t long_room = 0;
+    for (int i = 0; i < n_parts; ++i) any = any || parts[i]->partitioned;
+    for (int i = 0; i < n_parts; ++i) {
+        const sgnn_spmm_plan *q = parts[i];
+        // the regrouped arrays hold a partitioned part's long rows, or all edges of another part that has long rows
+        if (any && q->n_long > 0) long_room += q->partitioned ? q->long_edges : q->nnz;
+    }
+    if (long_room > INT32_MAX) return fail(SGNN_ERR_ARG, "stacked plans hold at most 2^31 - 1 regrouped edges");
+    p->partitioned = any;
+    p->h_rowptr.assign(1, 0);
+    SGNN_HIP_CHECK(hipMalloc(&p->col, sizeof(int32_t) * (size_t)std::max<int64_t>(p->nnz, 1)));
+    if (any) {
+        SGNN_HIP_CHECK(hipMalloc(&p->col_long, sizeof(int32_t) * (size_t)std::max<int64_t>(long_room, 1)));
+        SGNN_HIP_CHECK(hipMalloc(&p->eperm, sizeof(int32_t) * (size_t)std::max<int64_t>(long_room, 1)));
+    } else {
+        p->col_long = p->col;
+    }
+    std::vector<int32_t> long_rows, long_pbeg(1, 0), empty_rows;
+    std::vector<std::vector<int4>> work(kNumXCD);
+    int64_t row0 = 0, col0 = 0, edge0 = 0, long0 = 0, item0 = 0, long_edges = 0;
+    int rc;
+    for (int i = 0; i < n_parts; ++i) {
+        const sgnn_spmm_plan *q = parts[i];
+        for (int64_t m = 1; m <= q->M; ++m) p->h_rowptr.push_back(edge0 + q->h_rowptr[(size_t)m]);
+        if ((rc = shift_indices(q->col, p->col + edge0, q->nnz, col0, st)) != SGNN_OK) return rc;
+        std::vector<int32_t> rows, pbeg, empty;
+        std::vector<int4> cls;
+        if ((rc = download(empty, q->empty_rows, (size_t)q->n_empty, st)) != SGNN_OK) return rc;
+        for (int32_t r : empty) empty_rows.push_back((int32_t)(r + row0));
+        if (q->n_long > 0) {
+            if ((rc = download(rows, q->long_rows, (size_t)q->n_long, st)) != SGNN_OK) return rc;
+            if ((rc = download(pbeg, q->long_pbeg, (size_t)q->n_long + 1, st)) != SGNN_OK) return rc;
+            if ((rc = download(cls, q->cls_work, (size_t)kNumXCD * (size_t)q->max_cls_items, st)) != SGNN_OK) return rc;
+            for (int32_t r : rows) long_rows.push_back((int32_t)(r + row0));
+            for (size_t k = 1; k < pbeg.size(); ++k) long_pbeg.push_back((int32_t)(pbeg[k] + item0));
+            for (int c = 0; c < kNumXCD; ++c)
+                for (int k = 0; k < q->max_cls_items; ++k) {
+                    const int4 w = cls[(size_t)c * q->max_cls_items + k];
+                    if (w.z > 0) work[c].push_back(make_int4((int)(w.x + item0), (int)(w.y + (any ? long0 : edge0)), w.z, 0));
+                }
+            if (any) {
+                const int64_t n = q->partitioned ? q->long_edges : q->nnz;
+                if ((rc = shift_indices(q->partitioned ? q->col_long : q->col, p->col_long + long0, n, col0, st)) != SGNN_OK) return rc;
+                if ((rc = shift_indices(q->eperm, p->eperm + long0, n, edge0, st)) != SGNN_OK) return rc;
+                long0 += n;
+            }
+            item0 += q->n_items;
+            if (item0 > INT32_MAX / 2) return fail(SGNN_ERR_ARG, "too many long-row pieces");
+        }
+        long_edges += q->long_edges;
+        row0 += q->M;
+        col0 += q->K;
+        edge0 += q->nnz;
+    }
+    p->n_long = (int64_t)long_rows.size();
+    p->n_items = item0;
+    p->n_empty = (int64_t)empty_rows.size();
+    p->long_edges = long_edges;
+    for (int c = 0; c < kNumXCD; ++c) p->max_cls_items = std::max<int>(p->max_cls_items, (int)work[c].size());
+    std::vector<int4> cls_work((size_t)kNumXCD * (size_t)p->max_cls_items, make_int4(0, 0, 0, 0));
+    for (int c = 0; c < kNumXCD; ++c)
+        std::copy(work[c].begin(), work[c].end(), cls_work.begin() + (size_t)c * p->max_cls_items);
+    if ((rc = upload(&p->rowptr, p->h_rowptr, st)) != SGNN_OK) return rc;
+    if ((rc = upload(&p->empty_rows, empty_rows, st)) != SGNN_OK) return rc;
+    if (p->n_long > 0) {
+        if ((rc = upload(&p->long_rows, long_rows, st)) != SGNN_OK) return rc;
+        if ((rc = upload(&p->long_pbeg, long_pbeg, st)) != SGNN_OK) return rc;
+        if ((rc = upload(&p->cls_work, cls_work, st)) != SGNN_OK) return rc;
+    }
+    SGNN_HIP_CHECK(hipStreamSynchronize(st));
+    for (int which = 0; which < 3; ++which)
+        if ((rc = build_chunks(p, which, st)) != SGNN_OK) return rc;
+    if (any) p->long_edges = long_room;   // the length of the regrouped arrays, which the bound values and slots share
+    return SGNN_OK;
+}
+
+extern "C" int sgnn_spmm_plan_stack(sgnn_spmm_plan *const *parts, int n_parts, sgnn_stream_t stream, sgnn_spmm_plan **out) {
+    SGNN_REQUIRE(parts != nullptr && out != nullptr && n_parts >= 1, "parts / plan is null");
+    *out = nullptr;
+    int64_t M = 0, K = 0, nnz = 0;
+    int dev = 0;
+    SGNN_HIP_CHECK(hipGetDevice(&dev));
+    for (int i = 0; i < n_parts; ++i) {
+        const sgnn_spmm_plan *q = parts[i];
+        SGNN_REQUIRE(q != nullptr && q->parts.empty() && !q->stacked, "part %d is null, held as row blocks or itself stacked", i);
+        SGNN_REQUIRE(q->device == dev, "part %d was created on device %d, current device is %d", i, q->device, dev);
+        SGNN_REQUIRE(q->long_thresh == parts[0]->long_thresh, "the parts' long-row thresholds differ");
+        M += q->M; K += q->K; nnz += q->nnz;
+    }
+    SGNN_REQUIRE(M < INT32_MAX && K <= INT32_MAX && nnz <= part_edge_cap(), "M=%lld K=%lld nnz=%lld out of range for one plan",
+                 (long long)M, (long long)K, (long long)nnz);
+    std::unique_ptr<sgnn_spmm_plan, int (*)(sgnn_spmm_plan *)> p(new sgnn_spmm_plan(), sgnn_spmm_plan_destroy);
+    p->M = M; p->K = K; p->nnz = nnz;
+    p->long_thresh = parts[0]->long_thresh;
+    p->piece_edges = parts[0]->piece_edges;
+    p->stacked = true;
+    const int rc = plan_stack_impl(p.get(), parts, n_parts, (hipStream_t)stream);
+    if (rc != SGNN_OK) return rc;
+    *out = p.release();
+    return SGNN_OK;
+}
+
 extern "C" int sgnn_spmm_plan_info(const sgnn_spmm_plan *p, int64_t info[10]) {
     SGNN_REQUIRE(p != nullptr && info != nullptr, "null argument");
     info[0] = p->M; info[1] = p->K; info[2] = p->nnz; info[3] = p->n_long; info[4] = p->n_items;
@@ -1774,7 +1905,7 @@ static BandWindows band_windows(const sgnn_spmm_plan *p, int64_t F, bool even_ou
 // enough edges per band to pay for carrying its accumulator through `out` from band to band.
 static bool band_wanted(const sgnn_spmm_plan *p, int64_t F, const BandShape &b) {
     const int mode = env_int("SGNN_SPMM_BAND", -1);
-    if (mode == 0 || p->nnz == 0 || p->M == 0) return false;
+    if (mode == 0 || p->stacked || p->nnz == 0 || p->M == 0) return false;
     if (mode > 0) return true;
     if (b.n_bands < 3 || p->K * F * 4 < kBandMinDenseBytes) return false;
     return (double)p->nnz / (double)p->M / (double)b.n_bands >= kBandMinRowEdges;

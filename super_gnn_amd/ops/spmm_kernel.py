@@ -42,7 +42,17 @@ def distribute_work_for_row(rowptr: torch.Tensor, value: torch.Tensor, num_threa
 def disribute_work_for_col(other: torch.Tensor, num_threads_on_col: int) -> torch.Tensor:
     """Even split of the feature axis (super_gnn/ops/spmm_kernel.py:31-44; the misspelt name is the
     reference's)."""
-    num_cols = other.shape[-1]
+    return _col_splits(other.shape[-1], num_threads_on_col)
+
+
+def work_range(row_splits, rowptr, value, width):
+    """(row_splits, col_splits) as a product of this width leaves them; an existing row split is kept."""
+    if row_splits.size(0) == 0:
+        row_splits = distribute_work_for_row(rowptr, value, torch.get_num_threads())
+    return row_splits, _col_splits(width, 1)
+
+
+def _col_splits(num_cols, num_threads_on_col):
     target = num_cols // num_threads_on_col
     col_splits = torch.full((num_threads_on_col + 1,), num_cols, dtype=torch.int32)
     for i in range(num_threads_on_col):

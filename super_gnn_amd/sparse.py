@@ -65,6 +65,7 @@ class SparseTensor:
         self._colptr = self._row_T = self._value_T = None
         self._work_range = (torch.empty(0, dtype=torch.int32), torch.empty(0, dtype=torch.int32))
         self._work_range_T = (torch.empty(0, dtype=torch.int32), torch.empty(0, dtype=torch.int32))
+        self._used_width = self._used_width_T = None
         self._plan = None
         self._plan_T = None
         self.storage = _Storage(self)
@@ -114,16 +115,35 @@ class SparseTensor:
         out.index_put_((row, col), torch.ones_like(col, dtype=out.dtype) if val is None else val, accumulate=True)
         return out
 
+    def note_use(self, width, transposed=False):
+        """A product of this feature width ran on this matrix's behalf (stacked with others): the work range that the
+        façade would have stored is then computed when somebody asks for it."""
+        if transposed:
+            self._used_width_T = width
+        else:
+            self._used_width = width
+
     def get_work_range(self):
+        if self._used_width is not None:
+            from .ops.spmm_kernel import work_range
+            self._work_range = work_range(self._work_range[0], self._rowptr, self._value, self._used_width)
+            self._used_width = None
         return self._work_range
 
     def set_work_range(self, row_splits, col_splits):
+        self._used_width = None
         self._work_range = (row_splits, col_splits)
 
     def get_work_range_for_transpose(self):
+        if self._used_width_T is not None:
+            from .ops.spmm_kernel import work_range
+            self._build_transpose()
+            self._work_range_T = work_range(self._work_range_T[0], self._colptr, self._value_T, self._used_width_T)
+            self._used_width_T = None
         return self._work_range_T
 
     def set_work_range_for_transpose(self, row_splits, col_splits):
+        self._used_width_T = None
         self._work_range_T = (row_splits, col_splits)
 
     # ---- cached per-matrix state of this build ----------------------------------------------

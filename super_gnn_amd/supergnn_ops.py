@@ -112,6 +112,21 @@ class SpmmPlan:
         h = ctypes.c_void_p()
         check(lib.sgnn_spmm_plan_create(_ptr(rp), _ptr(cl), int(cl.dtype == torch.int64), self.M, self.K, self.nnz,
                                         int(long_row_threshold), int(piece_edges), _stream(), ctypes.byref(h)))
+        self._adopt(h, dev)
+
+    @classmethod
+    def stack(cls, plans):
+        """The plan of the block-diagonal matrix of ``plans`` (sgnn_spmm_plan_stack): same sums, one launch sequence."""
+        self = cls.__new__(cls)
+        self.M, self.K, self.nnz = (sum(getattr(p, k) for p in plans) for k in ("M", "K", "nnz"))
+        handles = (ctypes.c_void_p * len(plans))(*[p._h for p in plans])
+        _destroy_plan_handle()
+        h = ctypes.c_void_p()
+        check(lib.sgnn_spmm_plan_stack(handles, len(plans), _stream(), ctypes.byref(h)))
+        self._adopt(h, plans[0].device)
+        return self
+
+    def _adopt(self, h, dev):
         self._h = h
         self._bound = None   # (value tensor, version) whose long-row values the plan holds in its own order
         self._seen = None    # (value tensor, version) of the previous call
