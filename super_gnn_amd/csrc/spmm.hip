@@ -789,7 +789,7 @@ __global__ __launch_bounds__(kBlock) void spmm_empty_rows_kernel(const int32_t *
 template <int VEC, int G, int NV, int BITS, bool PERM>
 __global__ __launch_bounds__(kBlock) void spmm_piece_kernel(
     const int32_t *__restrict__ col_long, const int32_t *__restrict__ eperm, const float *__restrict__ val,
-    const DenseSrc dense, float *__restrict__ partial, const int4 *__restrict__ cls_work, int cls_stride, int F) {
+    const DenseSrc dense, float *__restrict__ partial, const int4 *__restrict__ cls_work, int cls_stride, int F, int keep) {
     constexpr int GPB = kBlock / G;
     constexpr int TILE = G * VEC * NV;
     const int gid = threadIdx.x / G, lig = threadIdx.x % G;
@@ -824,7 +824,10 @@ __global__ __launch_bounds__(kBlock) void spmm_piece_kernel(
                                              off_ld, act_ld, lig);
 #pragma unroll
         for (int v = 0; v < NV; ++v)
-            if (act[v]) vec_store_nt<VEC>(partial + (int64_t)item * F + off[v], acc[v]);
+            if (act[v]) {
+                if (keep) vec_store<VEC>(partial + (int64_t)item * F + off[v], acc[v]);
+                else vec_store_nt<VEC>(partial + (int64_t)item * F + off[v], acc[v]);
+            }
     }
 }
 
@@ -888,16 +891,19 @@ __global__ __launch_bounds__(kBlock) void spmm_hubrow_lds_kernel(
 }
 
 // ------------------------------------------------------------------------------------------------
-// Long rows, step 2: add a row's piece partials in piece order, epilogue, store.
+// Long rows, step 2: add a row's piece partials in piece order, epilogue, store.  A row's time is its chain of batches of UP
+// partials.  KEEP: the partials of the whole product are few enough (keep_partials) to stay in the L2s, written and read with
+// ordinary accesses instead of streaming ones: 200 k power-law nodes, F = 100 18.8 -> 14.2 us, fused 1 M rows 28.1 -> 20.0;
+// beyond that they only push dense rows out (1 M nodes, 32 M edges: the product 1.41 -> 1.47 ms, UP = 16 as well as 8).
 // ------------------------------------------------------------------------------------------------
-template <int VEC, int G, int NV>
+template <int VEC, int G, int NV, bool KEEP>
 __global__ __launch_bounds__(kBlock) void spmm_long_final_kernel(
     const int32_t *__restrict__ long_rows, const int32_t *__restrict__ long_pbeg,
     const float *__restrict__ partial, float *__restrict__ out, int n_long, int F, int64_t ldo,
     int accumulate, const float *__restrict__ row_div) {
     constexpr int GPB = kBlock / G;
     constexpr int TILE = G * VEC * NV;
-    constexpr int UP = 8;
+    constexpr int UP = KEEP ? 16 : 8;
     const int gid = threadIdx.x / G, lig = threadIdx.x % G;
     const int li = blockIdx.x * GPB + gid;
     if (li >= n_long) return;
@@ -919,7 +925,8 @@ __global__ __launch_bounds__(kBlock) void spmm_long_final_kernel(
 #pragma unroll
                 for (int u = 0; u < UP; ++u) {
                     const int si = s + u < s1 ? s + u : s1 - 1;
-                    vec_load_nt<VEC>(p[u], partial + (int64_t)si * F + off);
+                    if constexpr (KEEP) vec_load<VEC>(p[u], partial + (int64_t)si * F + off);
+                    else vec_load_nt<VEC>(p[u], partial + (int64_t)si * F + off);
                 }
 #pragma unroll
                 for (int u = 0; u < UP; ++u) {
@@ -1124,6 +1131,7 @@ struct PieceArgs {
     const int32_t *col_long; const int32_t *eperm; const float *val; float *partial;
     const int4 *cls_work;
     int max_cls_items; int F;
+    int keep;   // see keep_partials
 };
 struct FinalArgs {
     const int32_t *long_rows; const int32_t *long_pbeg; const float *partial; float *out; int n_long;
@@ -1140,6 +1148,9 @@ constexpr int kDeepChunks = kChunkGroupsWanted;
 static uint32_t short_spare_lds(int bits, int G, int NV, int64_t x_bytes) {
     return bits == 0 && NV == 1 && (G == 16 || G == 32) && x_bytes > (256ll << 20) ? 40000 : 0;
 }
+
+// Up to about the eight L2s together (32 MB), the long rows' partial sums are kept in them from the piece kernel to the final sum.
+static int keep_partials(int64_t n_items, int64_t F) { return n_items * F * 4 <= (40ll << 20); }
 
 template <int VEC, int G, int NV, int BITS>
 static void launch_all(const ShortArgs &a, const PieceArgs &s, const FinalArgs &f, hipStream_t st) {
@@ -1160,15 +1171,19 @@ static void launch_all(const ShortArgs &a, const PieceArgs &s, const FinalArgs &
             ProfScope prof(BITS == 0 ? K_SPMM_PIECE : K_FUSED_PIECE, ls, a.prof);
             if (s.eperm)
                 hipLaunchKernelGGL((spmm_piece_kernel<VEC, G, NV, BITS, true>), dim3(nb), dim3(kBlock), 0, ls, s.col_long,
-                                   s.eperm, s.val, a.dense, s.partial, s.cls_work, s.max_cls_items, s.F);
+                                   s.eperm, s.val, a.dense, s.partial, s.cls_work, s.max_cls_items, s.F, s.keep);
             else
                 hipLaunchKernelGGL((spmm_piece_kernel<VEC, G, NV, BITS, false>), dim3(nb), dim3(kBlock), 0, ls, s.col_long,
-                                   s.eperm, s.val, a.dense, s.partial, s.cls_work, s.max_cls_items, s.F);
+                                   s.eperm, s.val, a.dense, s.partial, s.cls_work, s.max_cls_items, s.F, s.keep);
         }
         const uint32_t nb = (uint32_t)((f.n_long + GPB - 1) / GPB);
         ProfScope prof(K_SPMM_LONG_FINAL, ls, a.prof);
-        hipLaunchKernelGGL((spmm_long_final_kernel<VEC, G, NV>), dim3(nb), dim3(kBlock), 0, ls, f.long_rows,
-                           f.long_pbeg, f.partial, f.out, f.n_long, f.F, f.ldo, f.accumulate, f.row_div);
+        if (s.keep)
+            hipLaunchKernelGGL((spmm_long_final_kernel<VEC, G, NV, true>), dim3(nb), dim3(kBlock), 0, ls, f.long_rows,
+                               f.long_pbeg, f.partial, f.out, f.n_long, f.F, f.ldo, f.accumulate, f.row_div);
+        else
+            hipLaunchKernelGGL((spmm_long_final_kernel<VEC, G, NV, false>), dim3(nb), dim3(kBlock), 0, ls, f.long_rows,
+                               f.long_pbeg, f.partial, f.out, f.n_long, f.F, f.ldo, f.accumulate, f.row_div);
     }
     if (a.n_chunks > 0) {
         const uint32_t nb = (uint32_t)((a.n_chunks + GPB - 1) / GPB);
@@ -2356,7 +2371,7 @@ static int spmm_run(sgnn_spmm_plan *p, const float *val, const DenseSrc &dense, 
     ShortArgs a{p->rowptr, p->col, val, dense, out, p->chunks[which], (int)p->n_chunks[which], p->empty_rows,
                 (int)p->n_empty, (int)F, ldo, accumulate, row_div, scratch == nullptr,
                 bits == 0 ? p->K * F * 4 : p->K * F * bits / 8};
-    PieceArgs s{p->col_long, p->eperm, val, partial, p->cls_work, p->max_cls_items, (int)F};
+    PieceArgs s{p->col_long, p->eperm, val, partial, p->cls_work, p->max_cls_items, (int)F, keep_partials(p->n_items, F)};
     if (val != nullptr && val == p->bound_val && p->val_long != nullptr) {
         s.eperm = nullptr;   // values already sit in regrouped order: contiguous reads, no indirection
         s.val = p->val_long;
