@@ -5,8 +5,8 @@
 
 The reference computes an nnz-balanced OpenMP row split on first use and caches it on the matrix
 (spmm_kernel.py:49-58); here the object that matters is the GPU schedule (SpmmPlan), cached the same
-way.  The row split is still computed once per matrix and stored through the work-range setters, so
-callers that read ``get_work_range()`` see what the reference would have put there."""
+way.  The row split is computed once per matrix, when ``get_work_range()`` is first called after a
+product: callers see what the reference would have put there."""
 import torch
 
 from ..supergnn_ops import quant_segments, spmm
@@ -66,15 +66,11 @@ def SPMM_forward(src, other: torch.Tensor, out: torch.Tensor, accumulate=None) -
     ``False`` writes out = A @ other, which equals zero-filling out and accumulating, bit for bit,
     without the fill and the read-back."""
     rowptr, col, value = src.csr()
-    col_splits = disribute_work_for_col(other, 1)
-    row_splits, _ = src.get_work_range()
-    if row_splits.size(0) == 0:   # once per matrix, as the reference does (spmm_kernel.py:49-53)
-        row_splits = distribute_work_for_row(rowptr, value, torch.get_num_threads())
-    src.set_work_range(row_splits, col_splits)
+    src.note_use(other.shape[-1])   # the work range is computed when asked for (the tensors alone took 6 us of every call)
     if value is not None:
         value = value.to(other.dtype)
     sparse_row = rowptr.shape[0] - 1
-    spmm(rowptr, col, value, other, out, sparse_row, row_splits, col_splits, plan=src.spmm_plan(), accumulate=accumulate)
+    spmm(rowptr, col, value, other, out, sparse_row, plan=src.spmm_plan(), accumulate=accumulate)
     return None
 
 
@@ -82,16 +78,11 @@ def SPMM_backward(src, other: torch.Tensor, out: torch.Tensor, accumulate=None) 
     colptr = src.storage.colptr()
     row_T = src.storage.row_T()
     value_T = src.storage.value_T()
-    col_splits = disribute_work_for_col(other, 1)
-    row_splits, _ = src.get_work_range_for_transpose()
-    if row_splits.size(0) == 0:   # spmm_kernel.py:82-85
-        row_splits = distribute_work_for_row(colptr, value_T, torch.get_num_threads())
-    src.set_work_range_for_transpose(row_splits, col_splits)
+    src.note_use(other.shape[-1], transposed=True)
     if value_T is not None:
         value_T = value_T.to(other.dtype)
     sparse_row = colptr.shape[0] - 1
-    return spmm(colptr, row_T, value_T, other, out, sparse_row, row_splits, col_splits, plan=src.spmm_plan_T(),
-                accumulate=accumulate)
+    return spmm(colptr, row_T, value_T, other, out, sparse_row, plan=src.spmm_plan_T(), accumulate=accumulate)
 
 
 def SPMM_forward_quantized(src, data_int8: torch.Tensor, quantized_params: torch.Tensor,

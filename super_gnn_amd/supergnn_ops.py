@@ -50,12 +50,12 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 def _stream():
     """The current stream's hipStream_t (the raw getter is ~8 us cheaper per call than the Stream object)."""
     if _raw_stream is not None:
-        return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return _raw_stream(torch.cuda.current_device())
+    return torch.cuda.current_stream().cuda_stream
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def _want(t, dtype, name):
@@ -86,6 +86,15 @@ class _Staged:
         if self.writeback:
             with torch.no_grad():
                 self.orig.copy_(self.dev)
+
+
+def _in_place(*tensors):
+    """True when every tensor can be handed to the library as it is: on the GPU and contiguous.  Staging objects for them
+    are 1 ... 2 us each, of calls whose kernels take 4 us."""
+    for t in tensors:
+        if t is not None and not (t.is_cuda and t.is_contiguous()):
+            return False
+    return True
 
 
 # -------------------------------------------------------------------------------------------------
@@ -164,12 +173,18 @@ class SpmmPlan:
             _want(row_div, torch.float32, "row_div")
             if row_div.numel() != self.M:
                 raise ValueError("row_div must have one entry per sparse row")
+        F = mat.shape[1]
+        if _in_place(value, mat, out, row_div):
+            if value is not None:
+                self._maybe_bind(value)
+            check(lib.sgnn_spmm_csr_f32(self._h, _ptr(value), mat.data_ptr(), out.data_ptr(), F, F, F, 1 if accumulate else 0,
+                                        _ptr(row_div), _stream()))
+            return
         dev = self.device
         s_val = _Staged(value, dev) if value is not None else None
         s_mat = _Staged(mat, dev)
         s_out = _Staged(out, dev, writeback=True)
         s_div = _Staged(row_div, dev) if row_div is not None else None
-        F = mat.shape[1]
         if value is not None and value.is_cuda and value.is_contiguous():
             self._maybe_bind(value)
         check(lib.sgnn_spmm_csr_f32(self._h, _ptr(s_val.dev) if s_val else None, _ptr(s_mat.dev), _ptr(s_out.dev),
@@ -365,13 +380,12 @@ def quant_segments(work_range, bits):
     """Device copies of the segment table and its packed-row offsets, cached on the tensor object
     (keyed by its version counter, so in-place edits rebuild them)."""
     _want(work_range, torch.int32, "work_range_per_proc")
-    dev = _device()
     cache = work_range.__dict__.setdefault("_sgnn_segments", {})
-    key = (int(bits), work_range._version, str(dev))
+    key = (int(bits), work_range._version, torch.cuda.current_device())
     s = cache.get(key)
     if s is None:
         cache.clear()
-        s = _Segments(work_range.detach().cpu(), int(bits), dev)
+        s = _Segments(work_range.detach().cpu(), int(bits), _device())
         cache[key] = s
     return s
 
@@ -419,18 +433,25 @@ def _quant_rows(inp, out_u8, params, segs, bits, row_index=None):
         raise ValueError(f"output holds {out_u8.numel()} bytes, {segs.n_packed * F} needed")
     if params.numel() < n * 2:
         raise ValueError(f"quantized_params holds {params.numel()} floats, {n * 2} needed")
+    if _in_place(inp, out_u8, params):
+        _launch_quant(inp, out_u8, params, bf16, segs, n, F, bits)
+        return
     dev = _device()
     s_in = _Staged(inp, dev)
     s_q = _Staged(out_u8, dev, writeback=True)
     s_p = _Staged(params, dev, writeback=True)
-    if bf16:
-        check(lib.sgnn_quant_pack_rows_wire_f32(_ptr(s_in.dev), F, None, n, _ptr(s_q.dev), _ptr(s_p.dev), 1, _ptr(segs.seg),
-                                                _ptr(segs.pseg), segs.P, n, segs.n_packed, F, bits, _stream()))
-    else:
-        check(lib.sgnn_quant_pack_rows_f32(_ptr(s_in.dev), _ptr(s_q.dev), _ptr(s_p.dev), _ptr(segs.seg), _ptr(segs.pseg),
-                                           segs.P, n, segs.n_packed, F, bits, _stream()))
+    _launch_quant(s_in.dev, s_q.dev, s_p.dev, bf16, segs, n, F, bits)
     s_q.commit()
     s_p.commit()
+
+
+def _launch_quant(inp, out_u8, params, bf16, segs, n, F, bits):
+    if bf16:
+        check(lib.sgnn_quant_pack_rows_wire_f32(_ptr(inp), F, None, n, _ptr(out_u8), _ptr(params), 1, _ptr(segs.seg),
+                                                _ptr(segs.pseg), segs.P, n, segs.n_packed, F, bits, _stream()))
+    else:
+        check(lib.sgnn_quant_pack_rows_f32(_ptr(inp), _ptr(out_u8), _ptr(params), _ptr(segs.seg), _ptr(segs.pseg),
+                                           segs.P, n, segs.n_packed, F, bits, _stream()))
 
 
 def _quant_gathered_rows(src, row_index, out_u8, params, bf16, segs, bits):
@@ -466,24 +487,31 @@ def _dequant_rows(inp_u8, out, params, segs, bits):
         raise ValueError(f"input holds {inp_u8.numel()} bytes, {segs.n_packed * F} needed")
     if params.numel() < n * 2:
         raise ValueError(f"dequantized_params holds {params.numel()} floats, {n * 2} needed")
+    if _in_place(inp_u8, params, out):
+        _launch_dequant(inp_u8, out, params, bf16, segs, n, F, bits)
+        return
     dev = _device()
     s_q = _Staged(inp_u8, dev)
     s_p = _Staged(params, dev)
     s_out = _Staged(out, dev, writeback=True)
+    _launch_dequant(s_q.dev, s_out.dev, s_p.dev, bf16, segs, n, F, bits)
+    s_out.commit()
+
+
+def _launch_dequant(inp_u8, out, params, bf16, segs, n, F, bits):
     if bf16:
-        check(lib.sgnn_unpack_dequant_rows_wire_f32(_ptr(s_q.dev), _ptr(s_out.dev), _ptr(s_p.dev), 1, _ptr(segs.seg),
+        check(lib.sgnn_unpack_dequant_rows_wire_f32(_ptr(inp_u8), _ptr(out), _ptr(params), 1, _ptr(segs.seg),
                                                     _ptr(segs.pseg), segs.P, n, segs.n_packed, F, bits, _stream()))
     else:
-        check(lib.sgnn_unpack_dequant_rows_f32(_ptr(s_q.dev), _ptr(s_out.dev), _ptr(s_p.dev), _ptr(segs.seg),
+        check(lib.sgnn_unpack_dequant_rows_f32(_ptr(inp_u8), _ptr(out), _ptr(params), _ptr(segs.seg),
                                                _ptr(segs.pseg), segs.P, n, segs.n_packed, F, bits, _stream()))
-    s_out.commit()
 
 
 _SINGLE_SEG = OrderedDict()
 
 
 def _single_segment(n, bits):
-    key = (int(n), int(bits), str(_device()))
+    key = (int(n), int(bits), torch.cuda.current_device())
     s = _SINGLE_SEG.get(key)
     if s is None:
         s = _Segments(torch.tensor([0, int(n)], dtype=torch.int32), int(bits), _device())
