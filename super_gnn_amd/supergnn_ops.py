@@ -139,6 +139,7 @@ class SpmmPlan:
         self._h = h
         self._bound = None   # (value tensor, version) whose long-row values the plan holds in its own order
         self._seen = None    # (value tensor, version) of the previous call
+        self.hand_binds = 0  # calls of bind_values / unbind_values so far
         self._bound_slots = None  # row-slot table (a tensor owned by a _Segments object) bound to the plan
         self.device = dev
 
@@ -155,8 +156,8 @@ class SpmmPlan:
         check(lib.sgnn_spmm_plan_schedule(self._h, int(F), buf))
         return dict(zip(("band", "band_cols", "n_bands", "n_slices"), list(buf)))
 
-    def run(self, value, mat, out, accumulate=True, row_div=None):
-        """out (+)= A @ mat on the current stream.  value None = all ones."""
+    def run(self, value, mat, out, accumulate=True, row_div=None, bind=True):
+        """out (+)= A @ mat on the current stream.  value None = all ones.  bind False: the caller binds the values itself."""
         _want(mat, torch.float32, "mat")
         _want(out, torch.float32, "out")
         if value is not None:
@@ -175,7 +176,7 @@ class SpmmPlan:
                 raise ValueError("row_div must have one entry per sparse row")
         F = mat.shape[1]
         if _in_place(value, mat, out, row_div):
-            if value is not None:
+            if value is not None and bind:
                 self._maybe_bind(value)
             check(lib.sgnn_spmm_csr_f32(self._h, _ptr(value), mat.data_ptr(), out.data_ptr(), F, F, F, 1 if accumulate else 0,
                                         _ptr(row_div), _stream()))
@@ -185,7 +186,7 @@ class SpmmPlan:
         s_mat = _Staged(mat, dev)
         s_out = _Staged(out, dev, writeback=True)
         s_div = _Staged(row_div, dev) if row_div is not None else None
-        if value is not None and value.is_cuda and value.is_contiguous():
+        if bind and value is not None and value.is_cuda and value.is_contiguous():
             self._maybe_bind(value)
         check(lib.sgnn_spmm_csr_f32(self._h, _ptr(s_val.dev) if s_val else None, _ptr(s_mat.dev), _ptr(s_out.dev),
                                     F, F, F, int(bool(accumulate)), _ptr(s_div.dev) if s_div else None, _stream()))
@@ -218,13 +219,15 @@ class SpmmPlan:
             raise ValueError("value must be a contiguous GPU tensor with one entry per edge")
         check(lib.sgnn_spmm_plan_bind_values(self._h, _ptr(value), _stream()))
         self._bound = self._seen = (value, value._version)
+        self.hand_binds += 1
 
     def unbind_values(self):
         """Forget the bound edge values: every later product reads the tensor it is given."""
         check(lib.sgnn_spmm_plan_bind_values(self._h, None, _stream()))
         self._bound = self._seen = None
+        self.hand_binds += 1
 
-    def run_quantized(self, value, data_int8, params, segs, bits, out, accumulate=True, row_div=None):
+    def run_quantized(self, value, data_int8, params, segs, bits, out, accumulate=True, row_div=None, bind=True):
         """out (+)= A @ dequantize(data_int8): the dense operand stays packed (row-group layout,
         ``segs`` from quant_segments()) and is decoded inside the gather."""
         _check_bits(bits)
@@ -255,7 +258,7 @@ class SpmmPlan:
             # the segment table of a partition never changes: carry each edge's slot with its column
             check(lib.sgnn_spmm_plan_bind_row_slots(self._h, _ptr(slots), _stream()))
             self._bound_slots = slots
-        if value is not None and value.is_contiguous():
+        if bind and value is not None and value.is_contiguous():
             self._maybe_bind(value)
         if bf16:
             check(lib.sgnn_spmm_csr_dq_wire_f32(self._h, _ptr(value), _ptr(data_int8), _ptr(params), 1, _ptr(slots), bits,

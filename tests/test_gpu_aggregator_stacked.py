@@ -53,3 +53,114 @@ def test_edited_values_are_seen():
     world.graphs[1].local_adj_t.csr()[2].mul_(2)
     got, want = _both(world, x, grad, 32, True)
     assert torch.equal(got[0], want[0]) and not torch.equal(got[0], before[0])
+
+
+def _mats(world):
+    return [m for g in world.graphs for m in (g.local_adj_t, *((g.adj_t_pre_post_aggr_from, g.adj_t_pre_post_aggr_to)
+                                                               if world.is_pre_delay else (g.remote_adj_t,)))]
+
+
+def _same(world, x, grad, bits, pre):
+    got, want = _both(world, x, grad, bits, pre)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    return got
+
+
+@pytest.mark.parametrize("bits", [32, 4])
+@pytest.mark.parametrize("P,pre", [(3, True), (5, True), (5, False)])
+def test_edits_reach_both_directions(P, pre, bits):
+    """Edits of the values and of the transposed values, before and after the plans hold the long rows' values (from the
+    second unchanged pass on), with no plan made anew."""
+    F = 64
+    world = _world(P, F, bits, pre, False)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x, grad = (torch.randn(N, F, generator=g, device="cuda") for _ in range(2))
+    before = _same(world, x, grad, bits, pre)
+    products = dict(world._stacked.products)
+    for passes in (1, 3):
+        for _ in range(passes):
+            before = _same(world, x, grad, bits, pre)
+        for m in _mats(world):
+            m.storage.value_T().mul_(5)
+        after = _same(world, x, grad, bits, pre)
+        assert torch.equal(after[0], before[0]) and not torch.equal(after[1], before[1])
+        before = _same(world, x, grad, bits, pre)
+        for m in _mats(world):
+            m.csr()[2].add_(1)
+        after = _same(world, x, grad, bits, pre)
+        assert not torch.equal(after[0], before[0]) and torch.equal(after[1], before[1])
+    assert all(world._stacked.products[k] is p for k, p in products.items())
+
+
+def _times_two_unseen(world):
+    """Edits that no version counter sees."""
+    for m in _mats(world):
+        m.csr()[2].data.mul_(2)
+        m.storage.value_T().data.mul_(2)
+
+
+def test_unseen_edits():
+    """Rows that are no long rows are read from the caller's tensors by every product; the long rows' values follow after
+    a rebinding by hand of the partitions' own plans."""
+    g = torch.Generator(device="cuda").manual_seed(4)
+    x, grad = (torch.randn(N, 64, generator=g, device="cuda") for _ in range(2))
+    short = _world(3, 64, 32, True, False)
+    for _ in range(3):
+        before = _same(short, x, grad, 32, True)
+    _times_two_unseen(short)
+    after = _same(short, x, grad, 32, True)
+    assert not torch.equal(after[0], before[0]) and not torch.equal(after[1], before[1])
+    for rebind in ("bind", "unbind"):
+        world = _world(5, 64, 32, True, False)
+        for _ in range(3):
+            before = _same(world, x, grad, 32, True)
+        assert any(p._bound is not None for p in world._stacked.products.values())
+        _times_two_unseen(world)
+        for m in _mats(world):
+            for plan, value in ((m.spmm_plan(), m.csr()[2]), (m.spmm_plan_T(), m.storage.value_T())):
+                plan.bind_values(value) if rebind == "bind" else plan.unbind_values()
+        for _ in range(3):
+            after = _same(world, x, grad, 32, True)
+            assert not torch.equal(after[0], before[0]) and not torch.equal(after[1], before[1])
+
+
+@pytest.mark.parametrize("bits", [32, 2])
+def test_replays_read_edited_values(bits):
+    from super_gnn_amd.aggregator import Aggregator, _world_forward
+    world = _world(3, 64, bits, True, False)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(N, 64, generator=g, device="cuda")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side), torch.no_grad():
+        for _ in range(3):
+            Aggregator.apply(world, x, 0, bits, True, True)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.no_grad(), torch.cuda.graph(graph):
+        out = Aggregator.apply(world, x, 0, bits, True, True)
+    results = []
+    for _ in range(4):
+        for m in _mats(world):
+            m.csr()[2].mul_(1.5)
+        x.add_(0.25)
+        graph.replay()
+        torch.cuda.synchronize()
+        with torch.no_grad():
+            want = Aggregator.apply(world, x, 0, bits, True, True)
+        plain = torch.cat(_world_forward(world, torch.split(x, world.partition_sizes), bits))
+        assert torch.equal(out, plain) and torch.equal(want, plain)
+        results.append(out.clone())
+    assert not torch.equal(results[0], results[1])
+
+
+def test_a_wrong_number_of_values_is_refused():
+    world = _world(3, 64, 32, True, False)
+    x = torch.randn(N, 64, device="cuda")
+    _both(world, x, x, 32, True)
+    a, b = world.graphs[0].local_adj_t, world.graphs[1].local_adj_t   # the total stays what it was
+    a._value, b._value = a._value[:-1].contiguous(), torch.cat([b._value, b._value[:1]])
+    from super_gnn_amd.aggregator import Aggregator
+    with pytest.raises(ValueError, match="entries"):
+        Aggregator.apply(world, x, 0, 32, True, True)
