@@ -32,10 +32,11 @@ from typing import List, Sequence
 
 import torch
 
+from ._lib import SgnnError
 from .ops.spmm_kernel import (SPMM_backward, SPMM_backward_quantized, SPMM_forward, SPMM_forward_quantized)
 from .quantizer import Quantizer_for_all_procs
 from .sparse import SparseTensor
-from .supergnn_ops import SpmmPlan, dequantize_tensor_for_all_procs, quant_segments, quantize_tensor_for_all_procs
+from .supergnn_ops import SpmmPlan, _capturing, dequantize_tensor_for_all_procs, quant_segments, quantize_tensor_for_all_procs
 
 
 def _cumulative(splits):
@@ -276,11 +277,26 @@ class _Product(object):
 
     def __init__(self, plans):
         self.plans = plans
-        self.plan = SpmmPlan.stack(plans)
-        self.value = torch.empty(self.plan.nnz, dtype=torch.float32, device=self.plan.device)
-        self._regrouped = bool(self.plan.info()["partitioned"])
+        self.plan = None        # the stacked plan, made by stack()
+        self._refused = False
         self._bound = self._seen = None   # [(values, version, hand binds of the part's plan)] as in SpmmPlan._maybe_bind
         self._bands = {}
+
+    def stack(self):
+        """Makes the stacked plan on the first call.  False where there is none: stacking may be refused (long-row thresholds
+        that differ, a part held as row blocks, no memory), which leaves the partitions' own products as they were, and
+        inside a graph capture nothing may be allocated."""
+        if self.plan is None and not self._refused:
+            if _capturing():
+                return False
+            try:
+                plan = SpmmPlan.stack(self.plans)
+                self.value = torch.empty(plan.nnz, dtype=torch.float32, device=plan.device)
+                self._regrouped = bool(plan.info()["partitioned"])
+                self.plan = plan
+            except (ValueError, SgnnError, torch.cuda.OutOfMemoryError):
+                self._refused = True
+        return self.plan is not None
 
     def takes_bands(self, F):
         """Whether one of the partitions' own fp32 products would take the band schedule."""
@@ -367,15 +383,16 @@ class _Stacked(object):
     def run_quantized(self, role, transposed, data, params, segs, bits, out):
         self.product(role, transposed).run_quantized(self._values(role, transposed), data, params, segs, bits, out)
 
-    def same_schedule(self, F, fused, backward):
-        """False where a partition's own product would run as column bands, which a stacked plan does not have."""
-        roles = [("local", backward)]
-        if self.index is None or backward:
-            if not (backward and fused):
-                roles.append(("to", backward and self.index is None))
-        if backward or not fused:
-            roles.append(("remote", backward))
-        return not any(self.product(*r).takes_bands(F) for r in roles)
+    def ready(self, F, fused, backward):
+        """True when the direction's products are there.  False where a partition's own product would run as column bands,
+        which a stacked plan does not have (asked of the parts' plans, so nothing is stacked in vain), or where stacking is
+        refused."""
+        pre = self.index is None
+        roles = [("local", backward, False), ("remote", backward, fused and not backward)]
+        if pre or backward:
+            roles.append(("to", backward and pre, fused and backward))
+        products = [(self.product(role, transposed), packed) for role, transposed, packed in roles]
+        return (not any(not packed and p.takes_bands(F) for p, packed in products)) and all(p.stack() for p, _ in products)
 
     @staticmethod
     def of(world, x, bits, backward=False):
@@ -404,7 +421,7 @@ class _Stacked(object):
             fits = sum(v.numel() for v in values) <= _STACKED_EDGES and "SGNN_SPMM_PART_EDGES" not in os.environ
             have = world._stacked = _Stacked(world, mats, indices) if fits else None
         fused = bits in (2, 4, 8) and x.shape[-1] % 2 == 0
-        if have is not None and not have.same_schedule(x.shape[-1], fused, backward):
+        if have is not None and not have.ready(x.shape[-1], fused, backward):
             return None
         if have is not None:
             for m in mats:

@@ -1791,15 +1791,22 @@ extern "C" int sgnn_spmm_plan_stack(sgnn_spmm_plan *const *parts, int n_parts, s
     }
     SGNN_REQUIRE(M < INT32_MAX && K <= INT32_MAX && nnz <= part_edge_cap(), "M=%lld K=%lld nnz=%lld out of range for one plan",
                  (long long)M, (long long)K, (long long)nnz);
-    std::unique_ptr<sgnn_spmm_plan, int (*)(sgnn_spmm_plan *)> p(new sgnn_spmm_plan(), sgnn_spmm_plan_destroy);
-    p->M = M; p->K = K; p->nnz = nnz;
-    p->long_thresh = parts[0]->long_thresh;
-    p->piece_edges = parts[0]->piece_edges;
-    p->stacked = true;
-    const int rc = plan_stack_impl(p.get(), parts, n_parts, (hipStream_t)stream);
-    if (rc != SGNN_OK) return rc;
-    *out = p.release();
-    return SGNN_OK;
+    // A caller may go on with the parts when there is no memory for the stacked plan: nothing is thrown at it, and no device
+    // error is left behind for its next launch check.
+    int rc = SGNN_OK;
+    try {
+        std::unique_ptr<sgnn_spmm_plan, int (*)(sgnn_spmm_plan *)> p(new sgnn_spmm_plan(), sgnn_spmm_plan_destroy);
+        p->M = M; p->K = K; p->nnz = nnz;
+        p->long_thresh = parts[0]->long_thresh;
+        p->piece_edges = parts[0]->piece_edges;
+        p->stacked = true;
+        rc = plan_stack_impl(p.get(), parts, n_parts, (hipStream_t)stream);
+        if (rc == SGNN_OK) *out = p.release();
+    } catch (const std::bad_alloc &) {
+        rc = fail(SGNN_ERR_HIP, "stacked plan: out of host memory");
+    }
+    if (rc != SGNN_OK) (void)hipGetLastError();
+    return rc;
 }
 
 extern "C" int sgnn_spmm_plan_info(const sgnn_spmm_plan *p, int64_t info[10]) {

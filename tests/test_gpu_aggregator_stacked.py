@@ -164,3 +164,34 @@ def test_a_wrong_number_of_values_is_refused():
     from super_gnn_amd.aggregator import Aggregator
     with pytest.raises(ValueError, match="entries"):
         Aggregator.apply(world, x, 0, 32, True, True)
+
+
+@pytest.mark.parametrize("bits", [32, 4])
+def test_no_stacking_where_the_parts_take_bands(bits, monkeypatch):
+    from super_gnn_amd.supergnn_ops import SpmmPlan
+    monkeypatch.setenv("SGNN_SPMM_BAND", "1")
+    monkeypatch.setattr(SpmmPlan, "stack", classmethod(lambda cls, plans: pytest.fail("stacked in vain")))
+    x = torch.randn(N, 64, generator=torch.Generator(device="cuda").manual_seed(6), device="cuda")
+    _same(_world(3, 64, bits, True, False), x, x.flip(0).contiguous(), bits, True)
+
+
+@pytest.mark.parametrize("error", ["memory", "library", "argument", "thresholds"])
+def test_the_parts_run_where_stacking_is_refused(error, monkeypatch):
+    from super_gnn_amd import _lib
+    from super_gnn_amd.supergnn_ops import SpmmPlan
+    world = _world(3, 64, 32, True, False)
+    if error == "thresholds":
+        m = world.graphs[1].local_adj_t
+        m._plan = SpmmPlan(*m.csr()[:2], m.sparse_size(1), long_row_threshold=4)
+    else:
+        what = {"memory": torch.cuda.OutOfMemoryError, "library": _lib.SgnnError, "argument": ValueError}[error]
+
+        def refuse(cls, plans):
+            raise what("no")
+        monkeypatch.setattr(SpmmPlan, "stack", classmethod(refuse))
+    x = torch.randn(N, 64, generator=torch.Generator(device="cuda").manual_seed(7), device="cuda")
+    for _ in range(2):
+        _same(world, x, x.flip(0).contiguous(), 32, True)
+    outs = world.aggregate(torch.split(x, world.partition_sizes))
+    from super_gnn_amd.aggregator import _world_forward
+    assert all(torch.equal(a, b) for a, b in zip(outs, _world_forward(world, torch.split(x, world.partition_sizes), 32)))
