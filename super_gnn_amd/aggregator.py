@@ -340,6 +340,16 @@ class _Product(object):
         self.plan.run_quantized(self.value, data, params, segs, bits, out, bind=False)
 
 
+def _sizes_fit(g, pre):
+    """Whether the partition's matrices have the row and column counts that place them in a block-diagonal matrix.  One by
+    one, a matrix that nothing is exchanged through is never looked at."""
+    n, sent, received = g.local_adj_t.sparse_size(0), sum(g.comm_splits.send_splits), sum(g.comm_splits.recv_splits)
+    remote = g.adj_t_pre_post_aggr_from if pre else g.remote_adj_t
+    if tuple(g.local_adj_t.sparse_sizes()) != (n, n) or tuple(remote.sparse_sizes()) != (n, received):
+        return False
+    return tuple(g.adj_t_pre_post_aggr_to.sparse_sizes()) == (sent, n) if pre else g.idx_nodes_send_to_others.numel() == sent
+
+
 class _Stacked(object):
     """The partitions of a world as ONE block-diagonal matrix per role, over the node features stacked in partition order
     and the arenas' rows.  A partition of a graph of this size is 10 ... 40 us of work per product, most of it the latency of
@@ -409,7 +419,7 @@ class _Stacked(object):
             if not pre:
                 indices.append(g.idx_nodes_send_to_others)
         for m in mats:
-            value = m.csr()[2]
+            value = None if m is None else m.csr()[2]   # a partition that exchanges nothing need not hold a matrix for it
             if value is None or value.device != x.device or value.dtype != torch.float32:
                 return None
             values.append(value)
@@ -418,7 +428,8 @@ class _Stacked(object):
         indices = [(t, t._version) for t in indices]
         have = world._stacked
         if have is None or not have.made_of(mats, indices):
-            fits = sum(v.numel() for v in values) <= _STACKED_EDGES and "SGNN_SPMM_PART_EDGES" not in os.environ
+            fits = (sum(v.numel() for v in values) <= _STACKED_EDGES and "SGNN_SPMM_PART_EDGES" not in os.environ
+                    and all(_sizes_fit(g, pre) for g in graphs))
             have = world._stacked = _Stacked(world, mats, indices) if fits else None
         fused = bits in (2, 4, 8) and x.shape[-1] % 2 == 0
         if have is not None and not have.ready(x.shape[-1], fused, backward):

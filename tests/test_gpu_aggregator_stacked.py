@@ -195,3 +195,46 @@ def test_the_parts_run_where_stacking_is_refused(error, monkeypatch):
     outs = world.aggregate(torch.split(x, world.partition_sizes))
     from super_gnn_amd.aggregator import _world_forward
     assert all(torch.equal(a, b) for a, b in zip(outs, _world_forward(world, torch.split(x, world.partition_sizes), 32)))
+
+
+@pytest.mark.parametrize("bits", [32, 4])
+@pytest.mark.parametrize("pre,kind", [(True, "missing"), (True, "empty"), (False, "empty")])
+def test_a_partition_without_neighbours(pre, kind, bits):
+    """Nothing is exchanged with the last partition: the matrices it holds for that may be missing or have no rows at all."""
+    from super_gnn_amd import SparseTensor, synth
+    from super_gnn_amd.aggregator import Aggregator, LoopbackWorld, _world_forward
+    from super_gnn_amd.data_manager import build_loopback_partitions
+    n = N // 3
+    rowptr, col = synth.uniform_degree_graph(2 * n, 7, seed=8)
+    rowptr = torch.cat([rowptr, rowptr[-1] + torch.arange(1, n + 1)])
+    col = torch.cat([col, torch.arange(2 * n, 3 * n, dtype=col.dtype)])   # the last third: self loops alone
+    graphs = build_loopback_partitions(rowptr, col, torch.rand(col.numel()), 3, 64, num_bits=bits, is_pre_delay=pre)
+    last = graphs[2]
+    assert sum(last.comm_splits.send_splits) == sum(last.comm_splits.recv_splits) == 0
+    none = torch.zeros(0, dtype=torch.int64, device="cuda")
+    empty = SparseTensor(rowptr=torch.zeros(1, dtype=torch.int64, device="cuda"), col=none, value=none.float(), sparse_sizes=(0, 0))
+    if pre:
+        last.adj_t_pre_post_aggr_to = None if kind == "missing" else empty
+        last.adj_t_pre_post_aggr_from = empty
+    else:
+        last.remote_adj_t = empty
+    world = LoopbackWorld(graphs, bits, pre)
+    x = torch.randn(N, 64, generator=torch.Generator(device="cuda").manual_seed(8), device="cuda")
+    a = x.clone().requires_grad_()
+    out = Aggregator.apply(world, a, 0, bits, pre, True)
+    out.backward(x)
+    assert torch.equal(out, torch.cat(_world_forward(world, torch.split(x, world.partition_sizes), bits)))
+    lone = graphs[2].local_adj_t.csr()[2][:, None] * x[2 * n:]
+    assert torch.equal(out[2 * n:], lone) and torch.equal(a.grad[2 * n:], lone)
+
+
+@pytest.mark.parametrize("dtype", [torch.int64, torch.float64])
+def test_edge_values_of_other_types(dtype):
+    """They are converted for the product, as SPMM_forward does."""
+    from super_gnn_amd.aggregator import Aggregator, LoopbackWorld, _world_forward
+    world = _world(3, 64, 32, True, False)
+    m = world.graphs[1].local_adj_t
+    m._value = (m._value * 8).to(dtype)
+    x = torch.randn(N, 64, generator=torch.Generator(device="cuda").manual_seed(9), device="cuda")
+    out = Aggregator.apply(LoopbackWorld(world.graphs, 32, True), x, 0, 32, True, True)
+    assert torch.equal(out, torch.cat(_world_forward(LoopbackWorld(world.graphs, 32, True), torch.split(x, world.partition_sizes), 32)))
