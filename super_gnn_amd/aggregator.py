@@ -36,7 +36,8 @@ from ._lib import SgnnError
 from .ops.spmm_kernel import (SPMM_backward, SPMM_backward_quantized, SPMM_forward, SPMM_forward_quantized)
 from .quantizer import Quantizer_for_all_procs
 from .sparse import SparseTensor
-from .supergnn_ops import SpmmPlan, _capturing, dequantize_tensor_for_all_procs, quant_segments, quantize_tensor_for_all_procs
+from .supergnn_ops import (SpmmPlan, _capturing, _checked_row_index, dequantize_tensor_for_all_procs, quant_segments,
+                           quantize_tensor_for_all_procs)
 
 
 def _cumulative(splits):
@@ -362,6 +363,8 @@ class _Stacked(object):
         graphs = world.graphs
         self.index = None
         if not world.is_pre_delay:
+            for g, n in zip(graphs, world.partition_sizes):   # past its own rows a partition's index would pick a neighbour's
+                _checked_row_index(g.idx_nodes_send_to_others, n)
             self.index = torch.cat([g.idx_nodes_send_to_others + n0 for g, n0 in zip(graphs, world.node_offsets)])
         # The partitions' segments one after the other: the packed rows then lie where the partitions' own calls put them.
         self.send_range = torch.tensor(_cumulative([k for g in graphs for k in g.comm_splits.send_splits]), dtype=torch.int32)
@@ -423,11 +426,14 @@ class _Stacked(object):
             if value is None or value.device != x.device or value.dtype != torch.float32:
                 return None
             values.append(value)
-        if any(t is None or t.device != x.device for t in indices):
+        if any(t is None or t.device != x.device or t.dtype != torch.int64 or t.dim() != 1 or not t.is_contiguous()
+               or t.is_inference() for t in indices):
             return None
         indices = [(t, t._version) for t in indices]
         have = world._stacked
         if have is None or not have.made_of(mats, indices):
+            if _capturing():
+                return None
             fits = (sum(v.numel() for v in values) <= _STACKED_EDGES and "SGNN_SPMM_PART_EDGES" not in os.environ
                     and all(_sizes_fit(g, pre) for g in graphs))
             have = world._stacked = _Stacked(world, mats, indices) if fits else None

@@ -238,3 +238,16 @@ def test_edge_values_of_other_types(dtype):
     x = torch.randn(N, 64, generator=torch.Generator(device="cuda").manual_seed(9), device="cuda")
     out = Aggregator.apply(LoopbackWorld(world.graphs, 32, True), x, 0, 32, True, True)
     assert torch.equal(out, torch.cat(_world_forward(LoopbackWorld(world.graphs, 32, True), torch.split(x, world.partition_sizes), 32)))
+
+
+@pytest.mark.parametrize("bits", [32, 4])
+@pytest.mark.parametrize("bad", [N // 3, -1])
+def test_boundary_rows_beyond_the_partition_are_refused(bad, bits):
+    """Stacked, such an index would pick a row of another partition."""
+    from super_gnn_amd.aggregator import Aggregator
+    world = _world(3, 64, bits, False, False)
+    x = torch.randn(N, 64, device="cuda")
+    Aggregator.apply(world, x, 0, bits, False, True)
+    world.graphs[1 if bad < 0 else 0].idx_nodes_send_to_others[0] = bad
+    with pytest.raises(IndexError):
+        Aggregator.apply(world, x, 0, bits, False, True)
