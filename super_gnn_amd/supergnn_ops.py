@@ -44,6 +44,15 @@ def _device():
     return torch.device("cuda", torch.cuda.current_device())
 
 
+def _device_index():
+    """The current device's number; without a GPU, the error that says so."""
+    try:
+        return torch.cuda.current_device()
+    except Exception:
+        _device()
+        raise
+
+
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
@@ -384,7 +393,7 @@ def quant_segments(work_range, bits):
     (keyed by its version counter, so in-place edits rebuild them)."""
     _want(work_range, torch.int32, "work_range_per_proc")
     cache = work_range.__dict__.setdefault("_sgnn_segments", {})
-    key = (int(bits), work_range._version, torch.cuda.current_device())
+    key = (int(bits), work_range._version, _device_index())
     s = cache.get(key)
     if s is None:
         cache.clear()
@@ -514,7 +523,7 @@ _SINGLE_SEG = OrderedDict()
 
 
 def _single_segment(n, bits):
-    key = (int(n), int(bits), torch.cuda.current_device())
+    key = (int(n), int(bits), _device_index())
     s = _SINGLE_SEG.get(key)
     if s is None:
         s = _Segments(torch.tensor([0, int(n)], dtype=torch.int32), int(bits), _device())
