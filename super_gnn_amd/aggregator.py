@@ -391,6 +391,10 @@ class _Stacked(object):
         return [m.storage.value_T() if transposed else m.csr()[2] for m in self._matrices(role)]
 
     def run(self, role, transposed, x, out, accumulate):
+        exchanged = 0 if role == "to" and self.index is None else 1
+        for m in self._matrices(role):
+            if role == "local" or m.sparse_size(exchanged):   # one by one, a partition that exchanges nothing skips the product
+                m.note_use(x.shape[-1], transposed)
         self.product(role, transposed).run(self._values(role, transposed), x, out, accumulate)
 
     def run_quantized(self, role, transposed, data, params, segs, bits, out):
@@ -440,9 +444,6 @@ class _Stacked(object):
         fused = bits in (2, 4, 8) and x.shape[-1] % 2 == 0
         if have is not None and not have.ready(x.shape[-1], fused, backward):
             return None
-        if have is not None:
-            for m in mats:
-                m.note_use(x.shape[-1], backward)
         return have
 
     def made_of(self, mats, indices):

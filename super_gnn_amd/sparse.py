@@ -7,7 +7,17 @@ It also owns what this build caches per matrix: the SpMM plans of A and of A^T."
 import numpy as np
 import torch
 
-from .supergnn_ops import SpmmPlan
+from .supergnn_ops import SpmmPlan, _capturing
+
+
+def _split_basis(rowptr, value):
+    from .ops.spmm_kernel import split_basis
+    return split_basis(rowptr, value)
+
+
+def _work_range(row_splits, basis, width):
+    from .ops.spmm_kernel import work_range
+    return work_range(row_splits, basis, width)
 
 
 class _Storage:
@@ -66,6 +76,7 @@ class SparseTensor:
         self._work_range = (torch.empty(0, dtype=torch.int32), torch.empty(0, dtype=torch.int32))
         self._work_range_T = (torch.empty(0, dtype=torch.int32), torch.empty(0, dtype=torch.int32))
         self._used_width = self._used_width_T = None
+        self._split_basis = self._split_basis_T = None
         self._plan = None
         self._plan_T = None
         self.storage = _Storage(self)
@@ -116,34 +127,40 @@ class SparseTensor:
         return out
 
     def note_use(self, width, transposed=False):
-        """A product of this feature width ran on this matrix's behalf (stacked with others): the work range that the
-        façade would have stored is then computed when somebody asks for it."""
+        """A product of this feature width runs on this matrix: what the façade would store as its work range is kept in the
+        cheapest form, and worked out when somebody asks for it.  (Inside a graph capture nothing can be computed now; the
+        next product, or the question itself, takes the values as they are then.)"""
         if transposed:
             self._used_width_T = width
+            if self._split_basis_T is None and self._work_range_T[0].numel() == 0 and not _capturing():
+                self._build_transpose()
+                self._split_basis_T = _split_basis(self._colptr, self._value_T)
         else:
             self._used_width = width
+            if self._split_basis is None and self._work_range[0].numel() == 0 and not _capturing():
+                self._split_basis = _split_basis(self._rowptr, self._value)
 
     def get_work_range(self):
         if self._used_width is not None:
-            from .ops.spmm_kernel import work_range
-            self._work_range = work_range(self._work_range[0], self._rowptr, self._value, self._used_width)
-            self._used_width = None
+            self._work_range = _work_range(self._work_range[0], self._split_basis or _split_basis(self._rowptr, self._value),
+                                           self._used_width)
+            self._used_width = self._split_basis = None
         return self._work_range
 
     def set_work_range(self, row_splits, col_splits):
-        self._used_width = None
+        self._used_width = self._split_basis = None
         self._work_range = (row_splits, col_splits)
 
     def get_work_range_for_transpose(self):
         if self._used_width_T is not None:
-            from .ops.spmm_kernel import work_range
             self._build_transpose()
-            self._work_range_T = work_range(self._work_range_T[0], self._colptr, self._value_T, self._used_width_T)
-            self._used_width_T = None
+            self._work_range_T = _work_range(self._work_range_T[0], self._split_basis_T or _split_basis(self._colptr, self._value_T),
+                                             self._used_width_T)
+            self._used_width_T = self._split_basis_T = None
         return self._work_range_T
 
     def set_work_range_for_transpose(self, row_splits, col_splits):
-        self._used_width_T = None
+        self._used_width_T = self._split_basis_T = None
         self._work_range_T = (row_splits, col_splits)
 
     # ---- cached per-matrix state of this build ----------------------------------------------

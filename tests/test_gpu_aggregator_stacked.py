@@ -251,3 +251,20 @@ def test_boundary_rows_beyond_the_partition_are_refused(bad, bits):
     world.graphs[1 if bad < 0 else 0].idx_nodes_send_to_others[0] = bad
     with pytest.raises(IndexError):
         Aggregator.apply(world, x, 0, bits, False, True)
+
+
+@pytest.mark.parametrize("bits", [32, 4])
+@pytest.mark.parametrize("pre", [False, True])
+def test_work_ranges(pre, bits):
+    """Stacked products leave the work ranges that the partitions' own products leave."""
+    from super_gnn_amd.aggregator import Aggregator, _world_backward, _world_forward
+    one, other = _world(3, 64, bits, pre, False), _world(3, 64, bits, pre, False)
+    x = torch.randn(N, 64, device="cuda", requires_grad=True)
+    Aggregator.apply(one, x, 0, bits, pre, True).sum().backward()
+    rows = torch.split(x.detach(), other.partition_sizes)
+    _world_forward(other, rows, bits)
+    _world_backward(other, rows, bits)
+    for a, b in zip(_mats(one), _mats(other)):
+        for ask in ("get_work_range", "get_work_range_for_transpose"):
+            for got, want in zip(getattr(a, ask)(), getattr(b, ask)()):
+                assert torch.equal(got, want)
