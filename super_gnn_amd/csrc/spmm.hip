@@ -1329,15 +1329,16 @@ struct sgnn_spmm_plan {
     int32_t *col = nullptr;     // device, owned
     // long rows
     int64_t n_long = 0, n_items = 0, long_edges = 0;
+    int64_t regrouped = 0;          // length of col_long and eperm where they are arrays of their own (partitioned)
     int max_cls_items = 0;
     int32_t *long_rows = nullptr;   // [n_long] row ids
     int32_t *long_pbeg = nullptr;   // [n_long + 1] first piece of each long row
-    int32_t *col_long = nullptr;    // [long_edges] columns regrouped by class inside each long row
-    int32_t *eperm = nullptr;       // [long_edges] original edge index of each regrouped edge
-    float *val_long = nullptr;      // [long_edges] bound edge values in regrouped order (sgnn_spmm_plan_bind_values)
+    int32_t *col_long = nullptr;    // [regrouped] columns regrouped by class inside each long row
+    int32_t *eperm = nullptr;       // [regrouped] original edge index of each regrouped edge
+    float *val_long = nullptr;      // [regrouped] bound edge values in regrouped order (sgnn_spmm_plan_bind_values)
     const float *bound_val = nullptr;  // the caller's array val_long was taken from
     int32_t *eslot_csr = nullptr;      // [nnz] row_slot[col[e]] in CSR order (sgnn_spmm_plan_bind_row_slots)
-    int32_t *eslot_long = nullptr;     // [long_edges] the same in regrouped order (partitioned plans)
+    int32_t *eslot_long = nullptr;     // [regrouped] the same in regrouped order (partitioned plans)
     const int32_t *bound_slots = nullptr;  // the caller's table they were taken from
     int4 *cls_work = nullptr;       // [8 * max_cls_items] (piece id, first edge in col_long / eperm, edges, 0) per class, zero-padded
     float *partial = nullptr;       // [n_items * F], grown on demand
@@ -1523,8 +1524,9 @@ static int plan_create_impl(sgnn_spmm_plan *p, const int64_t *rowptr, const void
             DevTmp<int32_t> d_long_off, d_cls_count;
             if ((rc = upload(&d_long_off.p, long_off, st)) != SGNN_OK) return rc;
             SGNN_HIP_CHECK(hipMalloc(&d_cls_count.p, sizeof(int32_t) * (size_t)p->n_long * kNumXCD));
-            SGNN_HIP_CHECK(hipMalloc(&p->col_long, sizeof(int32_t) * (size_t)p->long_edges));
-            SGNN_HIP_CHECK(hipMalloc(&p->eperm, sizeof(int32_t) * (size_t)p->long_edges));
+            p->regrouped = p->long_edges;
+            SGNN_HIP_CHECK(hipMalloc(&p->col_long, sizeof(int32_t) * (size_t)p->regrouped));
+            SGNN_HIP_CHECK(hipMalloc(&p->eperm, sizeof(int32_t) * (size_t)p->regrouped));
             hipLaunchKernelGGL(partition_long_rows_kernel, dim3((uint32_t)p->n_long), dim3(kBlock), 0, st, p->rowptr, p->col,
                                p->long_rows, d_long_off.p, p->col_long, p->eperm, d_cls_count.p);
             cls_count.resize((size_t)p->n_long * kNumXCD);
@@ -1709,6 +1711,7 @@ static int plan_stack_impl(sgnn_spmm_plan *p, sgnn_spmm_plan *const *parts, int 
     }
     if (long_room > INT32_MAX) return fail(SGNN_ERR_ARG, "stacked plans hold at most 2^31 - 1 regrouped edges");
     p->partitioned = any;
+    p->regrouped = any ? long_room : 0;
     p->h_rowptr.assign(1, 0);
     SGNN_HIP_CHECK(hipMalloc(&p->col, sizeof(int32_t) * (size_t)std::max<int64_t>(p->nnz, 1)));
     if (any) {
@@ -1772,7 +1775,6 @@ static int plan_stack_impl(sgnn_spmm_plan *p, sgnn_spmm_plan *const *parts, int 
     SGNN_HIP_CHECK(hipStreamSynchronize(st));
     for (int which = 0; which < 3; ++which)
         if ((rc = build_chunks(p, which, st)) != SGNN_OK) return rc;
-    if (any) p->long_edges = long_room;   // the length of the regrouped arrays, which the bound values and slots share
     return SGNN_OK;
 }
 
@@ -2413,14 +2415,14 @@ extern "C" int sgnn_spmm_plan_bind_values(sgnn_spmm_plan *p, const float *val, s
     p->bound_val = nullptr;
     ++p->bind_gen;  // band schedules refill their value copies on their next use
     if (val == nullptr) return SGNN_OK;
-    if (!p->partitioned || p->long_edges == 0) {  // nothing to regroup for the piece path
+    if (!p->partitioned || p->regrouped == 0) {  // nothing to regroup for the piece path
         p->bound_val = val;
         return SGNN_OK;
     }
-    if (p->val_long == nullptr) SGNN_HIP_CHECK(hipMalloc(&p->val_long, sizeof(float) * (size_t)p->long_edges));
-    const int64_t nb = (p->long_edges + kBlock - 1) / kBlock;
+    if (p->val_long == nullptr) SGNN_HIP_CHECK(hipMalloc(&p->val_long, sizeof(float) * (size_t)p->regrouped));
+    const int64_t nb = (p->regrouped + kBlock - 1) / kBlock;
     hipLaunchKernelGGL(permute_values_kernel, dim3((uint32_t)nb), dim3(kBlock), 0, (hipStream_t)stream, val, p->eperm,
-                       p->val_long, p->long_edges);
+                       p->val_long, p->regrouped);
     SGNN_HIP_CHECK(hipGetLastError());
     p->bound_val = val;
     return SGNN_OK;
@@ -2442,10 +2444,10 @@ extern "C" int sgnn_spmm_plan_bind_row_slots(sgnn_spmm_plan *p, const int32_t *r
     if (p->eslot_csr == nullptr) SGNN_HIP_CHECK(hipMalloc(&p->eslot_csr, sizeof(int32_t) * (size_t)p->nnz));
     hipLaunchKernelGGL(translate_columns_kernel, dim3((uint32_t)((p->nnz + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, p->col,
                        row_slot, p->eslot_csr, p->nnz);
-    if (p->partitioned && p->long_edges > 0) {
-        if (p->eslot_long == nullptr) SGNN_HIP_CHECK(hipMalloc(&p->eslot_long, sizeof(int32_t) * (size_t)p->long_edges));
-        hipLaunchKernelGGL(translate_columns_kernel, dim3((uint32_t)((p->long_edges + kBlock - 1) / kBlock)), dim3(kBlock), 0,
-                           st, p->col_long, row_slot, p->eslot_long, p->long_edges);
+    if (p->partitioned && p->regrouped > 0) {
+        if (p->eslot_long == nullptr) SGNN_HIP_CHECK(hipMalloc(&p->eslot_long, sizeof(int32_t) * (size_t)p->regrouped));
+        hipLaunchKernelGGL(translate_columns_kernel, dim3((uint32_t)((p->regrouped + kBlock - 1) / kBlock)), dim3(kBlock), 0,
+                           st, p->col_long, row_slot, p->eslot_long, p->regrouped);
     }
     SGNN_HIP_CHECK(hipGetLastError());
     p->bound_slots = row_slot;
