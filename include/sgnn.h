@@ -100,6 +100,10 @@ int sgnn_spmm_plan_info(const sgnn_spmm_plan *plan, int64_t info[10]);
  * (super_gnn/ops/csrc/spmm.cpp:502-510). */
 int sgnn_spmm_plan_schedule(const sgnn_spmm_plan *plan, int64_t F, int64_t info[4]);
 
+/* How the row-class schedule walks the short rows for the same operand: info[0] = chunks of short rows, info[1] = dense rows
+ * that a lane group keeps in flight (0: one row behind the other, -1: rows of more than 64 vectors, whose number is fixed). */
+int sgnn_spmm_plan_short_rows(const sgnn_spmm_plan *plan, int64_t F, int64_t info[2]);
+
 /* Optional: declare an edge-value array constant until the next bind.  The plan keeps a copy of the
  * long rows' values in its own (regrouped) edge order, and later sgnn_spmm_csr_f32 /
  * sgnn_spmm_csr_dq*_f32 calls that pass the SAME pointer read that copy contiguously instead of

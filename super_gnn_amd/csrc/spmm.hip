@@ -198,23 +198,6 @@ __device__ __forceinline__ uint32_t group_ballot(bool pred) {
 // Rows per chunk: each of the first nr+1 lanes of the group holds one rowptr entry.
 __host__ __device__ constexpr int chunk_row_limit(int G) { return (G < 32 ? G : 32) - 1; }
 
-// Gathers in flight per lane group of the short-row kernel.  Deep: the whole grid is resident at once and its time is the
-// longest chunk's chain of gathers, one memory latency per U of them.  Otherwise many rounds of waves follow each other, and
-// what counts is the bytes a CU has in flight: lines on their way occupy the XCD's 4 MB L2, and beyond about 64 KB per CU
-// they push out rows that others are about to use (uniform columns, F = 128: 30 k rows x 61 edges U = 1 / 2 / 4 / 8 52 / 55 /
-// 88 / 89 us, 100 k rows x 41 edges 245 / 270 / 280 / 281).  So about 2 KB per wave of 64 lanes.  Packed rows are 4 ... 16
-// times smaller.
-__host__ __device__ constexpr int short_unroll(int G, int NV, int bits, bool deep) {
-    if (NV > 1) return unroll_of(NV);
-    if (bits != 0) return G == 64 ? 8 : 4;
-    if (deep) return 8;
-    return G == 8 ? 8 : G == 16 ? 3 : G == 32 ? 2 : 6;
-}
-// Rows of 512 ... 1024 bytes keep every gather under its lane predicate: each then sits in an exec-mask region of its own
-// with a wait before it, i.e. one row in flight per wave, which is as much as the L2 bears (U = 1 without the predicate: 30 k
-// rows x 61 edges of F = 256 141 -> 152 us, 100 k x 41 535 -> 550).
-__host__ __device__ constexpr bool short_fenced(int G, int NV, int bits, bool deep) { return G == 64 && NV == 1 && bits == 0 && !deep; }
-
 // One lane group walks one chunk of consecutive rows for the feature columns [f_lo, f_hi) (both multiples
 // of VEC).  RP is the row-pointer type: the caller's int64 array, or the 32-bit per-band row pointers of a
 // band schedule.
@@ -356,7 +339,7 @@ __device__ __forceinline__ void short_chunk_body(
     }
 }
 
-template <int VEC, int G, int NV, int BITS, bool DEEP>
+template <int VEC, int G, int NV, int BITS, int U, bool FENCED>
 __global__ __launch_bounds__(kBlock) void spmm_short_kernel(
     const int64_t *__restrict__ rowptr, const int32_t *__restrict__ col, const float *__restrict__ val,
     const DenseSrc dense, float *__restrict__ out, const int4 *__restrict__ chunks, int n_chunks, int F,
@@ -368,7 +351,7 @@ __global__ __launch_bounds__(kBlock) void spmm_short_kernel(
     if (ci >= n_chunks) return;
     // A chunk record is (first row, row count, first edge, edge count): the column/weight loads
     // depend on it alone and are issued before the row pointers come back.
-    short_chunk_body<VEC, G, NV, BITS, int64_t, short_unroll(G, NV, BITS, DEEP), short_fenced(G, NV, BITS, DEEP)>(
+    short_chunk_body<VEC, G, NV, BITS, int64_t, U, FENCED>(
         rowptr, col, val, dense, out, chunks[ci], 0, F, ldo, accumulate, row_div, lig);
 }
 
@@ -1120,12 +1103,17 @@ __global__ __launch_bounds__(kBlock) void band_scatter_kernel(const int64_t *__r
 // ------------------------------------------------------------------------------------------------
 // Launch tables.
 // ------------------------------------------------------------------------------------------------
+struct ShortLoad {
+    int64_t chunks, edges;  // of the short rows
+    int64_t x_bytes;        // the dense operand
+    bool skewed;            // an eighth of the edges or more sit in long rows: a power-law graph, with popular columns
+};
 struct ShortArgs {
     const int64_t *rowptr; const int32_t *col; const float *val; DenseSrc dense; float *out;
     const int4 *chunks; int n_chunks; const int32_t *empty_rows; int n_empty;
     int F; int64_t ldo; int accumulate; const float *row_div;
     bool prof;   // false: no profiling events (the non-allocating entry point creates nothing)
-    int64_t x_bytes;  // the dense operand
+    ShortLoad load;
 };
 struct PieceArgs {
     const int32_t *col_long; const int32_t *eperm; const float *val; float *partial;
@@ -1138,15 +1126,49 @@ struct FinalArgs {
     int F; int64_t ldo; int accumulate; const float *row_div;
 };
 
-// Chunks that the chip holds at once, about: up to here the short-row kernel keeps the larger number of gathers in flight.
-constexpr int kDeepChunks = kChunkGroupsWanted;
+// Gathers in flight per lane group of the short-row kernel over fp32 rows of one vector per lane.  More of them shorten a
+// chunk's chain of memory latencies, which is what a small grid waits for; but lines on their way occupy the XCDs' 4 MB L2s
+// and push out rows that other waves are about to use.  Where the lines lie, with 16-byte lanes, us a product:
+//   * up to about 2048 waves there is nothing to push out: 8 (1500 rows x 40 edges of 200 k columns, F = 128 2 / 8 12.7 / 9.2);
+//   * power-law graphs gather popular rows and stand 8 while there are few chunks (25 k nodes, 200 k edges 2 / 8: F = 128
+//     52 / 47, F = 256 51 / 44); with more chunks 2 at G = 32 (200 k nodes, 4 M edges, F = 100 1 / 2 / 8 205 / 192 / 187,
+//     62 M edges 3.15 / 3.08 / 3.18 ms);
+//   * without popular rows 8 stays right only while the operand is small next to the L2s and the grid resident: F = 80 20 k
+//     rows x 61 edges 2 / 8 38 / 31, F = 128 10 k x 101 31 / 28, but 30 k x 61 55 / 89 and 15 k x 17 11.5 / 15; F = 160
+//     10 k x 33 20.5 / 18.3, 20 k x 17 28 / 26, 20 k nodes in eight blocks x 30 36 / 30, but 30 k x 61 96 / 127; F = 256 5 k
+//     x 61 17.6 / 16.7, but 8 k x 61 23 / 34;
+//   * rows of 512 ... 1024 bytes out of an operand beyond 21 MB stand one at a time (30 k x 61 fenced / 2 / 8: F = 200 114 /
+//     132 / 180, F = 256 141 / 182 / 221), unless the whole product is 256 MB or less (50 k x 5, F = 160 30 / 27 / 27) or a few
+//     chunks gather out of HBM (12 k rows x 30 of 1 M columns, F = 160 39 / 36 / 37; F = 80 2 / 8 25 / 24).
+// kFenced keeps every gather under its lane predicate: each then sits in an exec-mask region of its own, behind a wait for
+// the one before it, so that one row is in flight while the next addresses are ready (1 without the predicate: 30 k x 61 of
+// F = 256 141 -> 152 us, 100 k x 41 540 -> 553).
+constexpr int kFenced = 0;
+static int short_depth(int vec, int G, int F, const ShortLoad &w) {
+    constexpr int64_t kMB = 1000000;
+    const bool few = w.chunks <= kChunkGroupsWanted;   // about what the chip holds at once
+    if (G == 8 || w.chunks * G <= 2048 * 64) return 8;
+    if (G == 16) return few ? 8 : 3;
+    if (vec < 4) return few ? 8 : G == 32 ? 2 : kFenced;
+    if (w.skewed) return few ? 8 : G == 32 ? 2 : kFenced;
+    if (G == 32) return (few && w.x_bytes > 256 * kMB) || (w.chunks <= 10240 && w.x_bytes <= 8 * kMB) ? 8 : 2;
+    if (!few) return kFenced;
+    if (w.x_bytes > 256 * kMB || (F <= 160 ? w.x_bytes <= 13 * kMB : w.chunks <= 5120 && w.x_bytes <= 8 * kMB)) return 8;
+    return w.x_bytes <= 21 * kMB || w.edges * F * 4 <= 256 * kMB ? 2 : kFenced;
+}
 
 // Unused LDS that a workgroup of the short-row kernel asks for so that four of them fit a CU: a dense operand beyond the
 // 256 MB Infinity Cache is gathered from HBM, and there 32 KB in flight per CU are enough; more only lowers the L2's hit rate
 // (62 M-edge power-law graph, F = 128, U = 2: 3.37 -> 3.09 ms; 1 M uniform columns x 17 edges 1.30 -> 1.24 ms, F = 64 0.69 ->
 // 0.66; 80 MB operand: 0.20 -> 0.24 ms, so not there).
-static uint32_t short_spare_lds(int bits, int G, int NV, int64_t x_bytes) {
-    return bits == 0 && NV == 1 && (G == 16 || G == 32) && x_bytes > (256ll << 20) ? 40000 : 0;
+static uint32_t short_spare_lds(int G, int64_t x_bytes) {
+    return (G == 16 || G == 32) && x_bytes > (256ll << 20) ? 40000 : 0;
+}
+
+template <int VEC, int G, int NV, int BITS, int U, bool FENCED = false>
+static void launch_short(const ShortArgs &a, uint32_t nb, uint32_t lds, hipStream_t st) {
+    hipLaunchKernelGGL((spmm_short_kernel<VEC, G, NV, BITS, U, FENCED>), dim3(nb), dim3(kBlock), lds, st, a.rowptr, a.col, a.val,
+                       a.dense, a.out, a.chunks, a.n_chunks, a.F, a.ldo, a.accumulate, a.row_div, nb);
 }
 
 // Up to about the eight L2s together (32 MB), the long rows' partial sums are kept in them from the piece kernel to the final sum.
@@ -1188,13 +1210,19 @@ static void launch_all(const ShortArgs &a, const PieceArgs &s, const FinalArgs &
     if (a.n_chunks > 0) {
         const uint32_t nb = (uint32_t)((a.n_chunks + GPB - 1) / GPB);
         ProfScope prof(BITS == 0 ? K_SPMM_SHORT : K_FUSED_SHORT, st, a.prof);
-        constexpr bool kHasDeep = short_unroll(G, NV, BITS, true) != short_unroll(G, NV, BITS, false);
-        if (kHasDeep && a.n_chunks <= kDeepChunks)
-            hipLaunchKernelGGL((spmm_short_kernel<VEC, G, NV, BITS, kHasDeep>), dim3(nb), dim3(kBlock), 0, st, a.rowptr, a.col,
-                               a.val, a.dense, a.out, a.chunks, a.n_chunks, a.F, a.ldo, a.accumulate, a.row_div, nb);
-        else
-            hipLaunchKernelGGL((spmm_short_kernel<VEC, G, NV, BITS, false>), dim3(nb), dim3(kBlock), short_spare_lds(BITS, G, NV, a.x_bytes),
-                               st, a.rowptr, a.col, a.val, a.dense, a.out, a.chunks, a.n_chunks, a.F, a.ldo, a.accumulate, a.row_div, nb);
+        if constexpr (NV > 1) launch_short<VEC, G, NV, BITS, unroll_of(NV)>(a, nb, 0, st);
+        else if constexpr (BITS != 0) launch_short<VEC, G, NV, BITS, G == 64 ? 8 : 4>(a, nb, 0, st);   // packed rows are 4 ... 16 times smaller
+        else {
+            const int u = short_depth(VEC, G, a.F, a.load);
+            const uint32_t spare = u == 8 ? 0 : short_spare_lds(G, a.load.x_bytes);
+            if (u == 8) launch_short<VEC, G, NV, 0, 8>(a, nb, spare, st);
+            else if constexpr (G == 16) launch_short<VEC, G, NV, 0, 3>(a, nb, spare, st);
+            else if constexpr (G == 32) launch_short<VEC, G, NV, 0, 2>(a, nb, spare, st);
+            else if constexpr (G == 64) {
+                if (u == kFenced) launch_short<VEC, G, NV, 0, 6, true>(a, nb, spare, st);
+                else if constexpr (VEC == 4) launch_short<VEC, G, NV, 0, 2>(a, nb, spare, st);
+            }
+        }
     }
     if (a.n_empty > 0 && (!a.accumulate || a.row_div)) {
         const uint32_t nb = (uint32_t)((a.n_empty + GPB * kEmptyRowsPerGroup - 1) / (GPB * kEmptyRowsPerGroup));
@@ -2287,6 +2315,23 @@ static int64_t slice_width(int64_t F, int64_t K) {
     return ((F + n - 1) / n + 3) / 4 * 4;
 }
 
+// Power-law graphs of 5 k to 2.45 M nodes hold 14 ... 69 % of their edges in long rows.
+static ShortLoad short_load(const sgnn_spmm_plan *p, int64_t chunks, int64_t F) {
+    return ShortLoad{chunks, p->nnz - p->long_edges, p->K * F * 4, p->long_edges * 8 >= p->nnz};
+}
+
+extern "C" int sgnn_spmm_plan_short_rows(const sgnn_spmm_plan *p, int64_t F, int64_t info[2]) {
+    SGNN_REQUIRE(p != nullptr && info != nullptr, "null argument");
+    SGNN_REQUIRE(F > 0 && F < (1 << 24), "feature width F=%lld out of range", (long long)F);
+    if (!p->parts.empty()) p = p->parts[0];
+    const int vec = F % 4 == 0 ? 4 : F % 2 == 0 ? 2 : 1;
+    if (vec == 4) F = std::min(F, slice_width(F, p->K));
+    const int nvec = (int)(F / vec), gw = group_width(nvec);
+    info[0] = p->n_chunks[gw == 8 ? 0 : gw == 16 ? 1 : 2];
+    info[1] = nvec > 64 ? -1 : short_depth(vec, gw, (int)F, short_load(p, info[0], F));
+    return SGNN_OK;
+}
+
 static int spmm_run(sgnn_spmm_plan *p, const float *val, const DenseSrc &dense, int bits, float *out, int64_t F,
                     int64_t ldo, int accumulate, const float *row_div, hipStream_t st, float *scratch = nullptr,
                     size_t scratch_floats = 0, bool is_slice = false) {
@@ -2379,7 +2424,7 @@ static int spmm_run(sgnn_spmm_plan *p, const float *val, const DenseSrc &dense, 
     SGNN_REQUIRE(p->n_chunks[which] >= 0, "plan has no chunk list for this feature width (plan creation failed?)");
     ShortArgs a{p->rowptr, p->col, val, dense, out, p->chunks[which], (int)p->n_chunks[which], p->empty_rows,
                 (int)p->n_empty, (int)F, ldo, accumulate, row_div, scratch == nullptr,
-                bits == 0 ? p->K * F * 4 : p->K * F * bits / 8};
+                short_load(p, p->n_chunks[which], F)};
     PieceArgs s{p->col_long, p->eperm, val, partial, p->cls_work, p->max_cls_items, (int)F, keep_partials(p->n_items, F)};
     if (val != nullptr && val == p->bound_val && p->val_long != nullptr) {
         s.eperm = nullptr;   // values already sit in regrouped order: contiguous reads, no indirection

@@ -165,6 +165,12 @@ class SpmmPlan:
         check(lib.sgnn_spmm_plan_schedule(self._h, int(F), buf))
         return dict(zip(("band", "band_cols", "n_bands", "n_slices"), list(buf)))
 
+    def short_rows(self, F):
+        """Chunks of short rows, and the dense rows a lane group keeps in flight (sgnn_spmm_plan_short_rows)."""
+        buf = (ctypes.c_int64 * 2)()
+        check(lib.sgnn_spmm_plan_short_rows(self._h, int(F), buf))
+        return tuple(buf)
+
     def run(self, value, mat, out, accumulate=True, row_div=None, bind=True):
         """out (+)= A @ mat on the current stream.  value None = all ones.  bind False: the caller binds the values itself."""
         _want(mat, torch.float32, "mat")
