@@ -1160,9 +1160,10 @@ static int short_depth(int vec, int G, int F, const ShortLoad &w) {
 // Unused LDS that a workgroup of the short-row kernel asks for so that four of them fit a CU: a dense operand beyond the
 // 256 MB Infinity Cache is gathered from HBM, and there 32 KB in flight per CU are enough; more only lowers the L2's hit rate
 // (62 M-edge power-law graph, F = 128, U = 2: 3.37 -> 3.09 ms; 1 M uniform columns x 17 edges 1.30 -> 1.24 ms, F = 64 0.69 ->
-// 0.66; 80 MB operand: 0.20 -> 0.24 ms, so not there).
-static uint32_t short_spare_lds(int G, int64_t x_bytes) {
-    return (G == 16 || G == 32) && x_bytes > (256ll << 20) ? 40000 : 0;
+// 0.66; 80 MB operand: 0.20 -> 0.24 ms, so not there).  Narrower lanes at G = 32 have less in flight as it is (2.45 M x 13,
+// F = 50 1.50 -> 1.91 ms, F = 29 1.12 -> 1.49; at G = 16 F = 30 1.21 -> 1.16).
+static uint32_t short_spare_lds(int vec, int G, int64_t x_bytes) {
+    return ((vec >= 2 && G == 16) || (vec == 4 && G == 32)) && x_bytes > (256ll << 20) ? 40000 : 0;
 }
 
 template <int VEC, int G, int NV, int BITS, int U, bool FENCED = false>
@@ -1214,7 +1215,7 @@ static void launch_all(const ShortArgs &a, const PieceArgs &s, const FinalArgs &
         else if constexpr (BITS != 0) launch_short<VEC, G, NV, BITS, G == 64 ? 8 : 4>(a, nb, 0, st);   // packed rows are 4 ... 16 times smaller
         else {
             const int u = short_depth(VEC, G, a.F, a.load);
-            const uint32_t spare = u == 8 ? 0 : short_spare_lds(G, a.load.x_bytes);
+            const uint32_t spare = u == 8 ? 0 : short_spare_lds(VEC, G, a.load.x_bytes);
             if (u == 8) launch_short<VEC, G, NV, 0, 8>(a, nb, spare, st);
             else if constexpr (G == 16) launch_short<VEC, G, NV, 0, 3>(a, nb, spare, st);
             else if constexpr (G == 32) launch_short<VEC, G, NV, 0, 2>(a, nb, spare, st);
