@@ -1140,6 +1140,11 @@ struct FinalArgs {
 //   * rows of 512 ... 1024 bytes out of an operand beyond 21 MB stand one at a time (30 k x 61 fenced / 2 / 8: F = 200 114 /
 //     132 / 180, F = 256 141 / 182 / 221), unless the whole product is 256 MB or less (50 k x 5, F = 160 30 / 27 / 27) or a few
 //     chunks gather out of HBM (12 k rows x 30 of 1 M columns, F = 160 39 / 36 / 37; F = 80 2 / 8 25 / 24).
+// With narrower lanes an instruction brings a half or a quarter of the bytes, and rows end before 512:
+//   * two floats, G = 64: 4, that is 2 KB per wave (fenced / 2 / 4 / 8: 200 k power-law nodes, F = 90 252 / 211 / 194 / 190, 100 k x 41
+//     256 / 238 / 241 / 242; only uniform graphs at 114 ... 126 floats lose, 100 k x 41 of F = 126 311 -> 326); G = 32 2 (100 k x 41,
+//     F = 50 2 / 4 136 / 147);
+//   * one float: 8 (200 k power-law nodes, F = 29 2 / 8 143 / 123, F = 33 fenced / 8 158 / 150; 100 k x 41 105 / 99, 130 / 121).
 // kFenced keeps every gather under its lane predicate: each then sits in an exec-mask region of its own, behind a wait for
 // the one before it, so that one row is in flight while the next addresses are ready (1 without the predicate: 30 k x 61 of
 // F = 256 141 -> 152 us, 100 k x 41 540 -> 553).
@@ -1147,9 +1152,10 @@ constexpr int kFenced = 0;
 static int short_depth(int vec, int G, int F, const ShortLoad &w) {
     constexpr int64_t kMB = 1000000;
     const bool few = w.chunks <= kChunkGroupsWanted;   // about what the chip holds at once
-    if (G == 8 || w.chunks * G <= 2048 * 64) return 8;
+    if (G == 8 || vec == 1 || w.chunks * G <= 2048 * 64) return 8;
+    if (vec == 2 && G == 64) return few && w.skewed ? 8 : 4;
     if (G == 16) return few ? 8 : 3;
-    if (vec < 4) return few ? 8 : G == 32 ? 2 : kFenced;
+    if (vec == 2) return few ? 8 : 2;
     if (w.skewed) return few ? 8 : G == 32 ? 2 : kFenced;
     if (G == 32) return (few && w.x_bytes > 256 * kMB) || (w.chunks <= 10240 && w.x_bytes <= 8 * kMB) ? 8 : 2;
     if (!few) return kFenced;
@@ -1217,11 +1223,12 @@ static void launch_all(const ShortArgs &a, const PieceArgs &s, const FinalArgs &
             const int u = short_depth(VEC, G, a.F, a.load);
             const uint32_t spare = u == 8 ? 0 : short_spare_lds(VEC, G, a.load.x_bytes);
             if (u == 8) launch_short<VEC, G, NV, 0, 8>(a, nb, spare, st);
-            else if constexpr (G == 16) launch_short<VEC, G, NV, 0, 3>(a, nb, spare, st);
-            else if constexpr (G == 32) launch_short<VEC, G, NV, 0, 2>(a, nb, spare, st);
-            else if constexpr (G == 64) {
-                if (u == kFenced) launch_short<VEC, G, NV, 0, 6, true>(a, nb, spare, st);
-                else if constexpr (VEC == 4) launch_short<VEC, G, NV, 0, 2>(a, nb, spare, st);
+            else if constexpr (VEC > 1 && G == 16) launch_short<VEC, G, NV, 0, 3>(a, nb, spare, st);
+            else if constexpr (VEC > 1 && G == 32) launch_short<VEC, G, NV, 0, 2>(a, nb, spare, st);
+            else if constexpr (VEC == 2 && G == 64) launch_short<VEC, G, NV, 0, 4>(a, nb, spare, st);
+            else if constexpr (VEC == 4 && G == 64) {
+                if (u == 2) launch_short<VEC, G, NV, 0, 2>(a, nb, spare, st);
+                else launch_short<VEC, G, NV, 0, 6, true>(a, nb, spare, st);
             }
         }
     }

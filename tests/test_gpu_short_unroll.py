@@ -66,8 +66,9 @@ DEGREES = [1, 33, 0, 7, 64, 128, 2, 31, 65, 8, 16, 0, 100, 3, 32, 40]
 # The row counts stand on both sides of the dispatch's lines: 2048 waves, 10240, 16384 chunks, and the operand's size.
 FORMS = [(400, 500, DEGREES, 0, F, 8) for F in (20, 33, 64, 66, 100, 160, 256)] + [
     (60000, 500, DEGREES, 0, 20, 8), (60000, 500, DEGREES, 0, 64, 3), (60000, 500, DEGREES, 0, 100, 2), (60000, 500, DEGREES, 0, 128, 2),
-    (60000, 500, DEGREES, 0, 132, 0), (60000, 500, DEGREES, 0, 256, 0), (60000, 500, DEGREES, 0, 50, 2), (60000, 500, DEGREES, 0, 33, 0),
-    (60000, 500, DEGREES, 0, 66, 0), (60000, 500, DEGREES, 0, 30, 3), (60000, 500, DEGREES, 0, 13, 3), (60000, 500, DEGREES, 0, 29, 2),
+    (60000, 500, DEGREES, 0, 132, 0), (60000, 500, DEGREES, 0, 256, 0), (60000, 500, DEGREES, 0, 50, 2), (60000, 500, DEGREES, 0, 33, 8),
+    (60000, 500, DEGREES, 0, 66, 4), (60000, 500, DEGREES, 0, 30, 3), (60000, 500, DEGREES, 0, 13, 8), (60000, 500, DEGREES, 0, 29, 8),
+    (15000, 500, [17], 0, 66, 4), (15000, 500, [17], 0, 50, 8), (12000, 500, [17], 12, 66, 8), (60000, 500, DEGREES, 60, 90, 4),
     (9000, 15000, [17], 0, 128, 8), (9000, 16000, [17], 0, 128, 2), (15000, 500, [17], 0, 128, 2),
     (15000, 20000, [17], 0, 160, 8), (15000, 21000, [17], 0, 160, 2), (15000, 500, [17], 0, 164, 2), (5000, 7000, [17], 0, 256, 8),
     (5000, 9000, [17], 0, 256, 2), (15000, 20000, [17], 0, 256, 2), (16000, 22000, [17], 0, 256, 0), (14000, 22000, [17], 0, 256, 2),
