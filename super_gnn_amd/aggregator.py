@@ -264,9 +264,26 @@ def _world_backward(world, grads, bits, out_all=None):
     return outs
 
 
-# Up to this many edges (local, send and receive side) the partitions' matrices are also kept stacked as one, which
-# costs a second plan (about 12 bytes per edge and direction).  Beyond it a partition fills the chip by itself.
+# Up to this many edges (local, send and receive side) the partitions' matrices may also be kept stacked as one, which
+# costs a second plan (about 12 bytes per edge and direction).
 _STACKED_EDGES = 1 << 25
+
+
+def _worth_stacking(P, edges, F, separate):
+    """Stacking saves launches and the wait for each partition's longest row, P - 1 times; a partition of more work fills the
+    chip by itself, and its own operand stays in the caches better than all of them together.  What counts is the floats
+    that a partition's edges gather.  One pass in both directions, one by one -> stacked, us (power-law graphs, fp32): 64 M floats
+    a partition P = 8 1619 -> 903, P = 4 810 -> 508; 128 M P = 4 978 -> 709, P = 2 487 -> 417; 256 M P = 8 3738 -> 3551, P = 4 1744 ->
+    1683, P = 2 626 -> 572, but in pre/post mode 625 -> 623 and at int2 599 -> 624; 512 M P = 8 7424 -> 8078, P = 4 3448 -> 3637, P = 2
+    1324 -> 1361.
+    ``separate`` partitions come and go as tensors of their own, which costs two more passes over all rows: P = 8 64 M 1613 ->
+    1108, P = 4 64 M 813 -> 631, 128 M 978 -> 894 (uniform graph, 82 M: 2552 -> 2925); P = 2 509 -> 560 already at 51 M."""
+    floats = edges // P * F
+    if separate:
+        return P >= 4 and floats <= 80_000_000
+    return floats <= min(P, 4) << 26
+
+
 _BAND_SWITCHES = ("SGNN_SPMM_BAND", "SGNN_SPMM_BAND_COLS", "SGNN_SPMM_BAND_KB", "SGNN_SPMM_BAND_SLICES", "SGNN_SPMM_BAND_WINDOW")
 
 
@@ -412,7 +429,7 @@ class _Stacked(object):
         return (not any(not packed and p.takes_bands(F) for p, packed in products)) and all(p.stack() for p, _ in products)
 
     @staticmethod
-    def of(world, x, bits, backward=False):
+    def of(world, x, bits, backward=False, separate=False):
         """The world's stacked matrices, or None where the partitions run one by one.  They are made anew when a partition's
         matrix is replaced by another one, or its boundary index is replaced or edited."""
         graphs, pre = world.graphs, world.is_pre_delay
@@ -433,13 +450,15 @@ class _Stacked(object):
         if any(t is None or t.device != x.device or t.dtype != torch.int64 or t.dim() != 1 or not t.is_contiguous()
                or t.is_inference() for t in indices):
             return None
+        edges = sum(v.numel() for v in values)
+        if edges > _STACKED_EDGES or not _worth_stacking(len(graphs), edges, x.shape[-1], separate):
+            return None
         indices = [(t, t._version) for t in indices]
         have = world._stacked
         if have is None or not have.made_of(mats, indices):
             if _capturing():
                 return None
-            fits = (sum(v.numel() for v in values) <= _STACKED_EDGES and "SGNN_SPMM_PART_EDGES" not in os.environ
-                    and all(_sizes_fit(g, pre) for g in graphs))
+            fits = "SGNN_SPMM_PART_EDGES" not in os.environ and all(_sizes_fit(g, pre) for g in graphs)
             have = world._stacked = _Stacked(world, mats, indices) if fits else None
         fused = bits in (2, 4, 8) and x.shape[-1] % 2 == 0
         if have is not None and not have.ready(x.shape[-1], fused, backward):
@@ -531,7 +550,7 @@ def _per_partition(world, rows, together, one_by_one):
     sizes = world.partition_sizes
     if len(rows) == len(sizes) and all(r.dim() == 2 and r.is_cuda and r.dtype == torch.float32 and r.shape[1] == rows[0].shape[1]
                                        and r.shape[0] == n and r.device == rows[0].device for r, n in zip(rows, sizes)):
-        stacked = _Stacked.of(world, rows[0], world.num_bits, backward=together is _stacked_backward)
+        stacked = _Stacked.of(world, rows[0], world.num_bits, backward=together is _stacked_backward, separate=True)
         if stacked is not None:
             x = torch.cat(rows)
             out = torch.empty_like(x)

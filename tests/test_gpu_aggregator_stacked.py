@@ -268,3 +268,21 @@ def test_work_ranges(pre, bits):
         for ask in ("get_work_range", "get_work_range_for_transpose"):
             for got, want in zip(getattr(a, ask)(), getattr(b, ask)()):
                 assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("P,F,separate,stacked", [(2, 64, False, True), (2, 64, True, False), (8, 64, True, True)])
+def test_worlds_that_are_stacked(P, F, separate, stacked, monkeypatch):
+    """Two partitions that come as tensors of their own are not worth the copies."""
+    from super_gnn_amd.aggregator import Aggregator, _world_forward, _worth_stacking
+    from super_gnn_amd.supergnn_ops import SpmmPlan
+    made, stack = [], SpmmPlan.stack
+    monkeypatch.setattr(SpmmPlan, "stack", classmethod(lambda cls, plans: made.append(1) or stack(plans)))
+    world = _world(P, F, 32, True, False)
+    x = torch.randn(N, F, device="cuda")
+    rows = torch.split(x, world.partition_sizes)
+    out = torch.cat(world.aggregate(rows)) if separate else Aggregator.apply(world, x, 0, 32, True, True)
+    assert torch.equal(out, torch.cat(_world_forward(world, rows, 32))) and bool(made) == stacked
+    # by the floats that a partition's edges gather
+    assert _worth_stacking(8, 4_000_000, 128, False) and not _worth_stacking(8, 32_000_000, 128, False)
+    assert _worth_stacking(2, 2_000_000, 128, False) and not _worth_stacking(2, 4_000_000, 128, False)
+    assert _worth_stacking(8, 4_000_000, 128, True) and not _worth_stacking(8, 8_000_000, 128, True)
