@@ -291,7 +291,7 @@ class _Product(object):
     """The block-diagonal matrix of the partitions' matrices (or of their transposes): one plan made of the parts' plans.  The
     edge values are gathered from the partitions' own tensors at every call, so that an edit counts here whenever it counts
     in the partitions' own products: in place, through ``.data``, between the replays of a captured graph (eight partitions of
-    25 k nodes, forward and backward: 696 -> 743 us; a copy made once would answer with old values)."""
+    25 k nodes, forward and backward: 697 -> 728 us; a copy made once would answer with old values)."""
 
     def __init__(self, plans):
         self.plans = plans
@@ -358,6 +358,10 @@ class _Product(object):
         self.plan.run_quantized(self.value, data, params, segs, bits, out, bind=False)
 
 
+def _values(mats, transposed):
+    return [m.storage.value_T() if transposed else m.csr()[2] for m in mats]
+
+
 def _sizes_fit(g, pre):
     """Whether the partition's matrices have the row and column counts that place them in a block-diagonal matrix.  One by
     one, a matrix that nothing is exchanged through is never looked at."""
@@ -396,26 +400,13 @@ class _Stacked(object):
             return [g.adj_t_pre_post_aggr_from if pre else g.remote_adj_t for g in graphs]
         return [g.adj_t_pre_post_aggr_to if pre else _scatter_matrix(g, g.local_adj_t.sparse_size(0)) for g in graphs]
 
-    def product(self, role, transposed=False):
+    def _product(self, role, transposed, mats):
         """The role's product, made anew when a partition's plan is another one."""
-        plans = [m.spmm_plan_T() if transposed else m.spmm_plan() for m in self._matrices(role)]
+        plans = [m.spmm_plan_T() if transposed else m.spmm_plan() for m in mats]
         p = self.products.get((role, transposed))
         if p is None or any(a is not b for a, b in zip(p.plans, plans)):
             p = self.products[(role, transposed)] = _Product(plans)
         return p
-
-    def _values(self, role, transposed):
-        return [m.storage.value_T() if transposed else m.csr()[2] for m in self._matrices(role)]
-
-    def run(self, role, transposed, x, out, accumulate):
-        exchanged = 0 if role == "to" and self.index is None else 1
-        for m in self._matrices(role):
-            if role == "local" or m.sparse_size(exchanged):   # one by one, a partition that exchanges nothing skips the product
-                m.note_use(x.shape[-1], transposed)
-        self.product(role, transposed).run(self._values(role, transposed), x, out, accumulate)
-
-    def run_quantized(self, role, transposed, data, params, segs, bits, out):
-        self.product(role, transposed).run_quantized(self._values(role, transposed), data, params, segs, bits, out)
 
     def ready(self, F, fused, backward):
         """True when the direction's products are there.  False where a partition's own product would run as column bands,
@@ -425,8 +416,26 @@ class _Stacked(object):
         roles = [("local", backward, False), ("remote", backward, fused and not backward)]
         if pre or backward:
             roles.append(("to", backward and pre, fused and backward))
-        products = [(self.product(role, transposed), packed) for role, transposed, packed in roles]
-        return (not any(not packed and p.takes_bands(F) for p, packed in products)) and all(p.stack() for p, _ in products)
+        self.at_hand = {}
+        for role, transposed, packed in roles:
+            mats = self._matrices(role)
+            p = self.at_hand[role] = self._product(role, transposed, mats), mats, transposed
+            if not packed and p[0].takes_bands(F):
+                return False
+        return all(p.stack() for p, _, _ in self.at_hand.values())
+
+    def run(self, role, x, out, accumulate):
+        """One product of the direction that ready() was asked for."""
+        product, mats, transposed = self.at_hand[role]
+        exchanged = 0 if role == "to" and self.index is None else 1
+        for m in mats:
+            if role == "local" or m.sparse_size(exchanged):   # one by one, a partition that exchanges nothing skips the product
+                m.note_use(x.shape[-1], transposed)
+        product.run(_values(mats, transposed), x, out, accumulate)
+
+    def run_quantized(self, role, data, params, segs, bits, out):
+        product, mats, transposed = self.at_hand[role]
+        product.run_quantized(_values(mats, transposed), data, params, segs, bits, out)
 
     @staticmethod
     def of(world, x, bits, backward=False, separate=False):
@@ -483,23 +492,23 @@ def _stacked_forward(world, stacked, x, bits, out):
     with torch.cuda.stream(side):
         if rows:
             if stacked.index is None:
-                stacked.run("to", False, x, arena.send, False)
+                stacked.run("to", x, arena.send, False)
             elif not quantized:
                 torch.index_select(x, 0, stacked.index, out=arena.send)
             if quantized:
                 quantize_tensor_for_all_procs(x if stacked.index is not None else arena.send, arena.send_q, arena.send_params,
                                               stacked.send_range, stacked.segments, bits, row_index=stacked.index)
             arena.exchange("forward", quantized)
-    stacked.run("local", False, x, out, False)
+    stacked.run("local", x, out, False)
     main.wait_stream(side)
     if not rows:
         return
     if fused:
-        stacked.run_quantized("remote", False, arena.recv_q, arena.recv_params, quant_segments(stacked.recv_range, bits), bits, out)
+        stacked.run_quantized("remote", arena.recv_q, arena.recv_params, quant_segments(stacked.recv_range, bits), bits, out)
     else:
         if quantized:
             dequantize_tensor_for_all_procs(arena.recv_q, arena.recv, arena.recv_params, stacked.recv_range, stacked.segments, bits)
-        stacked.run("remote", False, arena.recv, out, True)
+        stacked.run("remote", arena.recv, out, True)
 
 
 def _stacked_backward(world, stacked, grad, bits, out):
@@ -514,21 +523,20 @@ def _stacked_backward(world, stacked, grad, bits, out):
     side.wait_stream(main)
     with torch.cuda.stream(side):
         if rows:
-            stacked.run("remote", True, grad, arena.recv, False)
+            stacked.run("remote", grad, arena.recv, False)
             if quantized:
                 quantize_tensor_for_all_procs(arena.recv, arena.recv_q, arena.recv_params, stacked.recv_range, stacked.segments, bits)
             arena.exchange("backward", quantized)
-    stacked.run("local", True, grad, out, False)
+    stacked.run("local", grad, out, False)
     main.wait_stream(side)
     if not rows:
         return
     if quantized and not fused:
         dequantize_tensor_for_all_procs(arena.send_q, arena.send, arena.send_params, stacked.send_range, stacked.segments, bits)
-    transposed = stacked.index is None
     if fused:
-        stacked.run_quantized("to", transposed, arena.send_q, arena.send_params, quant_segments(stacked.send_range, bits), bits, out)
+        stacked.run_quantized("to", arena.send_q, arena.send_params, quant_segments(stacked.send_range, bits), bits, out)
     else:
-        stacked.run("to", transposed, arena.send, out, True)
+        stacked.run("to", arena.send, out, True)
 
 
 class LoopbackAggregator(torch.autograd.Function):
