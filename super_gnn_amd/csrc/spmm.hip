@@ -875,9 +875,11 @@ __global__ __launch_bounds__(kBlock) void spmm_hubrow_lds_kernel(
 
 // ------------------------------------------------------------------------------------------------
 // Long rows, step 2: add a row's piece partials in piece order, epilogue, store.  A row's time is its chain of batches of UP
-// partials.  KEEP: the partials of the whole product are few enough (keep_partials) to stay in the L2s, written and read with
-// ordinary accesses instead of streaming ones: 200 k power-law nodes, F = 100 18.8 -> 14.2 us, fused 1 M rows 28.1 -> 20.0;
-// beyond that they only push dense rows out (1 M nodes, 32 M edges: the product 1.41 -> 1.47 ms, UP = 16 as well as 8).
+// partials.  KEEP: the partials of the whole product are few (keep_partials), written and read with ordinary accesses instead of
+// streaming ones and sixteen at a time: 200 k power-law nodes, F = 100 18.8 -> 14.2 us, fused 1 M rows 28.1 -> 20.0.  The reader
+// finds few of them in its own L2 either way (18 MB fetched of 18, hit rate 0.13 against 0.27: a row's pieces come from up to
+// eight XCDs), so they are taken to stay in the Infinity Cache.  More of them only push dense rows out (1 M nodes, 32 M edges:
+// the product 1.41 -> 1.47 ms, UP = 16 as well as 8).
 // ------------------------------------------------------------------------------------------------
 template <int VEC, int G, int NV, bool KEEP>
 __global__ __launch_bounds__(kBlock) void spmm_long_final_kernel(
@@ -1178,7 +1180,8 @@ static void launch_short(const ShortArgs &a, uint32_t nb, uint32_t lds, hipStrea
                        a.dense, a.out, a.chunks, a.n_chunks, a.F, a.ldo, a.accumulate, a.row_div, nb);
 }
 
-// Up to about the eight L2s together (32 MB), the long rows' partial sums are kept in them from the piece kernel to the final sum.
+// Long rows' partial sums written and read with ordinary accesses (see spmm_long_final_kernel): 18 MB (200 k nodes, 4 M edges,
+// F = 100) and 22 MB (the fused product) gain 5 and 8 us, the products of 32 M and 62 M edges lose 4 and 1 %.
 static int keep_partials(int64_t n_items, int64_t F) { return n_items * F * 4 <= (40ll << 20); }
 
 template <int VEC, int G, int NV, int BITS>
