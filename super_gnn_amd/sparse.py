@@ -15,9 +15,9 @@ def _split_basis(rowptr, value):
     return split_basis(rowptr, value)
 
 
-def _work_range(row_splits, basis, width):
+def _work_range(row_splits, basis, rowptr, width):
     from .ops.spmm_kernel import work_range
-    return work_range(row_splits, basis, width)
+    return work_range(row_splits, basis, rowptr, width)
 
 
 class _Storage:
@@ -143,7 +143,7 @@ class SparseTensor:
     def get_work_range(self):
         if self._used_width is not None:
             self._work_range = _work_range(self._work_range[0], self._split_basis or _split_basis(self._rowptr, self._value),
-                                           self._used_width)
+                                           self._rowptr, self._used_width)
             self._used_width = self._split_basis = None
         return self._work_range
 
@@ -155,7 +155,7 @@ class SparseTensor:
         if self._used_width_T is not None:
             self._build_transpose()
             self._work_range_T = _work_range(self._work_range_T[0], self._split_basis_T or _split_basis(self._colptr, self._value_T),
-                                             self._used_width_T)
+                                             self._colptr, self._used_width_T)
             self._used_width_T = self._split_basis_T = None
         return self._work_range_T
 

@@ -40,7 +40,12 @@ def _check(device):
         assert ask()[0] is rows and ask()[1].tolist() == [0, 8]
 
 
-def test_split_of_the_first_product():
+@pytest.mark.parametrize("large", [False, True])
+def test_split_of_the_first_product(large, monkeypatch):
+    if large:   # the form that keeps the prefix sums
+        basis = spmm_kernel.split_basis
+        monkeypatch.setattr(spmm_kernel, "split_basis",
+                            lambda rowptr, value: (*basis(rowptr, value)[:1], None, spmm_kernel.row_prefix(rowptr, value)))
     _check("cpu")
 
 
