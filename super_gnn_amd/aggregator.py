@@ -288,14 +288,12 @@ _BAND_SWITCHES = ("SGNN_SPMM_BAND", "SGNN_SPMM_BAND_COLS", "SGNN_SPMM_BAND_KB", 
 
 
 class _Product(object):
-    """The block-diagonal matrix of the partitions' matrices (or of their transposes): one plan made of the parts' plans.  The
-    edge values are gathered from the partitions' own tensors at every call, so that an edit counts here whenever it counts
-    in the partitions' own products: in place, through ``.data``, between the replays of a captured graph (eight partitions of
-    25 k nodes, forward and backward: 697 -> 728 us; a copy made once would answer with old values)."""
+    """The block-diagonal matrix of the partitions' matrices (or of their transposes): one plan made of the parts' plans."""
 
     def __init__(self, plans):
         self.plans = plans
         self.plan = None        # the stacked plan, made by stack()
+        self.value = None       # the edge values: this product's piece of the direction's space (_Stacked.ready)
         self._refused = False
         self._bound = self._seen = None   # [(values, version, hand binds of the part's plan)] as in SpmmPlan._maybe_bind
         self._bands = {}
@@ -309,7 +307,6 @@ class _Product(object):
                 return False
             try:
                 plan = SpmmPlan.stack(self.plans)
-                self.value = torch.empty(plan.nnz, dtype=torch.float32, device=plan.device)
                 self._regrouped = bool(plan.info()["partitioned"])
                 self.plan = plan
             except (ValueError, SgnnError, torch.cuda.OutOfMemoryError):
@@ -325,15 +322,18 @@ class _Product(object):
             self._bands[key] = any(p.schedule(F)["band"] for p in self.plans)
         return self._bands[key]
 
-    def _gather(self, values):
-        for v, p in zip(values, self.plans):
-            if v.numel() != p.nnz:
-                raise ValueError(f"value has {v.numel()} entries, the matrix has {p.nnz}")
-        torch.cat(values, out=self.value)
+    def move(self, value):
+        """Another place for the edge values."""
+        if self._bound is not None:
+            self.plan.unbind_values()
+        self._bound = self._seen = None
+        self.value = value
+
+    def _bind(self, values):
+        """Long rows are read in the plan's own edge order from their second unchanged use on, on the terms of the partitions'
+        plans: unchanged is the same address and version; binding or unbinding a part's plan by hand starts over."""
         if not self._regrouped:
             return   # every product reads self.value itself
-        # Long rows are read in the plan's own edge order from their second unchanged use on, on the terms of the partitions'
-        # plans: unchanged is the same address and version; binding or unbinding a part's plan by hand starts over.
         now = [(v, v._version, p.hand_binds) for v, p in zip(values, self.plans)]
         if self._bound is not None and any(a[2] != b[2] for a, b in zip(self._bound, now)):
             self.plan.unbind_values()
@@ -350,11 +350,11 @@ class _Product(object):
         return then is not None and all(a[0].data_ptr() == b[0].data_ptr() and a[1:] == b[1:] for a, b in zip(then, now))
 
     def run(self, values, x, out, accumulate):
-        self._gather(values)
+        self._bind(values)
         self.plan.run(self.value, x, out, accumulate=accumulate, bind=False)
 
     def run_quantized(self, values, data, params, segs, bits, out):
-        self._gather(values)
+        self._bind(values)
         self.plan.run_quantized(self.value, data, params, segs, bits, out, bind=False)
 
 
@@ -377,10 +377,14 @@ class _Stacked(object):
     and the arenas' rows.  A partition of a graph of this size is 10 ... 40 us of work per product, most of it the latency of
     the longest row and of the launches, P times in a row; stacked, the P products are one launch sequence that fills the
     chip (eight partitions of 25 k nodes, int2, forward and backward: 2.02 -> 0.75 ms; two of 100 k: 1.18 -> 1.01).  The rows
-    get the sums that the partitions' own products give them."""
+    get the sums that the partitions' own products give them.
+
+    The edge values are gathered from the partitions' own tensors in every pass, so that an edit counts here whenever it
+    counts in the partitions' own products: in place, through ``.data``, between the replays of a captured graph.  (Eight
+    partitions of 25 k nodes, forward and backward: 701 -> 729 us against a copy made once, which would answer with old values.)"""
 
     def __init__(self, world, mats, indices):
-        self.world, self.mats, self.indices, self.products = world, mats, indices, {}
+        self.world, self.mats, self.indices, self.products, self.spaces = world, mats, indices, {}, {}
         graphs = world.graphs
         self.index = None
         if not world.is_pre_delay:
@@ -419,23 +423,46 @@ class _Stacked(object):
         self.at_hand = {}
         for role, transposed, packed in roles:
             mats = self._matrices(role)
-            p = self.at_hand[role] = self._product(role, transposed, mats), mats, transposed
-            if not packed and p[0].takes_bands(F):
+            p = self._product(role, transposed, mats)
+            if not packed and p.takes_bands(F):
                 return False
-        return all(p.stack() for p, _, _ in self.at_hand.values())
+            self.at_hand[role] = p, mats, transposed, _values(mats, transposed)
+        if not all(p.stack() for p, *_ in self.at_hand.values()):
+            return False
+        return self._gather(backward)
+
+    def _gather(self, backward):
+        """The edge values of the direction's products into one space, each product's after the other's."""
+        products = [p for p, *_ in self.at_hand.values()]
+        have, space = self.spaces.get(backward, ((), None))
+        if len(have) != len(products) or any(a is not b for a, b in zip(have, products)):
+            if _capturing():
+                return False
+            space = torch.empty(sum(p.plan.nnz for p in products), dtype=torch.float32, device=products[0].plan.device)
+            for p, piece in zip(products, torch.split(space, [p.plan.nnz for p in products])):
+                p.move(piece)
+            self.spaces[backward] = products, space
+        everything = []
+        for p, _, _, values in self.at_hand.values():
+            for v, plan in zip(values, p.plans):
+                if v.numel() != plan.nnz:
+                    raise ValueError(f"value has {v.numel()} entries, the matrix has {plan.nnz}")
+            everything.extend(values)
+        torch.cat(everything, out=space)
+        return True
 
     def run(self, role, x, out, accumulate):
         """One product of the direction that ready() was asked for."""
-        product, mats, transposed = self.at_hand[role]
+        product, mats, transposed, values = self.at_hand[role]
         exchanged = 0 if role == "to" and self.index is None else 1
         for m in mats:
             if role == "local" or m.sparse_size(exchanged):   # one by one, a partition that exchanges nothing skips the product
                 m.note_use(x.shape[-1], transposed)
-        product.run(_values(mats, transposed), x, out, accumulate)
+        product.run(values, x, out, accumulate)
 
     def run_quantized(self, role, data, params, segs, bits, out):
-        product, mats, transposed = self.at_hand[role]
-        product.run_quantized(_values(mats, transposed), data, params, segs, bits, out)
+        product, _, _, values = self.at_hand[role]
+        product.run_quantized(values, data, params, segs, bits, out)
 
     @staticmethod
     def of(world, x, bits, backward=False, separate=False):
