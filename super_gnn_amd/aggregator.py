@@ -674,6 +674,8 @@ class LoopbackWorld(object):
     reference's bf16 wire format (communicator.py:283-294) from the quantizer to the consumer; None
     keeps them fp32."""
 
+    _stacked = None   # (on the class: a world saved by an earlier version comes back without it)
+
     def __init__(self, graphs: Sequence[object], num_bits: int, is_pre_delay: bool, params_wire_dtype=None) -> None:
         self.graphs = list(graphs)
         self.num_bits = int(num_bits)
@@ -685,7 +687,6 @@ class LoopbackWorld(object):
         self._current = None
         self._side = None
         self._in_degrees = None
-        self._stacked = None
 
     def arena(self, F, device, bits=None):
         """Buffers are kept per feature width and exchange format; the partitions' buffer attributes are

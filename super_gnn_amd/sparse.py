@@ -47,6 +47,10 @@ class _Storage:
 
 
 class SparseTensor:
+    # (on the class: a matrix saved by an earlier version comes back without them)
+    _used_width = _used_width_T = None
+    _split_basis = _split_basis_T = None
+
     def __init__(self, row=None, rowptr=None, col=None, value=None, sparse_sizes=None, is_sorted=False):
         if col is None:
             raise ValueError("col is required")
@@ -75,8 +79,6 @@ class SparseTensor:
         self._colptr = self._row_T = self._value_T = None
         self._work_range = (torch.empty(0, dtype=torch.int32), torch.empty(0, dtype=torch.int32))
         self._work_range_T = (torch.empty(0, dtype=torch.int32), torch.empty(0, dtype=torch.int32))
-        self._used_width = self._used_width_T = None
-        self._split_basis = self._split_basis_T = None
         self._plan = None
         self._plan_T = None
         self.storage = _Storage(self)

@@ -69,3 +69,20 @@ def test_prefix_in_slabs(slab):
     value = (value * 16).round()   # whole numbers: every order of the sums is exact
     whole = torch.cat([torch.zeros(1, dtype=torch.float64), value.double().cumsum(0)])[rowptr]
     assert torch.equal(spmm_kernel.row_prefix(rowptr, value, slab), whole)
+
+
+def test_matrices_and_worlds_saved_before_these_attributes():
+    """Objects unpickled from files of an earlier version hold none of the attributes that came later."""
+    import copy
+    from super_gnn_amd.aggregator import LoopbackWorld
+    m = copy.deepcopy(_matrix())
+    for name in ("_used_width", "_used_width_T", "_split_basis", "_split_basis_T"):
+        m.__dict__.pop(name, None)
+    assert m.get_work_range()[0].numel() == 0
+    m.note_use(16)
+    assert m.get_work_range()[1].tolist() == [0, 16]
+    m.note_use(16, transposed=True)
+    assert m.get_work_range_for_transpose()[1].tolist() == [0, 16]
+    world = LoopbackWorld([], 32, False)
+    world.__dict__.pop("_stacked", None)
+    assert world._stacked is None
