@@ -1,6 +1,7 @@
 """The partitions' stacked matrices against the partitions one by one: the same floats, for every exchange format, both
-modes, widths with and without the fused remote step, graphs without and with long rows (hubs in some partitions only, so
-that regrouped and plain long rows meet in one stacked plan)."""
+modes, widths with and without the fused remote step, graphs without and with long rows.  (At these sizes every long row is
+regrouped; test_gpu_plan_stack.py mixes regrouped and plain ones.)  Then what the stacked form must not change: edits of the
+values, bound or not, seen by a version counter or not; partitions that stacking does not fit; what is refused."""
 import pytest
 import torch
 
@@ -41,7 +42,8 @@ def test_stacked_equals_one_by_one(P, F, bits, pre):
         x = torch.randn(N, F, generator=g, device="cuda")
         grad = torch.randn(N, F, generator=g, device="cuda")
         got, want = _both(world, x, grad, bits, pre)
-        assert world._stacked is not None
+        # both directions took the stacked products: the first side of the comparison is not the second one again
+        assert all(world._stacked.products["local", back].plan is not None and back in world._stacked.spaces for back in (False, True))
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
@@ -53,6 +55,7 @@ def test_edited_values_are_seen():
     world.graphs[1].local_adj_t.csr()[2].mul_(2)
     got, want = _both(world, x, grad, 32, True)
     assert torch.equal(got[0], want[0]) and not torch.equal(got[0], before[0])
+    assert torch.equal(got[1], want[1]) and torch.equal(got[1], before[1])   # the transposed values are a copy of their own
 
 
 def _mats(world):
