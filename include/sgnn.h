@@ -77,7 +77,8 @@ int sgnn_spmm_plan_destroy(sgnn_spmm_plan *plan);
  * other, so that P small products become one call.  The parts' index arrays are copied (the parts may be
  * destroyed).  A row gets the sum, bit for bit, that its own plan's row-class schedule gives it; the stacked plan
  * never takes the band schedule.  Edge values are those of the parts, concatenated.  Refused (SGNN_ERR_ARG): parts
- * that are held as row blocks, or themselves stacked, or whose edges together do not fit one plan.
+ * that are held as row blocks, or themselves stacked, or whose long-row thresholds differ, or whose edges together do
+ * not fit one plan; without memory for it SGNN_ERR_HIP, and no device error stays behind: the parts are as they were.
  * Synchronises the stream. */
 int sgnn_spmm_plan_stack(sgnn_spmm_plan *const *parts, int n_parts, sgnn_stream_t stream, sgnn_spmm_plan **plan_out);
 
