@@ -376,8 +376,8 @@ class _Stacked(object):
     """The partitions of a world as ONE block-diagonal matrix per role, over the node features stacked in partition order
     and the arenas' rows.  A partition of a graph of this size is 10 ... 40 us of work per product, most of it the latency of
     the longest row and of the launches, P times in a row; stacked, the P products are one launch sequence that fills the
-    chip (eight partitions of 25 k nodes, int2, forward and backward: 2.02 -> 0.75 ms; two of 100 k: 1.18 -> 1.01).  The rows
-    get the sums that the partitions' own products give them.
+    chip (eight partitions of 25 k nodes, int2, forward and backward: 2.01 -> 0.73 ms).  The rows get the sums that the
+    partitions' own products give them.
 
     The edge values are gathered from the partitions' own tensors in every pass, so that an edit counts here whenever it
     counts in the partitions' own products: in place, through ``.data``, between the replays of a captured graph.  (Eight
