@@ -101,6 +101,12 @@ int sgnn_spmm_plan_info(const sgnn_spmm_plan *plan, int64_t info[10]);
  * (super_gnn/ops/csrc/spmm.cpp:502-510). */
 int sgnn_spmm_plan_schedule(const sgnn_spmm_plan *plan, int64_t F, int64_t info[4]);
 
+/* The tile schedule, which matrices with many edges per block of rows and columns take instead of the band schedule: 15
+ * wavefronts of a workgroup keep info[0] rows each in registers (0: the product does not take it) while the dense operand
+ * streams through LDS.  Same order of operations, so the same bits.  info[1] = edge streams the plan holds (one per number
+ * of rows, two at most; built on the first call that wants one). */
+int sgnn_spmm_plan_tiles(const sgnn_spmm_plan *plan, int64_t F, int64_t info[2]);
+
 /* How the row-class schedule walks the short rows for the same operand: info[0] = chunks of short rows, info[1] = dense rows
  * that a lane group keeps in flight (0: one row behind the other, -1: rows of more than 64 vectors, whose number is fixed). */
 int sgnn_spmm_plan_short_rows(const sgnn_spmm_plan *plan, int64_t F, int64_t info[2]);

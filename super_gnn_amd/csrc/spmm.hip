@@ -1299,6 +1299,8 @@ static int dispatch_shape_dq(int vec, int nvec, const ShortArgs &a, const PieceA
 
 }  // namespace sgnn
 
+#include "spmm_tile.hpp"
+
 using namespace sgnn;
 
 static int env_int(const char *name, int dflt) {
@@ -1358,6 +1360,20 @@ struct BandSchedule {
     }
 };
 
+// The edges as the tile schedule's streams, for one number of rows per wave (see spmm_tile.hpp).
+struct TileSchedule {
+    int rows_per_wave = 0, tiles = 0;
+    int64_t n_rb = 0, batches = 0;     // row blocks, batches of all streams
+    int32_t *stream = nullptr;         // [batches * 32] words and values, kTileSlack bytes beyond
+    int32_t *batch0 = nullptr;         // [n_rb * kTileConsumers] each wave's first batch
+    int32_t *slot_edge = nullptr;      // [batches * kTileBatch] CSR index of every slot, -1: padding
+    uint64_t val_gen = 0;              // plan bind generation the values were filled under (0: not from a bound array)
+    uint64_t last_use = 0;
+    ~TileSchedule() {
+        (void)hipFree(stream); (void)hipFree(batch0); (void)hipFree(slot_edge);
+    }
+};
+
 struct sgnn_spmm_plan {
     int device = 0;
     int64_t M = 0, K = 0, nnz = 0;
@@ -1389,6 +1405,8 @@ struct sgnn_spmm_plan {
     int cols_sorted = -1;           // -1 unknown, 0 some row's columns are out of order, 1 every row is column-sorted
     uint64_t bind_gen = 1;          // bumped by every sgnn_spmm_plan_bind_values
     std::vector<BandSchedule *> bands;
+    std::vector<TileSchedule *> tiles;
+    double tile_spread = 0.0;       // batches of the row blocks' longest streams over their average (0: not known)
     float *band_xs = nullptr;       // the dense operand restaged slice by slice (see band_restage_kernel), grown on demand
     size_t band_xs_floats = 0;
     // A matrix with 2^31 edges or more is held as consecutive row blocks, each a plan of its own with fewer
@@ -1460,6 +1478,7 @@ extern "C" int sgnn_spmm_plan_destroy(sgnn_spmm_plan *p) {
     (void)hipFree(p->empty_rows);
     for (int i = 0; i < 3; ++i) (void)hipFree(p->chunks[i]);
     for (BandSchedule *b : p->bands) delete b;
+    for (TileSchedule *t : p->tiles) delete t;
     (void)hipFree(p->band_xs);
     delete p;
     return SGNN_OK;
@@ -2179,6 +2198,23 @@ static void launch_fill_or_divide(float *out, int64_t M, int F, int64_t ldo, con
     else hipLaunchKernelGGL((rows_fill_or_divide_kernel<VEC, false>), dim3(nb), dim3(kBlock), 0, st, out, M, F, ldo, row_div);
 }
 
+// The workspace for a restaged operand of `floats` floats; *ok is false when there is no room.
+static int grow_xs(sgnn_spmm_plan *root, size_t floats, bool *ok) {
+    SGNN_HIP_CHECK(hipDeviceSynchronize());  // the old workspace may still be read by queued work
+    (void)hipFree(root->band_xs);
+    root->band_xs = nullptr;
+    root->band_xs_floats = 0;
+    root->xs_serial = 0;
+    *ok = hipMalloc(&root->band_xs, floats * sizeof(float)) == hipSuccess;
+    if (!*ok) {
+        (void)hipGetLastError();
+        root->band_xs = nullptr;
+        return SGNN_OK;
+    }
+    root->band_xs_floats = floats;
+    return SGNN_OK;
+}
+
 // The product through the band schedule.  may_build = false (the non-allocating entry point): use a schedule
 // only if an earlier call has built it; *done tells whether the product was carried out here.
 static int spmm_run_band(sgnn_spmm_plan *p, const BandWindows &bw, const float *val, const DenseSrc &dense, float *out, int64_t F,
@@ -2215,17 +2251,9 @@ static int spmm_run_band(sgnn_spmm_plan *p, const BandWindows &bw, const float *
             p->bands.push_back(bs);
         }
         if (xs_floats > root->band_xs_floats) {
-            SGNN_HIP_CHECK(hipDeviceSynchronize());  // the old workspace may still be read by queued work
-            (void)hipFree(root->band_xs);
-            root->band_xs = nullptr;
-            root->band_xs_floats = 0;
-            root->xs_serial = 0;
-            if (hipMalloc(&root->band_xs, xs_floats * sizeof(float)) != hipSuccess) {
-                (void)hipGetLastError();
-                root->band_xs = nullptr;
-                return SGNN_OK;   // no room for the restaged operand: the row-class schedule runs
-            }
-            root->band_xs_floats = xs_floats;
+            bool ok = false;
+            const int rc = grow_xs(root, xs_floats, &ok);
+            if (rc != SGNN_OK || !ok) return rc;   // no room for the restaged operand: the row-class schedule runs
         }
     }
     const bool weighted = val != nullptr;
@@ -2297,13 +2325,183 @@ static int spmm_run_band(sgnn_spmm_plan *p, const BandWindows &bw, const float *
     return SGNN_OK;
 }
 
+// ------------------------------------------------------------------------------------------------
+// Tile schedule, host side.
+// ------------------------------------------------------------------------------------------------
+constexpr double kTileSpread = 1.25;   // see tile_build
+constexpr int kMaxTileSchedules = 2;   // row counts a plan keeps streams for (12 bytes per edge each)
+
+// Estimated time of a product, in clocks of the chip: the rounds of workgroups times the tiles of a sweep times the clocks
+// of a tile, which go with its edges (240 edges of 104 columns 1480 clocks, 640 2950, 4800 20800) down to what the stream
+// of tiles takes.
+static double tile_clocks(const sgnn_spmm_plan *p, int64_t F, int rows) {
+    const double tiles = (double)((p->K + kTileCols - 1) / kTileCols), slices = (double)((F + 63) / 64);
+    const double blocks = (double)((p->M + (int64_t)rows * kTileConsumers - 1) / ((int64_t)rows * kTileConsumers));
+    const double e = (double)p->nnz / (double)p->M * rows * kTileConsumers / tiles;
+    return std::ceil(blocks * slices / 256.0) * tiles * std::max(1200.0, std::max(600.0 + 3.7 * e, 4.3 * e));
+}
+
+// How the tile schedule would take a product of width F: rows per wave, 0 where it is not the one to use as far as the shape
+// of the matrix tells.
+static int tile_rows(const sgnn_spmm_plan *p, int64_t F) {
+    if (p->stacked || p->nnz == 0 || p->M == 0 || p->cols_sorted == 0 || p->K > (int64_t)kTileMax * kTileCols) return 0;
+    const int mode = env_int("SGNN_SPMM_BAND", -1);
+    if (mode == 0 || mode == 1) return 0;
+    // (below a density of 1 / 2000 the stream of the operand alone takes longer than the other schedules)
+    if (mode < 2 && (p->tile_spread > kTileSpread || (double)p->nnz * 2000.0 < (double)p->M * (double)p->K)) return 0;
+    // One chain of fmas per row: where the row classes would take the product, which add up long rows in parts, only if there
+    // are none (a chain of 370 edges is off by 3.0e-7, the parts by 1.3e-7).
+    if (mode < 2 && p->long_edges > 0 && !band_wanted(p, F, band_window_shape(p, 0, (int)F, true, F > kBandWindowCols))) return 0;
+    const double others = 0.9 * 8.9 * (double)p->nnz * (double)F / 64.0 / 256.0;   // band schedule: 8.9 clocks per edge of 64 floats and CU
+    if (mode < 2 && (double)((p->K + kTileCols - 1) / kTileCols) * 1200.0 > others) return 0;
+    int best = kTileRows;
+    for (int r = kTileRows; r >= 16; r -= 3)
+        if (tile_clocks(p, F, r) < 0.97 * tile_clocks(p, F, best)) best = r;
+    return mode > 1 || tile_clocks(p, F, best) < others ? best : 0;
+}
+
+static int tile_build(sgnn_spmm_plan *p, int rows, hipStream_t st, TileSchedule **out) {
+    std::unique_ptr<TileSchedule> ts(new TileSchedule());
+    ts->rows_per_wave = rows;
+    ts->tiles = (int)((p->K + kTileCols - 1) / kTileCols);
+    ts->n_rb = (p->M + (int64_t)rows * kTileConsumers - 1) / ((int64_t)rows * kTileConsumers);
+    const int64_t waves = ts->n_rb * kTileConsumers;
+    DevTmp<int32_t> counts;   // batches of each wave
+    SGNN_BAND_ALLOC(&counts.p, sizeof(int32_t) * (size_t)waves);
+    hipLaunchKernelGGL(tile_count_kernel, dim3((uint32_t)waves), dim3(kBlock), sizeof(int) * (size_t)ts->tiles, st, p->rowptr, p->col, p->M,
+                       rows, ts->tiles, counts.p);
+    SGNN_HIP_CHECK(hipGetLastError());
+    std::vector<int32_t> h, first((size_t)waves);
+    const int rc = download(h, counts.p, (size_t)waves, st);
+    if (rc != SGNN_OK) return rc;
+    int64_t longest = 0;
+    for (int64_t b = 0; b < ts->n_rb; ++b) {
+        int32_t most = 0;
+        for (int w = 0; w < kTileConsumers; ++w) {
+            const size_t i = (size_t)(b * kTileConsumers + w);
+            first[i] = (int32_t)ts->batches;
+            ts->batches += h[i];
+            most = std::max(most, h[i]);
+        }
+        longest += most;
+    }
+    p->tile_spread = (double)longest * kTileConsumers / (double)ts->batches;
+    // a workgroup takes as long as its longest stream: rows of very different lengths are not for this schedule
+    if (ts->batches > (INT32_MAX >> 5) || (p->tile_spread > kTileSpread && env_int("SGNN_SPMM_BAND", -1) < 2)) {
+        p->tile_spread = 1e9;
+        return SGNN_OK;
+    }
+    SGNN_BAND_ALLOC(&ts->stream, (size_t)ts->batches * (8 * kTileBatch) + kTileSlack);
+    SGNN_BAND_ALLOC(&ts->slot_edge, sizeof(int32_t) * (size_t)ts->batches * kTileBatch);
+    SGNN_BAND_ALLOC(&ts->batch0, sizeof(int32_t) * (size_t)waves);
+    SGNN_HIP_CHECK(hipMemcpyAsync(ts->batch0, first.data(), sizeof(int32_t) * (size_t)waves, hipMemcpyHostToDevice, st));
+    hipLaunchKernelGGL(tile_build_kernel, dim3((uint32_t)waves), dim3(64), 2 * sizeof(int) * (size_t)ts->tiles, st, p->rowptr, p->col, p->M,
+                       rows, ts->tiles, ts->batch0, counts.p, ts->stream, ts->slot_edge);
+    SGNN_HIP_CHECK(hipGetLastError());
+    SGNN_HIP_CHECK(hipStreamSynchronize(st));
+    *out = ts.release();
+    return SGNN_OK;
+}
+
+// The product through the tile schedule; as spmm_run_band.
+static int spmm_run_tile(sgnn_spmm_plan *p, int rows, const float *val, const DenseSrc &dense, float *out, int64_t F, int64_t ldo,
+                         int accumulate, const float *row_div, hipStream_t st, bool may_build, bool *done) {
+    *done = false;
+    sgnn_spmm_plan *root = p->whole ? p->whole : p;
+    const int n_slices = (int)((F + 63) / 64);
+    const size_t xs_floats = (size_t)n_slices * (size_t)p->K * 64 + kTileCols * 64;   // the last tile may reach beyond the last row
+    TileSchedule *ts = nullptr;
+    for (TileSchedule *c : p->tiles)
+        if (c->rows_per_wave == rows) ts = c;
+    if (ts == nullptr || xs_floats > root->band_xs_floats) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (may_build) SGNN_HIP_CHECK(hipStreamIsCapturing(st, &cap));
+        if (!may_build || cap != hipStreamCaptureStatusNone) {   // nothing can be built: the streams of another row count do
+            if (ts == nullptr && !p->tiles.empty()) ts = p->tiles[0];
+            if (ts == nullptr || xs_floats > root->band_xs_floats) return SGNN_OK;
+        }
+    }
+    if (ts == nullptr) {
+        bool sorted = false;
+        int rc = band_rows_sorted(p, st, &sorted);
+        if (rc != SGNN_OK) return rc;
+        if (!sorted) return SGNN_OK;
+        if (p->tiles.size() >= (size_t)kMaxTileSchedules) {
+            SGNN_HIP_CHECK(hipDeviceSynchronize());   // queued launches may still read it
+            const size_t victim = p->tiles[0]->last_use < p->tiles[1]->last_use ? 0 : 1;
+            delete p->tiles[victim];
+            p->tiles.erase(p->tiles.begin() + (long)victim);
+        }
+        rc = tile_build(p, rows, st, &ts);
+        if (rc == SGNN_ERR_HIP && band_build_out_of_memory()) return SGNN_OK;   // no room: the other schedules run
+        if (rc != SGNN_OK) return rc;
+        if (ts == nullptr) return SGNN_OK;
+        p->tiles.push_back(ts);
+    }
+    if (xs_floats > root->band_xs_floats) {
+        bool ok = false;
+        const int rc = grow_xs(root, xs_floats, &ok);
+        if (rc != SGNN_OK || !ok) return rc;
+    }
+    const bool bound = val != nullptr && val == p->bound_val;
+    if (val != nullptr && !(bound && ts->val_gen == p->bind_gen)) {
+        const int64_t slots = ts->batches * kTileBatch;
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        SGNN_HIP_CHECK(hipStreamIsCapturing(st, &cap));
+        hipLaunchKernelGGL(tile_values_kernel, dim3((uint32_t)((slots + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, val, ts->slot_edge,
+                           ts->stream, slots);
+        ts->val_gen = bound && cap == hipStreamCaptureStatusNone ? p->bind_gen : 0;   // (a captured launch has not run)
+    }
+    if (p->whole == nullptr) ++root->call_serial;
+    ts->last_use = ++root->band_use_clock;
+    // the restaged operand of this layout is told from a band schedule's by its slice count's sign
+    if (!(root->xs_serial == root->call_serial && root->xs_F == (int)F && root->xs_slices == -n_slices)) {
+        ProfScope prof(K_SPMM_BAND_RESTAGE, st, may_build);
+        const int64_t n = (int64_t)n_slices * p->K * 16;
+        hipLaunchKernelGGL(band_restage_kernel, dim3((uint32_t)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, dense.x, dense.ldx,
+                           root->band_xs, p->K, (int)F, 64, 64, n_slices);
+        root->xs_serial = root->call_serial;
+        root->xs_F = (int)F; root->xs_slice_pad = 64; root->xs_slices = -n_slices;
+    }
+    auto kernel = val ? spmm_tile_kernel<true> : spmm_tile_kernel<false>;
+    {
+        static std::mutex mu;
+        static bool lds_allowed[kMaxDevices][2];
+        std::lock_guard<std::mutex> lock(mu);
+        bool &allowed = lds_allowed[p->device % kMaxDevices][val != nullptr];
+        if (!allowed) {
+            SGNN_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kTileLds));
+            allowed = true;
+        }
+    }
+    {
+        ProfScope prof(K_SPMM_BAND, st, may_build);
+        const int64_t total = ts->n_rb * n_slices;
+        const TileArgs a{root->band_xs, p->K, ts->stream, ts->batch0, out, row_div, p->M, ldo, ts->tiles, ts->rows_per_wave,
+                         (int)ts->n_rb, n_slices, (int)F, accumulate};
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)((total + kNumXCD - 1) / kNumXCD * kNumXCD)), dim3(1024), kTileLds, st, a);
+    }
+    SGNN_HIP_CHECK(hipGetLastError());
+    *done = true;
+    return SGNN_OK;
+}
+
 extern "C" int sgnn_spmm_plan_schedule(const sgnn_spmm_plan *p, int64_t F, int64_t info[4]) {
     SGNN_REQUIRE(p != nullptr && info != nullptr, "null argument");
     SGNN_REQUIRE(F > 0 && F < (1 << 24), "feature width F=%lld out of range", (long long)F);
     if (!p->parts.empty()) p = p->parts[0];  // row blocks decide one by one; the first one's answer is reported
     const BandWindows bw = band_windows(p, F, true);
-    info[0] = (band_wanted(p, F, bw.w[0]) && p->cols_sorted != 0) ? 1 : 0;
+    info[0] = ((band_wanted(p, F, bw.w[0]) || tile_rows(p, F) > 0) && p->cols_sorted != 0) ? 1 : 0;
     info[1] = bw.w[0].band_cols; info[2] = bw.w[0].n_bands; info[3] = bw.total_slices;
+    return SGNN_OK;
+}
+
+extern "C" int sgnn_spmm_plan_tiles(const sgnn_spmm_plan *p, int64_t F, int64_t info[2]) {
+    SGNN_REQUIRE(p != nullptr && info != nullptr, "null argument");
+    SGNN_REQUIRE(F > 0 && F < (1 << 24), "feature width F=%lld out of range", (long long)F);
+    if (!p->parts.empty()) p = p->parts[0];
+    info[0] = tile_rows(p, F);
+    info[1] = (int64_t)p->tiles.size();
     return SGNN_OK;
 }
 
@@ -2385,6 +2583,12 @@ static int spmm_run(sgnn_spmm_plan *p, const float *val, const DenseSrc &dense, 
         vec = 2;
     }
     if (bits == 0 && !is_slice) {
+        const int tr = tile_rows(p, F);
+        if (tr > 0) {
+            bool done = false;
+            const int rc = spmm_run_tile(p, tr, val, dense, out, F, ldo, accumulate, row_div, st, scratch == nullptr, &done);
+            if (rc != SGNN_OK || done) return rc;
+        }
         const BandWindows bw = band_windows(p, F, ldo % 2 == 0 && aligned(out, 8));
         if (band_wanted(p, F, bw.w[0])) {
             bool done = false;

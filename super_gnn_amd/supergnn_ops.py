@@ -165,6 +165,12 @@ class SpmmPlan:
         check(lib.sgnn_spmm_plan_schedule(self._h, int(F), buf))
         return dict(zip(("band", "band_cols", "n_bands", "n_slices"), list(buf)))
 
+    def tiles(self, F):
+        """Rows per wavefront of the tile schedule (0: another schedule), and the streams held (sgnn_spmm_plan_tiles)."""
+        buf = (ctypes.c_int64 * 2)()
+        check(lib.sgnn_spmm_plan_tiles(self._h, int(F), buf))
+        return tuple(buf)
+
     def short_rows(self, F):
         """Chunks of short rows, and the dense rows a lane group keeps in flight (sgnn_spmm_plan_short_rows)."""
         buf = (ctypes.c_int64 * 2)()
