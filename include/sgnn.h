@@ -167,7 +167,7 @@ int sgnn_spmm_csr_f32(sgnn_spmm_plan *plan, const float *val, const float *x, fl
  *     bands into different chunks).  The simple way to guarantee that is one sgnn_spmm_csr_f32 call with the same
  *     F and the same kind of weights beforehand.  Otherwise the row-class kernels run: same result on rows of up
  *     to 128 edges, bit for bit; longer rows are summed per piece instead of in one chain (within the fp32
- *     tolerance, not the same bits);
+ *     tolerance, not the same bits).  The tile schedule in the same way: streams for any number of rows will do;
  *   - the scratch address is looked up when a plan is created, so the call itself performs no lazy symbol
  *     lookup, and it records no profiling events (sgnn_profile_enable does not see its kernels). */
 int sgnn_spmm_csr_f32_noalloc(sgnn_spmm_plan *plan, const float *val, const float *x, float *out,
@@ -287,6 +287,24 @@ int sgnn_quant_v1_f32(const float *x, uint8_t *q, const int64_t *range, float *p
 /* Replaces dequantize_tensor_v1 (super_gnn/ops/csrc/quantization_arm.cpp:704-757). */
 int sgnn_dequant_v1_f32(const uint8_t *q, float *x, const int64_t *range, const float *params,
                         int64_t n, int64_t F, sgnn_stream_t stream);
+
+/* ---------------------------------------------------------------------------------------------
+ * Layer passes (examples/graphsage/sage.py:176-211: conv -> dropout -> norm -> relu)
+ * ------------------------------------------------------------------------------------------- */
+
+/* y = relu((x - mean) * rstd * weight + bias) per row of C floats (a multiple of 4 up to 1024; all pointers 16-byte
+ * aligned), stats[n, 2] = (mean, rstd = 1 / sqrt(variance + eps)).  NaN stays NaN. */
+int sgnn_norm_relu_f32(const float *x, const float *weight, const float *bias, float eps, float *y, float *stats, int64_t n, int64_t C,
+                       sgnn_stream_t stream);
+
+/* Floats of workspace the gradient needs. */
+int64_t sgnn_norm_relu_workspace(int64_t n, int64_t C);
+
+/* Its gradient for rows that came out of a dropout: the norm's operand was mask * scale * x (mask[n, C] bytes of 0 or 1; null:
+ * x itself, scale 1).  gx: gradient w.r.t. x; gw, gb: w.r.t. weight and bias, summed over the rows in a fixed order. */
+int sgnn_norm_relu_backward_f32(const float *g, const float *x, const uint8_t *mask, float scale, const float *stats,
+                                const float *weight, const float *bias, float *gx, float *workspace, float *gw, float *gb, int64_t n, int64_t C,
+                                sgnn_stream_t stream);
 
 /* ---------------------------------------------------------------------------------------------
  * Measurement helpers (no reference counterpart; the reference times with std::chrono under

@@ -13,6 +13,7 @@ from torch import Tensor
 from torch.nn import LayerNorm, Linear, Parameter
 
 from .aggregator import Aggregator, LoopbackWorld
+from .supergnn_ops import norm_relu, norm_relu_backward
 
 
 def _column_sum(g: Tensor) -> Tensor:
@@ -80,6 +81,60 @@ class _SageCombine(torch.autograd.Function):
         return g_agg, g_x, None, g_wn, g_ws, g_b
 
 
+class _DropoutNormRelu(torch.autograd.Function):
+    """relu(layer_norm(dropout(x))) with the norm and the rectifier in one pass forward, and everything in one pass backward.
+    The dropout itself is torch's, so that the masks are those of its generator."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias, eps, p):
+        dropped, mask = torch.native_dropout(x, p, True) if p > 0 else (x, None)
+        y, stats = norm_relu(dropped, weight, bias, eps)
+        ctx.save_for_backward(x, mask, stats, weight, bias)
+        ctx.eps, ctx.scale = eps, 1.0 / (1.0 - p)
+        return y
+
+    @staticmethod
+    def backward(ctx, g):
+        x, mask, stats, weight, bias = ctx.saved_tensors
+        if torch.is_grad_enabled():   # a gradient that is differentiated itself
+            with torch.enable_grad():
+                dropped = x if mask is None else x * mask * ctx.scale
+                y = F.relu(F.layer_norm(dropped, weight.shape, weight, bias, ctx.eps))
+                wanted = [t for t, need in zip((x, weight, bias), ctx.needs_input_grad) if need]
+                found = iter(torch.autograd.grad(y, wanted, g, create_graph=True))
+            return tuple(next(found) if need else None for need in ctx.needs_input_grad[:3]) + (None, None)
+        return norm_relu_backward(g.contiguous(), x, mask, ctx.scale, stats, weight, bias) + (None, None)
+
+
+_global_hooks = getattr(torch.nn.modules.module, "_has_any_global_hook", lambda: False)
+
+
+def _fusable(norm, x):
+    """Whether the one-pass kernels stand for dropout, ``norm`` and the rectifier: a plain LayerNorm over fp32 rows on the GPU,
+    with nothing attached that would see the modules' own calls."""
+    if type(norm) is not LayerNorm or type(x) is not torch.Tensor or not x.is_cuda or x.dtype != torch.float32 or x.dim() != 2:
+        return False
+    n, C = x.shape
+    if n == 0 or n >= 1 << 31 or C % 4 or C > 1024 or tuple(norm.normalized_shape) != (C,) or not x.is_contiguous() or x.data_ptr() % 16:
+        return False
+    for t in (norm.weight, norm.bias):
+        if type(t) is not Parameter or t.dtype != torch.float32 or t.device != x.device or not t.is_contiguous() or t.data_ptr() % 16:
+            return False
+    if norm._forward_hooks or norm._forward_pre_hooks or norm._backward_hooks or norm._backward_pre_hooks or _global_hooks():
+        return False
+    return not (torch.is_autocast_enabled() or torch.jit.is_tracing() or torch.compiler.is_compiling())
+
+
+def _dropout_norm_relu(x, norm, p, training):
+    """The stretch between two convolutions (sage.py:186-204)."""
+    if norm is not None and 0 <= p < 1 and _fusable(norm, x):
+        return _DropoutNormRelu.apply(x, norm.weight, norm.bias, norm.eps, p if training else 0.0)
+    x = F.dropout(x, p=p, training=training)
+    if norm is not None:
+        x = norm(x)
+    return F.relu(x)
+
+
 class LoopbackSAGEConv(torch.nn.Module):
     def __init__(self, in_channels: int, out_channels: int, normalize: bool = True, bias: bool = True):
         super().__init__()
@@ -123,11 +178,9 @@ class LoopbackSAGE(torch.nn.Module):
 
     def forward(self, world: LoopbackWorld, feats: Sequence[Tensor]) -> List[Tensor]:
         for i, conv in enumerate(self.convs[:-1]):
-            feats = conv(world, feats)
-            feats = [F.dropout(x, p=self.dropout, training=self.training) for x in feats]
-            if self.norms is not None:
-                feats = [self.norms[i](x) for x in feats]
-            feats = [F.relu(x) for x in feats]
+            norm = None if self.norms is None else self.norms[i]
+            feats = [F.dropout(x, p=self.dropout, training=self.training) for x in conv(world, feats)]   # the generator's order
+            feats = [_dropout_norm_relu(x, norm, 0.0, False) for x in feats]
         feats = self.convs[-1](world, feats)
         return [F.log_softmax(x, dim=1) for x in feats]
 
@@ -193,9 +246,6 @@ class DistSAGE(torch.nn.Module):
     def forward(self, graph, nodes_feats, labels=None, label_mask=None):
         for i, conv in enumerate(self.convs[:-1]):
             nodes_feats = conv(graph, nodes_feats, i)
-            nodes_feats = F.dropout(nodes_feats, p=self.dropout, training=self.training)
-            if self.norms is not None:
-                nodes_feats = self.norms[i](nodes_feats)
-            nodes_feats = F.relu(nodes_feats)
+            nodes_feats = _dropout_norm_relu(nodes_feats, None if self.norms is None else self.norms[i], self.dropout, self.training)
         nodes_feats = self.convs[-1](graph, nodes_feats, len(self.convs) - 1)
         return F.log_softmax(nodes_feats, dim=1)

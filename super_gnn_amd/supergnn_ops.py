@@ -654,3 +654,24 @@ def dequantize_tensor_v1(input, output, quantized_nodes_feat_range, quantized_pa
     s_out = _Staged(output, dev, writeback=True)
     check(lib.sgnn_dequant_v1_f32(_ptr(s_q.dev), _ptr(s_out.dev), _ptr(s_r.dev), _ptr(s_p.dev), n, F, _stream()))
     s_out.commit()
+
+
+# -------------------------------------------------------------------------------------------------
+# Layer passes
+# -------------------------------------------------------------------------------------------------
+def norm_relu(x, weight, bias, eps):
+    """relu(layer_norm(x)) of contiguous fp32 rows on the GPU, and each row's (mean, 1 / standard deviation)."""
+    n, C = x.shape
+    y, stats = torch.empty_like(x), torch.empty((n, 2), dtype=torch.float32, device=x.device)
+    check(lib.sgnn_norm_relu_f32(x.data_ptr(), weight.data_ptr(), bias.data_ptr(), eps, y.data_ptr(), stats.data_ptr(), n, C, _stream()))
+    return y, stats
+
+
+def norm_relu_backward(g, x, mask, scale, stats, weight, bias):
+    """Gradients of relu(layer_norm(mask * scale * x)) w.r.t. x, weight and bias; mask None: no dropout."""
+    n, C = x.shape
+    gx, gw, gb = torch.empty_like(x), torch.empty_like(weight), torch.empty_like(bias)
+    work = torch.empty(lib.sgnn_norm_relu_workspace(n, C), dtype=torch.float32, device=x.device)
+    check(lib.sgnn_norm_relu_backward_f32(g.data_ptr(), x.data_ptr(), _ptr(mask), scale, stats.data_ptr(), weight.data_ptr(), bias.data_ptr(),
+                                          gx.data_ptr(), work.data_ptr(), gw.data_ptr(), gb.data_ptr(), n, C, _stream()))
+    return gx, gw, gb
