@@ -2351,7 +2351,7 @@ static int tile_rows(const sgnn_spmm_plan *p, int64_t F) {
     if (mode < 2 && (p->tile_spread > kTileSpread || (double)p->nnz * 2000.0 < (double)p->M * (double)p->K)) return 0;
     // One chain of fmas per row: where the row classes would take the product, which add up long rows in parts, only if there
     // are none (a chain of 370 edges is off by 3.0e-7, the parts by 1.3e-7).
-    if (mode < 2 && p->long_edges > 0 && !band_wanted(p, F, band_window_shape(p, 0, (int)F, true, F > kBandWindowCols))) return 0;
+    if (mode < 2 && p->long_edges > 0 && !band_wanted(p, F, band_windows(p, F, true).w[0])) return 0;
     const double others = 0.9 * 8.9 * (double)p->nnz * (double)F / 64.0 / 256.0;   // band schedule: 8.9 clocks per edge of 64 floats and CU
     if (mode < 2 && (double)((p->K + kTileCols - 1) / kTileCols) * 1200.0 > others) return 0;
     int best = kTileRows;

@@ -93,6 +93,13 @@ def test_default_rule_takes_tiles_for_dense_matrices_alone():
     assert ops.SpmmPlan(rp, cl, 200000).tiles(602)[0] == 0
 
 
+@pytest.mark.parametrize("F", [1, 511, 512, 513, 2049, 30000, 40001])
+def test_rule_answers_for_every_width(F):
+    """Long rows in a dense matrix: the rule asks what the band schedule would do, whose windows are 512 columns wide."""
+    plan = _plan(600, 500, 60, 11, hubs=3, hub_deg=450)[3]
+    assert plan.tiles(F)[0] == 0
+
+
 def test_unsorted_rows_keep_the_other_schedules(monkeypatch):
     monkeypatch.setenv("SGNN_SPMM_BAND", "2")
     rowptr, col, val, plan = _plan(300, 400, 50, 9, dup=True)
