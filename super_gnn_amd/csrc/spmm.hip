@@ -339,22 +339,6 @@ __device__ __forceinline__ void short_chunk_body(
     }
 }
 
-template <int VEC, int G, int NV, int BITS, int U, bool FENCED>
-__global__ __launch_bounds__(kBlock) void spmm_short_kernel(
-    const int64_t *__restrict__ rowptr, const int32_t *__restrict__ col, const float *__restrict__ val,
-    const DenseSrc dense, float *__restrict__ out, const int4 *__restrict__ chunks, int n_chunks, int F,
-    int64_t ldo, int accumulate, const float *__restrict__ row_div, uint32_t nblocks) {
-    constexpr int GPB = kBlock / G;
-    const uint32_t lb = xcd_contiguous_block(blockIdx.x, nblocks);
-    const int gid = threadIdx.x / G, lig = threadIdx.x % G;
-    const int ci = (int)lb * GPB + gid;
-    if (ci >= n_chunks) return;
-    // A chunk record is (first row, row count, first edge, edge count): the column/weight loads
-    // depend on it alone and are issued before the row pointers come back.
-    short_chunk_body<VEC, G, NV, BITS, int64_t, U, FENCED>(
-        rowptr, col, val, dense, out, chunks[ci], 0, F, ldo, accumulate, row_div, lig);
-}
-
 // ------------------------------------------------------------------------------------------------
 // Band schedule (dense-degree matrices whose dense operand does not fit the L2 caches).
 //
@@ -715,14 +699,13 @@ __global__ __launch_bounds__(kBlock) void rows_fill_or_divide_kernel(float *__re
 // dependent id -> address chain once, not once per row.
 constexpr int kEmptyRowsPerGroup = 4;
 template <int VEC, int G, int NV>
-__global__ __launch_bounds__(kBlock) void spmm_empty_rows_kernel(const int32_t *__restrict__ empty_rows, int n_empty,
-                                                                 float *__restrict__ out, int F, int64_t ldo,
-                                                                 int accumulate, const float *__restrict__ row_div) {
+__device__ __forceinline__ void empty_rows_body(int block, const int32_t *__restrict__ empty_rows, int n_empty, float *__restrict__ out, int F,
+                                                int64_t ldo, int accumulate, const float *__restrict__ row_div) {
     constexpr int GPB = kBlock / G;
     constexpr int TILE = G * VEC * NV;
     constexpr int R = kEmptyRowsPerGroup;
     const int gid = threadIdx.x / G, lig = threadIdx.x % G;
-    const int i0 = (blockIdx.x * GPB + gid) * R;
+    const int i0 = (block * GPB + gid) * R;
     if (i0 >= n_empty) return;
     int64_t rows[R];
     float divs[R];
@@ -876,21 +859,22 @@ __global__ __launch_bounds__(kBlock) void spmm_hubrow_lds_kernel(
 // ------------------------------------------------------------------------------------------------
 // Long rows, step 2: add a row's piece partials in piece order, epilogue, store.  A row's time is its chain of batches of UP
 // partials.  KEEP: the partials of the whole product are few (keep_partials), written and read with ordinary accesses instead of
-// streaming ones and sixteen at a time: 200 k power-law nodes, F = 100 18.8 -> 14.2 us, fused 1 M rows 28.1 -> 20.0.  The reader
-// finds few of them in its own L2 either way (18 MB fetched of 18, hit rate 0.13 against 0.27: a row's pieces come from up to
-// eight XCDs), so they are taken to stay in the Infinity Cache.  More of them only push dense rows out (1 M nodes, 32 M edges:
-// the product 1.41 -> 1.47 ms, UP = 16 as well as 8).
+// streaming ones, and summed in the short rows' launch.  (A launch of its own took 14.2 us with ordinary accesses sixteen at a
+// time, 18.8 with streaming ones, 200 k power-law nodes, F = 100; six at a time keep the joint kernel within the 64
+// registers that eight waves per SIMD have.)  The reader finds few of the partials in its own L2 either way (18 MB fetched of 18,
+// hit rate 0.13 against 0.27: a row's pieces come from up to eight XCDs), so they are taken to stay in the Infinity Cache.
+// More of them only push dense rows out (1 M nodes, 32 M edges: the product 1.41 -> 1.47 ms, UP = 16 as well as 8).
 // ------------------------------------------------------------------------------------------------
 template <int VEC, int G, int NV, bool KEEP>
-__global__ __launch_bounds__(kBlock) void spmm_long_final_kernel(
-    const int32_t *__restrict__ long_rows, const int32_t *__restrict__ long_pbeg,
+__device__ __forceinline__ void long_final_body(
+    int block, const int32_t *__restrict__ long_rows, const int32_t *__restrict__ long_pbeg,
     const float *__restrict__ partial, float *__restrict__ out, int n_long, int F, int64_t ldo,
     int accumulate, const float *__restrict__ row_div) {
     constexpr int GPB = kBlock / G;
     constexpr int TILE = G * VEC * NV;
-    constexpr int UP = KEEP ? 16 : 8;
+    constexpr int UP = KEEP ? 6 : 8;
     const int gid = threadIdx.x / G, lig = threadIdx.x % G;
-    const int li = blockIdx.x * GPB + gid;
+    const int li = block * GPB + gid;
     if (li >= n_long) return;
     const int64_t row = long_rows[li];
     const int s0 = long_pbeg[li], s1 = long_pbeg[li + 1];
@@ -910,7 +894,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_final_kernel(
 #pragma unroll
                 for (int u = 0; u < UP; ++u) {
                     const int si = s + u < s1 ? s + u : s1 - 1;
-                    if constexpr (KEEP) vec_load<VEC>(p[u], partial + (int64_t)si * F + off);
+                    if constexpr (KEEP) vec_load<VEC>(p[u], partial + (uint32_t)(si * F + off));   // (at most 40 MB)
                     else vec_load_nt<VEC>(p[u], partial + (int64_t)si * F + off);
                 }
 #pragma unroll
@@ -928,6 +912,53 @@ __global__ __launch_bounds__(kBlock) void spmm_long_final_kernel(
             vec_store_nt<VEC>(orow + off, acc);
         }
     }
+}
+
+template <int VEC, int G, int NV>
+__global__ __launch_bounds__(kBlock) void spmm_long_final_kernel(
+    const int32_t *__restrict__ long_rows, const int32_t *__restrict__ long_pbeg,
+    const float *__restrict__ partial, float *__restrict__ out, int n_long, int F, int64_t ldo,
+    int accumulate, const float *__restrict__ row_div) {
+    long_final_body<VEC, G, NV, false>((int)blockIdx.x, long_rows, long_pbeg, partial, out, n_long, F, ldo, accumulate, row_div);
+}
+
+// The short rows, and with them what else may run beside them: the long rows' final sum where its partials are kept
+// (keep_partials) and the rows without edges.  Both are short and wait for memory, and a launch of their own costs the
+// ramp-up and the tail of one (200 k power-law nodes, F = 100, transposed 192 -> 173 us; fused 1 M rows 580 -> 564).  Workgroups in this order: final sum (the longest chains), short rows, empty rows; the final
+// sum's number is a multiple of eight, so that the short rows' workgroups stay on their XCDs.
+struct RowTails {
+    const int32_t *long_rows, *long_pbeg;
+    const float *partial;
+    int n_long;
+    uint32_t final_blocks;
+    const int32_t *empty_rows;
+    int n_empty;
+    uint32_t short_blocks;
+};
+template <int VEC, int G, int NV, int BITS, int U, bool FENCED>
+__global__ __launch_bounds__(kBlock) void spmm_short_kernel(
+    const int64_t *__restrict__ rowptr, const int32_t *__restrict__ col, const float *__restrict__ val,
+    const DenseSrc dense, float *__restrict__ out, const int4 *__restrict__ chunks, int n_chunks, int F,
+    int64_t ldo, int accumulate, const float *__restrict__ row_div, const RowTails t) {
+    constexpr int GPB = kBlock / G;
+    uint32_t b = blockIdx.x;
+    if (b < t.final_blocks) {
+        long_final_body<VEC, G, NV, true>((int)b, t.long_rows, t.long_pbeg, t.partial, out, t.n_long, F, ldo, accumulate, row_div);
+        return;
+    }
+    b -= t.final_blocks;
+    if (b >= t.short_blocks) {
+        empty_rows_body<VEC, G, NV>((int)(b - t.short_blocks), t.empty_rows, t.n_empty, out, F, ldo, accumulate, row_div);
+        return;
+    }
+    const uint32_t lb = xcd_contiguous_block(b, t.short_blocks);
+    const int gid = threadIdx.x / G, lig = threadIdx.x % G;
+    const int ci = (int)lb * GPB + gid;
+    if (ci >= n_chunks) return;
+    // A chunk record is (first row, row count, first edge, edge count): the column/weight loads
+    // depend on it alone and are issued before the row pointers come back.
+    short_chunk_body<VEC, G, NV, BITS, int64_t, U, FENCED>(
+        rowptr, col, val, dense, out, chunks[ci], 0, F, ldo, accumulate, row_div, lig);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1175,9 +1206,9 @@ static uint32_t short_spare_lds(int vec, int G, int64_t x_bytes) {
 }
 
 template <int VEC, int G, int NV, int BITS, int U, bool FENCED = false>
-static void launch_short(const ShortArgs &a, uint32_t nb, uint32_t lds, hipStream_t st) {
+static void launch_short(const ShortArgs &a, const RowTails &t, uint32_t nb, uint32_t lds, hipStream_t st) {
     hipLaunchKernelGGL((spmm_short_kernel<VEC, G, NV, BITS, U, FENCED>), dim3(nb), dim3(kBlock), lds, st, a.rowptr, a.col, a.val,
-                       a.dense, a.out, a.chunks, a.n_chunks, a.F, a.ldo, a.accumulate, a.row_div, nb);
+                       a.dense, a.out, a.chunks, a.n_chunks, a.F, a.ldo, a.accumulate, a.row_div, t);
 }
 
 // Long rows' partial sums written and read with ordinary accesses (see spmm_long_final_kernel): 18 MB (200 k nodes, 4 M edges,
@@ -1187,6 +1218,7 @@ static int keep_partials(int64_t n_items, int64_t F) { return n_items * F * 4 <=
 template <int VEC, int G, int NV, int BITS>
 static void launch_all(const ShortArgs &a, const PieceArgs &s, const FinalArgs &f, hipStream_t st) {
     constexpr int GPB = kBlock / G;
+    RowTails tails{f.long_rows, f.long_pbeg, f.partial, f.n_long, 0, a.empty_rows, a.n_empty, 0};
     // The long rows (pieces + final sum) and the short rows write disjoint output rows; all kernels go to the
     // caller's stream one after the other (issuing the long rows on a second stream measured -1 ... +5 %).
     hipStream_t ls = st;
@@ -1208,38 +1240,34 @@ static void launch_all(const ShortArgs &a, const PieceArgs &s, const FinalArgs &
                 hipLaunchKernelGGL((spmm_piece_kernel<VEC, G, NV, BITS, false>), dim3(nb), dim3(kBlock), 0, ls, s.col_long,
                                    s.eperm, s.val, a.dense, s.partial, s.cls_work, s.max_cls_items, s.F, s.keep);
         }
-        const uint32_t nb = (uint32_t)((f.n_long + GPB - 1) / GPB);
-        ProfScope prof(K_SPMM_LONG_FINAL, ls, a.prof);
-        if (s.keep)
-            hipLaunchKernelGGL((spmm_long_final_kernel<VEC, G, NV, true>), dim3(nb), dim3(kBlock), 0, ls, f.long_rows,
+        if (s.keep) {
+            tails.final_blocks = (uint32_t)((f.n_long + GPB - 1) / GPB + kNumXCD - 1) / kNumXCD * kNumXCD;
+        } else {
+            const uint32_t nb = (uint32_t)((f.n_long + GPB - 1) / GPB);
+            ProfScope prof(K_SPMM_LONG_FINAL, ls, a.prof);
+            hipLaunchKernelGGL((spmm_long_final_kernel<VEC, G, NV>), dim3(nb), dim3(kBlock), 0, ls, f.long_rows,
                                f.long_pbeg, f.partial, f.out, f.n_long, f.F, f.ldo, f.accumulate, f.row_div);
-        else
-            hipLaunchKernelGGL((spmm_long_final_kernel<VEC, G, NV, false>), dim3(nb), dim3(kBlock), 0, ls, f.long_rows,
-                               f.long_pbeg, f.partial, f.out, f.n_long, f.F, f.ldo, f.accumulate, f.row_div);
-    }
-    if (a.n_chunks > 0) {
-        const uint32_t nb = (uint32_t)((a.n_chunks + GPB - 1) / GPB);
-        ProfScope prof(BITS == 0 ? K_SPMM_SHORT : K_FUSED_SHORT, st, a.prof);
-        if constexpr (NV > 1) launch_short<VEC, G, NV, BITS, unroll_of(NV)>(a, nb, 0, st);
-        else if constexpr (BITS != 0) launch_short<VEC, G, NV, BITS, G == 64 ? 8 : 4>(a, nb, 0, st);   // packed rows are 4 ... 16 times smaller
-        else {
-            const int u = short_depth(VEC, G, a.F, a.load);
-            const uint32_t spare = u == 8 ? 0 : short_spare_lds(VEC, G, a.load.x_bytes);
-            if (u == 8) launch_short<VEC, G, NV, 0, 8>(a, nb, spare, st);
-            else if constexpr (VEC > 1 && G == 16) launch_short<VEC, G, NV, 0, 3>(a, nb, spare, st);
-            else if constexpr (VEC > 1 && G == 32) launch_short<VEC, G, NV, 0, 2>(a, nb, spare, st);
-            else if constexpr (VEC == 2 && G == 64) launch_short<VEC, G, NV, 0, 4>(a, nb, spare, st);
-            else if constexpr (VEC == 4 && G == 64) {
-                if (u == 2) launch_short<VEC, G, NV, 0, 2>(a, nb, spare, st);
-                else launch_short<VEC, G, NV, 0, 6, true>(a, nb, spare, st);
-            }
         }
     }
-    if (a.n_empty > 0 && (!a.accumulate || a.row_div)) {
-        const uint32_t nb = (uint32_t)((a.n_empty + GPB * kEmptyRowsPerGroup - 1) / (GPB * kEmptyRowsPerGroup));
-        ProfScope prof(K_SPMM_EMPTY_ROWS, st, a.prof);
-        hipLaunchKernelGGL((spmm_empty_rows_kernel<VEC, G, NV>), dim3(nb), dim3(kBlock), 0, st, a.empty_rows, a.n_empty,
-                           a.out, a.F, a.ldo, a.accumulate, a.row_div);
+    tails.short_blocks = (uint32_t)((a.n_chunks + GPB - 1) / GPB);
+    const uint32_t empty_blocks = a.n_empty > 0 && (!a.accumulate || a.row_div)
+                                      ? (uint32_t)((a.n_empty + GPB * kEmptyRowsPerGroup - 1) / (GPB * kEmptyRowsPerGroup)) : 0;
+    const uint32_t nb = tails.final_blocks + tails.short_blocks + empty_blocks;
+    if (nb == 0) return;
+    ProfScope prof(a.n_chunks == 0 && tails.final_blocks == 0 ? K_SPMM_EMPTY_ROWS : BITS == 0 ? K_SPMM_SHORT : K_FUSED_SHORT, st, a.prof);
+    if constexpr (NV > 1) launch_short<VEC, G, NV, BITS, unroll_of(NV)>(a, tails, nb, 0, st);
+    else if constexpr (BITS != 0) launch_short<VEC, G, NV, BITS, G == 64 ? 8 : 4>(a, tails, nb, 0, st);   // packed rows are 4 ... 16 times smaller
+    else {
+        const int u = short_depth(VEC, G, a.F, a.load);
+        const uint32_t spare = u == 8 ? 0 : short_spare_lds(VEC, G, a.load.x_bytes);
+        if (u == 8) launch_short<VEC, G, NV, 0, 8>(a, tails, nb, spare, st);
+        else if constexpr (VEC > 1 && G == 16) launch_short<VEC, G, NV, 0, 3>(a, tails, nb, spare, st);
+        else if constexpr (VEC > 1 && G == 32) launch_short<VEC, G, NV, 0, 2>(a, tails, nb, spare, st);
+        else if constexpr (VEC == 2 && G == 64) launch_short<VEC, G, NV, 0, 4>(a, tails, nb, spare, st);
+        else if constexpr (VEC == 4 && G == 64) {
+            if (u == 2) launch_short<VEC, G, NV, 0, 2>(a, tails, nb, spare, st);
+            else launch_short<VEC, G, NV, 0, 6, true>(a, tails, nb, spare, st);
+        }
     }
 }
 
