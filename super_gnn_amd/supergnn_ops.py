@@ -28,8 +28,11 @@ from collections import OrderedDict
 
 import torch
 
-from . import _lib
+from . import _direct, _lib
 from ._lib import check, lib
+
+_direct.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in (
+    "sgnn_quant_pack_rows_f32", "sgnn_quant_pack_rows_wire_f32", "sgnn_unpack_dequant_rows_f32", "sgnn_unpack_dequant_rows_wire_f32")))
 
 __all__ = [
     "spmm", "quantize_tensor", "dequantize_tensor", "quantize_tensor_for_all_procs",
@@ -443,6 +446,11 @@ def _checked_row_index(row_index, n_src):
 
 
 def _quant_rows(inp, out_u8, params, segs, bits, row_index=None):
+    if row_index is None:
+        queued = _direct.quant_rows(inp, out_u8, params, segs.seg, segs.pseg, segs.n_rows, segs.n_packed, bits)   # 0: something is not plain
+        if queued:
+            check(queued)
+            return
     _want(inp, torch.float32, "input")
     _want(out_u8, torch.uint8, "output")
     bf16 = _params_kind(params, "quantized_params")
@@ -499,6 +507,10 @@ def _quant_gathered_rows(src, row_index, out_u8, params, bf16, segs, bits):
 
 
 def _dequant_rows(inp_u8, out, params, segs, bits):
+    queued = _direct.dequant_rows(out, inp_u8, params, segs.seg, segs.pseg, segs.n_rows, segs.n_packed, bits)
+    if queued:
+        check(queued)
+        return
     _want(inp_u8, torch.uint8, "input")
     _want(out, torch.float32, "output")
     bf16 = _params_kind(params, "dequantized_params")
