@@ -306,6 +306,13 @@ int sgnn_norm_relu_backward_f32(const float *g, const float *x, const uint8_t *m
                                 const float *weight, const float *bias, float *gx, float *workspace, float *gw, float *gb, int64_t n, int64_t C,
                                 sgnn_stream_t stream);
 
+/* out[c] = sum over n > 0 rows of x[n, C], in a fixed order (C and alignment as above; workspace: as many floats as
+ * sgnn_norm_relu_workspace(n, C)). */
+int sgnn_column_sum_f32(const float *x, float *workspace, float *out, int64_t n, int64_t C, sgnn_stream_t stream);
+
+/* w[n_out, n_in] += g^T a over a few rows of g[rows, n_out] and a[rows, n_in]. */
+int sgnn_rest_product_f32(const float *g, const float *a, float *w, int64_t rows, int64_t n_out, int64_t n_in, sgnn_stream_t stream);
+
 /* ---------------------------------------------------------------------------------------------
  * Measurement helpers (no reference counterpart; the reference times with std::chrono under
  * #define PROFILE, super_gnn/ops/csrc/spmm.cpp:12,352-354,518-523)

@@ -42,6 +42,8 @@ SIGNATURES = {
     "sgnn_norm_relu_f32": (_int, [_vp, _vp, _vp, ctypes.c_float, _vp, _vp, _i64, _i64, _vp]),
     "sgnn_norm_relu_workspace": (_i64, [_i64, _i64]),
     "sgnn_norm_relu_backward_f32": (_int, [_vp, _vp, _vp, ctypes.c_float, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _vp]),
+    "sgnn_column_sum_f32": (_int, [_vp, _vp, _vp, _i64, _i64, _vp]),
+    "sgnn_rest_product_f32": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _vp]),
     "sgnn_profile_enable": (_int, [_int]),
     "sgnn_profile_read": (_int, [_int, ctypes.POINTER(_i64), ctypes.POINTER(ctypes.c_double)]),
     "sgnn_profile_kernel_name": (ctypes.c_char_p, [_int]),

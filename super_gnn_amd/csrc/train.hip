@@ -174,32 +174,114 @@ __global__ __launch_bounds__(kNormBlock) void norm_relu_backward_kernel(
     __syncthreads();
     for (int i = threadIdx.x; i < 2 * C; i += kNormBlock) {
         const int which = i >= C, c = i - which * C;
-        float s = 0.0f;
+        double s = 0.0;
 #pragma unroll
-        for (int q = 0; q < kGroups; ++q) s += sums[q][which][c];
-        partial[(int64_t)blockIdx.x * 2 * C + i] = s;
+        for (int q = 0; q < kGroups; ++q) s += (double)sums[q][which][c];
+        partial[(int64_t)blockIdx.x * 2 * C + i] = (float)s;
     }
 }
 
-// out[i] = sum over blocks of partial[block][i]: 16 columns and 16 parts of the blocks per workgroup, in fixed order.
-__global__ __launch_bounds__(256) void norm_partial_sum_kernel(const float *__restrict__ partial, float *__restrict__ gw,
-                                                               float *__restrict__ gb, int blocks, int C) {
-    __shared__ float part[16][17];
+// Sums over the rows of each column, per workgroup: partial[block][C].  Bound by memory (150 k x 256: 55 us as torch's sum,
+// whose 64 workgroups leave most of the chip idle -> 27 us with the sum of the partials).
+template <int G, int NV>
+__global__ __launch_bounds__(kNormBlock) void column_sum_kernel(const float *__restrict__ x, float *__restrict__ partial, int64_t n, int C) {
+    constexpr int kGroups = kNormBlock / G, kRows = 4;
+    __shared__ float sums[kGroups][G * NV * 4];
+    const int lig = threadIdx.x % G, group = threadIdx.x / G;
+    float acc[NV][4] = {};
+    const int64_t step = (int64_t)gridDim.x * kGroups * kRows;
+    for (int64_t row0 = ((int64_t)blockIdx.x * kGroups + group) * kRows; row0 < n; row0 += step) {
+        float v[kRows][NV][4];
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) {
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                const int c = 4 * (lig + G * k);
+                if (row0 + r < n && c < C) {
+                    vec_load<4>(v[r][k], x + (row0 + r) * C + c);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[r][k][e] = 0.0f;
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < kRows; ++r)
+#pragma unroll
+            for (int k = 0; k < NV; ++k)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[k][e] += v[r][k][e];
+    }
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sums[group][4 * (lig + G * k) + e] = acc[k][e];
+    __syncthreads();
+    for (int c = threadIdx.x; c < C; c += kNormBlock) {
+        double s = 0.0;
+#pragma unroll
+        for (int q = 0; q < kGroups; ++q) s += (double)sums[q][c];
+        partial[(int64_t)blockIdx.x * C + c] = (float)s;
+    }
+}
+
+// (a, b)[i] = sum over blocks of partial[block][i], the first n_a columns in a: 16 columns and 16 parts of the blocks per
+// workgroup, in fixed order and 64 bits (the sums of 1024 workgroups lose more than their rows do otherwise).
+__global__ __launch_bounds__(256) void partial_sum_kernel(const float *__restrict__ partial, float *__restrict__ a, float *__restrict__ b,
+                                                          int blocks, int n_a, int n) {
+    __shared__ double part[16][17];
     const int c = threadIdx.x & 15, q = threadIdx.x >> 4, i = blockIdx.x * 16 + c;
-    float s = 0.0f;
-    if (i < 2 * C) {
+    double s = 0.0;
+    if (i < n) {
 #pragma unroll 8
-        for (int b = q; b < blocks; b += 16) s += partial[(int64_t)b * 2 * C + i];
+        for (int k = q; k < blocks; k += 16) s += (double)partial[(int64_t)k * n + i];
     }
     part[q][c] = s;
     __syncthreads();
-    if (q == 0 && i < 2 * C) {
-        float t = 0.0f;
+    if (q == 0 && i < n) {
+        double t = 0.0;
 #pragma unroll
         for (int k = 0; k < 16; ++k) t += part[k][c];
-        if (i < C) gw[i] = t;
-        else gb[i - C] = t;
+        if (i < n_a) a[i] = (float)t;
+        else b[i - n_a] = (float)t;
     }
+}
+
+// w[i, j] += sum over rows r of g[r, i] * a[r, j], for the few rows a batched product over equal slabs leaves over: the library gives
+// the whole product to one workgroup (12 ... 25 us for 48 rows of 47 ... 256 columns, six times a training step of three layers).
+// 64 x 64 outputs per workgroup, 4 x 4 per thread, 64 rows of both operands in LDS at a time: the latency of one round of loads.
+constexpr int kRestRows = 64;
+__global__ __launch_bounds__(256) void rest_product_kernel(const float *__restrict__ g, const float *__restrict__ a, float *__restrict__ w,
+                                                           int rows, int n_out, int n_in) {
+    __shared__ float gs[kRestRows][64], as[kRestRows][64];
+    const int i0 = blockIdx.x * 64, j0 = blockIdx.y * 64, ti = threadIdx.x / 16, tj = threadIdx.x % 16;
+    float acc[4][4] = {};
+    for (int r0 = 0; r0 < rows; r0 += kRestRows) {
+        float gv[kRestRows * 64 / 256], av[kRestRows * 64 / 256];
+#pragma unroll
+        for (int k = 0; k < kRestRows * 64 / 256; ++k) {
+            const int r = r0 + (threadIdx.x + 256 * k) / 64, c = threadIdx.x % 64;
+            gv[k] = r < rows && i0 + c < n_out ? g[(int64_t)r * n_out + i0 + c] : 0.0f;
+            av[k] = r < rows && j0 + c < n_in ? a[(int64_t)r * n_in + j0 + c] : 0.0f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kRestRows * 64 / 256; ++k) {
+            gs[(threadIdx.x + 256 * k) / 64][threadIdx.x % 64] = gv[k];
+            as[(threadIdx.x + 256 * k) / 64][threadIdx.x % 64] = av[k];
+        }
+        __syncthreads();
+        for (int r = 0; r < kRestRows && r0 + r < rows; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(gs[r][ti + 16 * i], as[r][tj + 16 * j], acc[i][j]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (i0 + ti + 16 * i < n_out && j0 + tj + 16 * j < n_in) w[(int64_t)(i0 + ti + 16 * i) * n_in + j0 + tj + 16 * j] += acc[i][j];
 }
 
 // f(G, NV) with the lane group of rows of C floats: the narrowest of 8 ... 64 lanes, one to four vectors each.
@@ -259,8 +341,32 @@ extern "C" int sgnn_norm_relu_backward_f32(const float *g, const float *x, const
         hipLaunchKernelGGL((norm_relu_backward_kernel<gl, nv>), dim3((uint32_t)blocks), dim3(kNormBlock), 0, (hipStream_t)stream, g, x, mask, scale,
                            reinterpret_cast<const float2 *>(stats), weight, bias, gx, workspace, n, (int)C);
     });
-    hipLaunchKernelGGL(norm_partial_sum_kernel, dim3((uint32_t)((2 * C + 15) / 16)), dim3(256), 0, (hipStream_t)stream, workspace, gw, gb, blocks,
+    hipLaunchKernelGGL(partial_sum_kernel, dim3((uint32_t)((2 * C + 15) / 16)), dim3(256), 0, (hipStream_t)stream, workspace, gw, gb, blocks,
+                       (int)C, (int)(2 * C));
+    SGNN_HIP_CHECK(hipGetLastError());
+    return SGNN_OK;
+}
+
+extern "C" int sgnn_column_sum_f32(const float *x, float *workspace, float *out, int64_t n, int64_t C, sgnn_stream_t stream) {
+    const int rc = check_norm(x, x, x, x, n, C);
+    if (rc != SGNN_OK) return rc;
+    SGNN_REQUIRE(n > 0 && workspace && out, "null argument or no rows");
+    const int blocks = norm_blocks(n, C);
+    with_norm_shape(C, [&](auto g, auto nv) {
+        hipLaunchKernelGGL((column_sum_kernel<g, nv>), dim3((uint32_t)blocks), dim3(kNormBlock), 0, (hipStream_t)stream, x, workspace, n, (int)C);
+    });
+    hipLaunchKernelGGL(partial_sum_kernel, dim3((uint32_t)((C + 15) / 16)), dim3(256), 0, (hipStream_t)stream, workspace, out, out, blocks, (int)C,
                        (int)C);
+    SGNN_HIP_CHECK(hipGetLastError());
+    return SGNN_OK;
+}
+
+extern "C" int sgnn_rest_product_f32(const float *g, const float *a, float *w, int64_t rows, int64_t n_out, int64_t n_in, sgnn_stream_t stream) {
+    SGNN_REQUIRE(rows >= 0 && rows < (1 << 20) && n_out > 0 && n_in > 0 && n_out < (1 << 20) && n_in < (1 << 20), "sizes out of range");
+    if (rows == 0) return SGNN_OK;
+    SGNN_REQUIRE(g && a && w, "null argument");
+    hipLaunchKernelGGL(rest_product_kernel, dim3((uint32_t)((n_out + 63) / 64), (uint32_t)((n_in + 63) / 64)), dim3(256), 0, (hipStream_t)stream, g, a,
+                       w, (int)rows, (int)n_out, (int)n_in);
     SGNN_HIP_CHECK(hipGetLastError());
     return SGNN_OK;
 }

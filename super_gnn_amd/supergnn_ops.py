@@ -687,3 +687,16 @@ def norm_relu_backward(g, x, mask, scale, stats, weight, bias):
     check(lib.sgnn_norm_relu_backward_f32(g.data_ptr(), x.data_ptr(), _ptr(mask), scale, stats.data_ptr(), weight.data_ptr(), bias.data_ptr(),
                                           gx.data_ptr(), work.data_ptr(), gw.data_ptr(), gb.data_ptr(), n, C, _stream()))
     return gx, gw, gb
+
+
+def column_sum(x):
+    """Sum over the rows of a contiguous fp32 matrix on the GPU."""
+    n, C = x.shape
+    out, work = torch.empty(C, dtype=torch.float32, device=x.device), torch.empty(lib.sgnn_norm_relu_workspace(n, C), dtype=torch.float32, device=x.device)
+    check(lib.sgnn_column_sum_f32(x.data_ptr(), work.data_ptr(), out.data_ptr(), n, C, _stream()))
+    return out
+
+
+def add_rest_product(g, a, w):
+    """w += g^T a for a few rows; contiguous fp32 matrices on the GPU."""
+    check(lib.sgnn_rest_product_f32(g.data_ptr(), a.data_ptr(), w.data_ptr(), g.shape[0], g.shape[1], a.shape[1], _stream()))

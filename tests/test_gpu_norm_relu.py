@@ -79,3 +79,33 @@ def test_special_values_and_second_derivatives():
         first, = torch.autograd.grad((f(xs) ** 2).sum(), xs, create_graph=True)
         grads.append(torch.autograd.grad((first ** 2).sum(), xs)[0])
     assert torch.allclose(*grads, rtol=1e-3, atol=1e-4)
+
+
+@pytest.mark.parametrize("n,C", [(1, 4), (3, 36), (4, 64), (5, 68), (1023, 128), (4097, 256), (150000, 256), (300, 516), (64, 1024)])
+def test_column_sum_matches_float64(n, C):
+    from super_gnn_amd.supergnn_ops import column_sum
+    x = torch.randn(n, C, generator=torch.Generator().manual_seed(n), dtype=torch.float32)
+    got, want = column_sum(x.cuda()).double().cpu(), x.double().sum(0)
+    # a thread's chain of n / 4096 rows and a tree over the workgroups: well below a sequential sum's n roundings
+    assert bool(((got - want).abs() <= (n ** 0.5 + 16) * EPS * x.abs().double().sum(0)).all())
+
+
+@pytest.mark.parametrize("rows,n_out,n_in", [(0, 8, 8), (1, 1, 1), (15, 64, 65), (16, 63, 64), (17, 47, 256), (48, 256, 256), (63, 130, 100)])
+def test_rest_product_matches_float64(rows, n_out, n_in):
+    from super_gnn_amd.supergnn_ops import add_rest_product
+    g, a, w = (torch.randn(*s, generator=torch.Generator().manual_seed(s[-1])) for s in ((rows, n_out), (rows, n_in), (n_out, n_in)))
+    want, mass = w.double() + g.double().t() @ a.double(), w.abs().double() + g.abs().double().t() @ a.abs().double()
+    got = w.cuda()
+    add_rest_product(g.cuda(), a.cuda(), got)
+    assert bool(((got.double().cpu() - want).abs() <= (rows + 1) * EPS * mass).all())
+
+
+def test_weight_gradient_of_rows_that_slabs_leave_over():
+    from super_gnn_amd.layers import _weight_grad
+    for n in (65536, 65537, 65599):
+        g, a = (torch.randn(n, c, generator=torch.Generator().manual_seed(c)).cuda() for c in (8, 12))
+        want = g.double().t() @ a.double()
+        bound = 64 * EPS * (g.abs().double().t() @ a.abs().double())
+        with torch.no_grad():
+            assert bool(((_weight_grad(g, a).double() - want).abs() <= bound).all())
+        assert bool(((_weight_grad(g, a).double() - want).abs() <= bound).all())   # as in a gradient that is differentiated
