@@ -1371,6 +1371,7 @@ struct BandSchedule {
     int32_t *eperm_bm = nullptr;       // [nnz] CSR index of each band-major edge
     float *val_bm = nullptr;           // [nnz] edge values in band-major order
     uint64_t val_gen = 0;              // plan bind generation val_bm was filled under (0 = not from a bound array)
+    bool graph_fills = false;          // a captured product fills val_bm (see values_due)
     uint64_t last_use = 0;             // the plan's band_use_clock at this schedule's last product
     int64_t M = 0, K = 0;
     std::vector<int32_t> h_rowptr_bm;  // host: [n_bands * (M+1)] where each (band, row) starts in the band-major arrays
@@ -1396,6 +1397,7 @@ struct TileSchedule {
     int32_t *batch0 = nullptr;         // [n_rb * kTileConsumers] each wave's first batch
     int32_t *slot_edge = nullptr;      // [batches * kTileBatch] CSR index of every slot, -1: padding
     uint64_t val_gen = 0;              // plan bind generation the values were filled under (0: not from a bound array)
+    bool graph_fills = false;          // a captured product fills the values (see values_due)
     uint64_t last_use = 0;
     ~TileSchedule() {
         (void)hipFree(stream); (void)hipFree(batch0); (void)hipFree(slot_edge);
@@ -2243,6 +2245,20 @@ static int grow_xs(sgnn_spmm_plan *root, size_t floats, bool *ok) {
     return SGNN_OK;
 }
 
+// Whether a product has to fill its schedule's copy of the edge values, which all products through the schedule share.  A bound
+// array's values stay (where `keep` says that binding counts).  A captured product always fills, so that a replay neither
+// finds another array's values nor misses an edit; after one, every product does, since a replay may have come between.
+template <typename Schedule>
+static int values_due(const sgnn_spmm_plan *p, Schedule *s, const float *val, bool keep, hipStream_t st, bool *due) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    SGNN_HIP_CHECK(hipStreamIsCapturing(st, &cap));
+    if (cap != hipStreamCaptureStatusNone) s->graph_fills = true;
+    const bool stays = keep && val == p->bound_val && !s->graph_fills;
+    *due = !stays || s->val_gen != p->bind_gen;
+    s->val_gen = stays ? p->bind_gen : 0;
+    return SGNN_OK;
+}
+
 // The product through the band schedule.  may_build = false (the non-allocating entry point): use a schedule
 // only if an earlier call has built it; *done tells whether the product was carried out here.
 static int spmm_run_band(sgnn_spmm_plan *p, const BandWindows &bw, const float *val, const DenseSrc &dense, float *out, int64_t F,
@@ -2300,12 +2316,12 @@ static int spmm_run_band(sgnn_spmm_plan *p, const BandWindows &bw, const float *
     }
     const float *val_bm = nullptr;
     if (weighted) {
-        const bool bound = val == p->bound_val;
-        if (!(bound && bs->val_gen == p->bind_gen)) {
+        bool due = false;
+        const int rc = values_due(p, bs, val, true, st, &due);
+        if (rc != SGNN_OK) return rc;
+        if (due)
             hipLaunchKernelGGL(permute_values_kernel, dim3((uint32_t)((p->nnz + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, val,
                                bs->eperm_bm, bs->val_bm, p->nnz);
-            bs->val_gen = bound ? p->bind_gen : 0;
-        }
         val_bm = bs->val_bm;
     }
     const int iF = (int)F;
@@ -2471,14 +2487,17 @@ static int spmm_run_tile(sgnn_spmm_plan *p, int rows, const float *val, const De
         const int rc = grow_xs(root, xs_floats, &ok);
         if (rc != SGNN_OK || !ok) return rc;
     }
-    const bool bound = val != nullptr && val == p->bound_val;
-    if (val != nullptr && !(bound && ts->val_gen == p->bind_gen)) {
-        const int64_t slots = ts->batches * kTileBatch;
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        SGNN_HIP_CHECK(hipStreamIsCapturing(st, &cap));
-        hipLaunchKernelGGL(tile_values_kernel, dim3((uint32_t)((slots + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, val, ts->slot_edge,
-                           ts->stream, slots);
-        ts->val_gen = bound && cap == hipStreamCaptureStatusNone ? p->bind_gen : 0;   // (a captured launch has not run)
+    if (val != nullptr) {
+        // Without long rows the row classes read the caller's array in every product, so edits of it count here as well.
+        // (20 k rows of 65 edges, F = 602: the fill is 10 of 145 us; 114 M edges: 0.6 of 11.0 ms, saved where the values are bound)
+        bool due = false;
+        const int rc = values_due(p, ts, val, p->long_edges > 0, st, &due);
+        if (rc != SGNN_OK) return rc;
+        if (due) {
+            const int64_t slots = ts->batches * kTileBatch;
+            hipLaunchKernelGGL(tile_values_kernel, dim3((uint32_t)((slots + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, val, ts->slot_edge,
+                               ts->stream, slots);
+        }
     }
     if (p->whole == nullptr) ++root->call_serial;
     ts->last_use = ++root->band_use_clock;

@@ -1,0 +1,110 @@
+"""What the schedules of the SpMM that keep state in the plan may not change: products read the edge values they are given,
+whatever ran before on the same plan; captured products keep what they were captured with.  Against the CPU oracle, bit for
+bit (every row in CSR order with one fma per edge, under every schedule)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as orc
+from _util import random_csr
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+SHORT = (4000, 1500, 80, 602)     # no row of more than 128 edges, and the default rule takes tiles
+
+
+class _Case:
+    """A matrix with its plan, operand and a row sample of the oracle's result."""
+
+    def __init__(self, M, K, deg, F, seed=1, **kw):
+        from super_gnn_amd import supergnn_ops as ops
+        self.rowptr, self.col, val = random_csr(M, K, deg, seed=seed, **kw)
+        self.M, self.K, self.F = M, K, F
+        self.plan = ops.SpmmPlan(torch.from_numpy(self.rowptr).to(DEV), torch.from_numpy(self.col).to(DEV), K)
+        self.value = torch.from_numpy(val).to(DEV)
+        self.x = self.operand(F)
+        self.out = torch.empty(M, F, device=DEV)
+
+    def operand(self, F):
+        return torch.randn(self.K, F, generator=torch.Generator().manual_seed(F)).to(DEV)
+
+    def product(self, value, x=None, out=None):
+        x, out = self.x if x is None else x, self.out if out is None else out
+        out.fill_(7.0)
+        self.plan.run(value, x, out, accumulate=False)
+        return out
+
+    def want(self, value, x=None):
+        x = self.x if x is None else x
+        rows = 200                                           # from the middle on
+        r0 = (self.M - rows) // 2
+        lo, hi = self.rowptr[r0], self.rowptr[r0 + rows]
+        want = np.zeros((rows, x.shape[1]), np.float32)
+        orc.spmm_accumulate(self.rowptr[r0:r0 + rows + 1] - lo, self.col[lo:hi],
+                            np.ones(hi - lo, np.float32) if value is None else value[lo:hi].cpu().numpy(), x.cpu().numpy(), want)
+        return slice(r0, r0 + rows), want
+
+    def check(self, value, x=None, out=None, what=""):
+        rows, want = self.want(value, x)
+        equal = np.array_equal((self.out if out is None else out)[rows].cpu().numpy(), want)
+        assert equal, what
+
+
+def test_rows_that_are_not_long_are_read_from_the_callers_array():
+    """An edit that no version counter sees, after the plan has bound the values by itself."""
+    c = _Case(*SHORT)
+    assert c.plan.tiles(c.F)[0] > 0 and c.plan.info()["long_rows"] == 0
+    for i in range(3):
+        c.product(c.value)
+        c.check(c.value, what=i)
+    c.value.data.mul_(2)
+    c.product(c.value)
+    c.check(c.value, what="edited through .data")
+    c.value.add_(1)
+    c.product(c.value)
+    c.check(c.value, what="edited in place")
+
+
+def _captured(c, value):
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        c.plan.run(value, c.x, c.out, accumulate=False)
+    return graph
+
+
+@pytest.mark.parametrize("kind", ["short", "long", "short, tiles forced", "bands"])
+@pytest.mark.parametrize("bound", [False, True])
+def test_replays_and_eager_products_do_not_see_each_others_values(kind, bound, monkeypatch):
+    """A captured product reads its own array, edited or not, after eager products with other values, and the eager products
+    that follow a replay read theirs."""
+    if kind == "short":
+        c = _Case(*SHORT)
+    else:
+        monkeypatch.setenv("SGNN_SPMM_BAND", "1" if kind == "bands" else "2")
+        c = _Case(700, 900, 40, 130, **({"hubs": 5, "hub_deg": 600} if kind == "long" else {}))
+    for _ in range(3):
+        c.product(c.value)
+    assert c.plan.tiles(c.F)[1] == (kind != "bands")
+    if not bound:
+        c.plan.unbind_values()
+    graph = _captured(c, c.value)
+    other = c.value * 3 + 1
+    for i in range(3):
+        c.out.fill_(7.0)
+        graph.replay()
+        c.check(c.value, what=("replay", i))
+        eager = torch.empty_like(c.out)
+        for j in range(3):                                   # unbound, bound, bound and unchanged
+            c.product(other, out=eager)
+            c.check(other, out=eager, what=("eager", i, j))
+        c.out.fill_(7.0)
+        graph.replay()
+        c.check(c.value, what=("replay after other values", i))
+        c.product(other, out=eager)
+        c.check(other, out=eager, what=("eager after a replay", i))
+        c.value.mul_(1.5)
+        c.out.fill_(7.0)
+        graph.replay()
+        c.check(c.value, what=("replay of edited values", i))
+        torch.cuda.synchronize()
