@@ -1371,7 +1371,7 @@ struct BandSchedule {
     int32_t *eperm_bm = nullptr;       // [nnz] CSR index of each band-major edge
     float *val_bm = nullptr;           // [nnz] edge values in band-major order
     uint64_t val_gen = 0;              // plan bind generation val_bm was filled under (0 = not from a bound array)
-    bool graph_fills = false;          // a captured product fills val_bm (see values_due)
+    bool captured = false;             // a captured product names these buffers
     uint64_t last_use = 0;             // the plan's band_use_clock at this schedule's last product
     int64_t M = 0, K = 0;
     std::vector<int32_t> h_rowptr_bm;  // host: [n_bands * (M+1)] where each (band, row) starts in the band-major arrays
@@ -1397,7 +1397,7 @@ struct TileSchedule {
     int32_t *batch0 = nullptr;         // [n_rb * kTileConsumers] each wave's first batch
     int32_t *slot_edge = nullptr;      // [batches * kTileBatch] CSR index of every slot, -1: padding
     uint64_t val_gen = 0;              // plan bind generation the values were filled under (0: not from a bound array)
-    bool graph_fills = false;          // a captured product fills the values (see values_due)
+    bool captured = false;             // a captured product names these buffers
     uint64_t last_use = 0;
     ~TileSchedule() {
         (void)hipFree(stream); (void)hipFree(batch0); (void)hipFree(slot_edge);
@@ -1439,6 +1439,8 @@ struct sgnn_spmm_plan {
     double tile_spread = 0.0;       // batches of the row blocks' longest streams over their average (0: not known)
     float *band_xs = nullptr;       // the dense operand restaged slice by slice (see band_restage_kernel), grown on demand
     size_t band_xs_floats = 0;
+    bool band_xs_captured = false, partial_captured = false;   // a captured product names the buffer
+    std::vector<void *> kept;       // buffers grown out of that captured products may still name
     // A matrix with 2^31 edges or more is held as consecutive row blocks, each a plan of its own with fewer
     // edges than that (the kernels' edge offsets are 32-bit); every call on the whole runs the blocks in turn.
     std::vector<sgnn_spmm_plan *> parts;
@@ -1509,6 +1511,7 @@ extern "C" int sgnn_spmm_plan_destroy(sgnn_spmm_plan *p) {
     for (int i = 0; i < 3; ++i) (void)hipFree(p->chunks[i]);
     for (BandSchedule *b : p->bands) delete b;
     for (TileSchedule *t : p->tiles) delete t;
+    for (void *b : p->kept) (void)hipFree(b);
     (void)hipFree(p->band_xs);
     delete p;
     return SGNN_OK;
@@ -2228,11 +2231,31 @@ static void launch_fill_or_divide(float *out, int64_t M, int F, int64_t ldo, con
     else hipLaunchKernelGGL((rows_fill_or_divide_kernel<VEC, false>), dim3(nb), dim3(kBlock), 0, st, out, M, F, ldo, row_div);
 }
 
+static int is_capturing(hipStream_t st, bool *yes) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    SGNN_HIP_CHECK(hipStreamIsCapturing(st, &cap));
+    *yes = cap != hipStreamCaptureStatusNone;
+    return SGNN_OK;
+}
+
+// Gives up a buffer that a larger one replaces.  Queued work may still read it, and a captured product names it for as long as
+// its graph is replayed, so the plan then keeps it to its own end.
+static int give_up(sgnn_spmm_plan *p, float **buf, bool *captured) {
+    if (*captured) {
+        p->kept.push_back(*buf);
+    } else if (*buf != nullptr) {
+        SGNN_HIP_CHECK(hipDeviceSynchronize());
+        (void)hipFree(*buf);
+    }
+    *buf = nullptr;
+    *captured = false;
+    return SGNN_OK;
+}
+
 // The workspace for a restaged operand of `floats` floats; *ok is false when there is no room.
 static int grow_xs(sgnn_spmm_plan *root, size_t floats, bool *ok) {
-    SGNN_HIP_CHECK(hipDeviceSynchronize());  // the old workspace may still be read by queued work
-    (void)hipFree(root->band_xs);
-    root->band_xs = nullptr;
+    const int rc = give_up(root, &root->band_xs, &root->band_xs_captured);
+    if (rc != SGNN_OK) return rc;
     root->band_xs_floats = 0;
     root->xs_serial = 0;
     *ok = hipMalloc(&root->band_xs, floats * sizeof(float)) == hipSuccess;
@@ -2249,14 +2272,10 @@ static int grow_xs(sgnn_spmm_plan *root, size_t floats, bool *ok) {
 // array's values stay (where `keep` says that binding counts).  A captured product always fills, so that a replay neither
 // finds another array's values nor misses an edit; after one, every product does, since a replay may have come between.
 template <typename Schedule>
-static int values_due(const sgnn_spmm_plan *p, Schedule *s, const float *val, bool keep, hipStream_t st, bool *due) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    SGNN_HIP_CHECK(hipStreamIsCapturing(st, &cap));
-    if (cap != hipStreamCaptureStatusNone) s->graph_fills = true;
-    const bool stays = keep && val == p->bound_val && !s->graph_fills;
-    *due = !stays || s->val_gen != p->bind_gen;
+static bool values_due(const sgnn_spmm_plan *p, Schedule *s, const float *val, bool keep) {
+    const bool stays = keep && val == p->bound_val && !s->captured, due = !stays || s->val_gen != p->bind_gen;
     s->val_gen = stays ? p->bind_gen : 0;
-    return SGNN_OK;
+    return due;
 }
 
 // The product through the band schedule.  may_build = false (the non-allocating entry point): use a schedule
@@ -2282,12 +2301,14 @@ static int spmm_run_band(sgnn_spmm_plan *p, const BandWindows &bw, const float *
             // A plan keeps the schedules of at most kMaxBandSchedules band widths (each holds a band-major copy of
             // the edge list): the one used longest ago makes room.
             if (p->bands.size() >= (size_t)kMaxBandSchedules) {
-                SGNN_HIP_CHECK(hipDeviceSynchronize());   // queued launches may still read it
-                size_t victim = 0;
-                for (size_t i = 1; i < p->bands.size(); ++i)
-                    if (p->bands[i]->last_use < p->bands[victim]->last_use) victim = i;
-                delete p->bands[victim];
-                p->bands.erase(p->bands.begin() + (long)victim);
+                size_t victim = p->bands.size();
+                for (size_t i = 0; i < p->bands.size(); ++i)
+                    if (!p->bands[i]->captured && (victim == p->bands.size() || p->bands[i]->last_use < p->bands[victim]->last_use)) victim = i;
+                if (victim < p->bands.size()) {
+                    SGNN_HIP_CHECK(hipDeviceSynchronize());   // queued launches may still read it
+                    delete p->bands[victim];
+                    p->bands.erase(p->bands.begin() + (long)victim);
+                }
             }
             rc = band_build(p, sh0.band_cols, sh0.n_bands, st, &bs);
             if (rc == SGNN_ERR_HIP && band_build_out_of_memory()) return SGNN_OK;  // no room for the band-major copy: the row-class schedule runs
@@ -2314,12 +2335,13 @@ static int spmm_run_band(sgnn_spmm_plan *p, const BandWindows &bw, const float *
         }
         cls[w] = cl;
     }
+    bool capturing = false;
+    const int crc = is_capturing(st, &capturing);
+    if (crc != SGNN_OK) return crc;
+    if (capturing) bs->captured = root->band_xs_captured = true;
     const float *val_bm = nullptr;
     if (weighted) {
-        bool due = false;
-        const int rc = values_due(p, bs, val, true, st, &due);
-        if (rc != SGNN_OK) return rc;
-        if (due)
+        if (values_due(p, bs, val, true))
             hipLaunchKernelGGL(permute_values_kernel, dim3((uint32_t)((p->nnz + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, val,
                                bs->eperm_bm, bs->val_bm, p->nnz);
         val_bm = bs->val_bm;
@@ -2454,16 +2476,15 @@ static int spmm_run_tile(sgnn_spmm_plan *p, int rows, const float *val, const De
     sgnn_spmm_plan *root = p->whole ? p->whole : p;
     const int n_slices = (int)((F + 63) / 64);
     const size_t xs_floats = (size_t)n_slices * (size_t)p->K * 64 + kTileCols * 64;   // the last tile may reach beyond the last row
+    bool capturing = false;
+    const int crc = is_capturing(st, &capturing);
+    if (crc != SGNN_OK) return crc;
     TileSchedule *ts = nullptr;
     for (TileSchedule *c : p->tiles)
         if (c->rows_per_wave == rows) ts = c;
-    if (ts == nullptr || xs_floats > root->band_xs_floats) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (may_build) SGNN_HIP_CHECK(hipStreamIsCapturing(st, &cap));
-        if (!may_build || cap != hipStreamCaptureStatusNone) {   // nothing can be built: the streams of another row count do
-            if (ts == nullptr && !p->tiles.empty()) ts = p->tiles[0];
-            if (ts == nullptr || xs_floats > root->band_xs_floats) return SGNN_OK;
-        }
+    if ((ts == nullptr || xs_floats > root->band_xs_floats) && (!may_build || capturing)) {   // nothing can be built: the streams of another row count do
+        if (ts == nullptr && !p->tiles.empty()) ts = p->tiles[0];
+        if (ts == nullptr || xs_floats > root->band_xs_floats) return SGNN_OK;
     }
     if (ts == nullptr) {
         bool sorted = false;
@@ -2472,7 +2493,8 @@ static int spmm_run_tile(sgnn_spmm_plan *p, int rows, const float *val, const De
         if (!sorted) return SGNN_OK;
         if (p->tiles.size() >= (size_t)kMaxTileSchedules) {
             SGNN_HIP_CHECK(hipDeviceSynchronize());   // queued launches may still read it
-            const size_t victim = p->tiles[0]->last_use < p->tiles[1]->last_use ? 0 : 1;
+            const size_t victim = p->tiles[0]->captured || (p->tiles[1]->last_use < p->tiles[0]->last_use && !p->tiles[1]->captured) ? 1 : 0;
+            if (p->tiles[victim]->captured) return SGNN_OK;
             delete p->tiles[victim];
             p->tiles.erase(p->tiles.begin() + (long)victim);
         }
@@ -2487,17 +2509,13 @@ static int spmm_run_tile(sgnn_spmm_plan *p, int rows, const float *val, const De
         const int rc = grow_xs(root, xs_floats, &ok);
         if (rc != SGNN_OK || !ok) return rc;
     }
-    if (val != nullptr) {
-        // Without long rows the row classes read the caller's array in every product, so edits of it count here as well.
-        // (20 k rows of 65 edges, F = 602: the fill is 10 of 145 us; 114 M edges: 0.6 of 11.0 ms, saved where the values are bound)
-        bool due = false;
-        const int rc = values_due(p, ts, val, p->long_edges > 0, st, &due);
-        if (rc != SGNN_OK) return rc;
-        if (due) {
-            const int64_t slots = ts->batches * kTileBatch;
-            hipLaunchKernelGGL(tile_values_kernel, dim3((uint32_t)((slots + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, val, ts->slot_edge,
-                               ts->stream, slots);
-        }
+    if (capturing) ts->captured = root->band_xs_captured = true;
+    // Without long rows the row classes read the caller's array in every product, so edits of it count here as well.
+    // (20 k rows of 65 edges, F = 602: the fill is 10 of 145 us; 114 M edges: 0.6 of 11.0 ms, saved where the values are bound)
+    if (val != nullptr && values_due(p, ts, val, p->long_edges > 0)) {
+        const int64_t slots = ts->batches * kTileBatch;
+        hipLaunchKernelGGL(tile_values_kernel, dim3((uint32_t)((slots + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, val, ts->slot_edge,
+                           ts->stream, slots);
     }
     if (p->whole == nullptr) ++root->call_serial;
     ts->last_use = ++root->band_use_clock;
@@ -2669,15 +2687,16 @@ static int spmm_run(sgnn_spmm_plan *p, const float *val, const DenseSrc &dense, 
         partial = scratch;
     } else if (p->n_items > 0) {
         const size_t need = (size_t)p->n_items * (size_t)F;
+        bool capturing = false;
+        int rc = is_capturing(st, &capturing);
+        if (rc != SGNN_OK) return rc;
         if (need > p->partial_floats) {
-            // The old buffer may still be read by work queued on another stream: drain first.
-            SGNN_HIP_CHECK(hipDeviceSynchronize());
-            (void)hipFree(p->partial);
-            p->partial = nullptr;
+            if ((rc = give_up(p, &p->partial, &p->partial_captured)) != SGNN_OK) return rc;
             p->partial_floats = 0;
             SGNN_HIP_CHECK(hipMalloc(&p->partial, need * sizeof(float)));
             p->partial_floats = need;
         }
+        if (capturing) p->partial_captured = true;
         partial = p->partial;
     }
     const int nvec = (int)(F / vec);

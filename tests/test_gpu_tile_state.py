@@ -108,3 +108,27 @@ def test_replays_and_eager_products_do_not_see_each_others_values(kind, bound, m
         graph.replay()
         c.check(c.value, what=("replay of edited values", i))
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("kind", ["tiles", "bands", "row classes"])
+def test_captured_products_keep_their_buffers(kind, monkeypatch):
+    """Wider products later on need a larger workspace, other schedules of the same matrix and larger partial sums; what a
+    captured product names stays."""
+    monkeypatch.setenv("SGNN_SPMM_BAND", {"tiles": "2", "bands": "1", "row classes": "0"}[kind])
+    c = _Case(1500, 1200, 30, 64, hubs=6, hub_deg=700)
+    for _ in range(3):
+        c.product(c.value)
+    first = c.out.clone()
+    graph = _captured(c, c.value)
+    for F in (80, 96, 112, 130, 602):
+        x = c.operand(F)
+        wide = torch.empty(c.M, F, device=DEV)
+        c.product(c.value, x, wide)
+        if kind != "row classes":
+            c.check(c.value, x, wide, what=F)
+        fresh = [torch.full((1 << 20,), float("nan"), device=DEV) for _ in range(8)]   # whatever has been freed is written over
+        c.out.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c.out, first), F
+        del fresh
