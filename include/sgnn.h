@@ -104,7 +104,8 @@ int sgnn_spmm_plan_schedule(const sgnn_spmm_plan *plan, int64_t F, int64_t info[
 /* The tile schedule, which matrices with many edges per block of rows and columns take instead of the band schedule: 15
  * wavefronts of a workgroup keep info[0] rows each in registers (0: the product does not take it) while the dense operand
  * streams through LDS.  Same order of operations, so the same bits.  info[1] = edge streams the plan holds (one per number
- * of rows, two at most; built on the first call that wants one). */
+ * of rows, three at most; built on the first call that wants one and kept: a width that finds no place takes the held streams
+ * that suit it best). */
 int sgnn_spmm_plan_tiles(const sgnn_spmm_plan *plan, int64_t F, int64_t info[2]);
 
 /* How the row-class schedule walks the short rows for the same operand: info[0] = chunks of short rows, info[1] = dense rows

@@ -1398,7 +1398,6 @@ struct TileSchedule {
     int32_t *slot_edge = nullptr;      // [batches * kTileBatch] CSR index of every slot, -1: padding
     uint64_t val_gen = 0;              // plan bind generation the values were filled under (0: not from a bound array)
     bool captured = false;             // a captured product names these buffers
-    uint64_t last_use = 0;
     ~TileSchedule() {
         (void)hipFree(stream); (void)hipFree(batch0); (void)hipFree(slot_edge);
     }
@@ -2395,7 +2394,8 @@ static int spmm_run_band(sgnn_spmm_plan *p, const BandWindows &bw, const float *
 // Tile schedule, host side.
 // ------------------------------------------------------------------------------------------------
 constexpr double kTileSpread = 1.25;   // see tile_build
-constexpr int kMaxTileSchedules = 2;   // row counts a plan keeps streams for (12 bytes per edge each)
+constexpr int kMaxTileSchedules = 3;   // row counts a plan keeps streams for (12 bytes per slot each)
+constexpr double kTileBuildGain = 0.9; // share of the held streams' estimate below which another row count gets its own
 
 // Estimated time of a product, in clocks of the chip: the rounds of workgroups times the tiles of a sweep times the clocks
 // of a tile, which go with its edges (240 edges of 104 columns 1480 clocks, 640 2950, 4800 20800) down to what the stream
@@ -2405,6 +2405,11 @@ static double tile_clocks(const sgnn_spmm_plan *p, int64_t F, int rows) {
     const double blocks = (double)((p->M + (int64_t)rows * kTileConsumers - 1) / ((int64_t)rows * kTileConsumers));
     const double e = (double)p->nnz / (double)p->M * rows * kTileConsumers / tiles;
     return std::ceil(blocks * slices / 256.0) * tiles * std::max(1200.0, std::max(600.0 + 3.7 * e, 4.3 * e));
+}
+
+// The estimate to stay below: that of the band schedule, 8.9 clocks per edge of 64 floats and CU, less a tenth.
+static double tile_others(const sgnn_spmm_plan *p, int64_t F) {
+    return env_int("SGNN_SPMM_BAND", -1) > 1 ? 1e300 : 0.9 * 8.9 * (double)p->nnz * (double)F / 64.0 / 256.0;
 }
 
 // How the tile schedule would take a product of width F: rows per wave, 0 where it is not the one to use as far as the shape
@@ -2418,12 +2423,12 @@ static int tile_rows(const sgnn_spmm_plan *p, int64_t F) {
     // One chain of fmas per row: where the row classes would take the product, which add up long rows in parts, only if there
     // are none (a chain of 370 edges is off by 3.0e-7, the parts by 1.3e-7).
     if (mode < 2 && p->long_edges > 0 && !band_wanted(p, F, band_windows(p, F, true).w[0])) return 0;
-    const double others = 0.9 * 8.9 * (double)p->nnz * (double)F / 64.0 / 256.0;   // band schedule: 8.9 clocks per edge of 64 floats and CU
-    if (mode < 2 && (double)((p->K + kTileCols - 1) / kTileCols) * 1200.0 > others) return 0;
+    const double others = tile_others(p, F);
+    if ((double)((p->K + kTileCols - 1) / kTileCols) * 1200.0 > others) return 0;
     int best = kTileRows;
     for (int r = kTileRows; r >= 16; r -= 3)
         if (tile_clocks(p, F, r) < 0.97 * tile_clocks(p, F, best)) best = r;
-    return mode > 1 || tile_clocks(p, F, best) < others ? best : 0;
+    return tile_clocks(p, F, best) < others ? best : 0;
 }
 
 static int tile_build(sgnn_spmm_plan *p, int rows, hipStream_t st, TileSchedule **out) {
@@ -2469,6 +2474,32 @@ static int tile_build(sgnn_spmm_plan *p, int rows, hipStream_t st, TileSchedule 
     return SGNN_OK;
 }
 
+// The streams that a product of width F takes: the held ones with the lowest estimate, or streams built for `rows` where that
+// is clearly lower still and a place is free.  The result does not depend on the number of rows, so nothing is ever evicted and
+// widths in turn settle on what there is.  *ts stays null where the other schedules are to run.
+static int tile_streams(sgnn_spmm_plan *p, std::vector<TileSchedule *> &held, int64_t F, int rows, hipStream_t st, bool may_build,
+                        TileSchedule **ts) {
+    for (TileSchedule *c : held)
+        if (*ts == nullptr || tile_clocks(p, F, c->rows_per_wave) < tile_clocks(p, F, (*ts)->rows_per_wave)) *ts = c;
+    const double have = *ts ? tile_clocks(p, F, (*ts)->rows_per_wave) : 1e300;
+    if (may_build && held.size() < (size_t)kMaxTileSchedules && tile_clocks(p, F, rows) < kTileBuildGain * have) {
+        bool sorted = false;
+        int rc = band_rows_sorted(p, st, &sorted);
+        if (rc != SGNN_OK || !sorted) return rc;
+        TileSchedule *made = nullptr;
+        rc = tile_build(p, rows, st, &made);
+        if (rc == SGNN_ERR_HIP && band_build_out_of_memory()) rc = SGNN_OK;   // no room: what there is runs
+        if (rc != SGNN_OK) return rc;
+        if (made != nullptr) {
+            held.push_back(made);
+            *ts = made;
+            return SGNN_OK;
+        }
+    }
+    if (*ts != nullptr && have >= tile_others(p, F)) *ts = nullptr;
+    return SGNN_OK;
+}
+
 // The product through the tile schedule; as spmm_run_band.
 static int spmm_run_tile(sgnn_spmm_plan *p, int rows, const float *val, const DenseSrc &dense, float *out, int64_t F, int64_t ldo,
                          int accumulate, const float *row_div, hipStream_t st, bool may_build, bool *done) {
@@ -2477,36 +2508,16 @@ static int spmm_run_tile(sgnn_spmm_plan *p, int rows, const float *val, const De
     const int n_slices = (int)((F + 63) / 64);
     const size_t xs_floats = (size_t)n_slices * (size_t)p->K * 64 + kTileCols * 64;   // the last tile may reach beyond the last row
     bool capturing = false;
-    const int crc = is_capturing(st, &capturing);
-    if (crc != SGNN_OK) return crc;
+    int rc = is_capturing(st, &capturing);
+    if (rc != SGNN_OK) return rc;
+    may_build = may_build && !capturing;
     TileSchedule *ts = nullptr;
-    for (TileSchedule *c : p->tiles)
-        if (c->rows_per_wave == rows) ts = c;
-    if ((ts == nullptr || xs_floats > root->band_xs_floats) && (!may_build || capturing)) {   // nothing can be built: the streams of another row count do
-        if (ts == nullptr && !p->tiles.empty()) ts = p->tiles[0];
-        if (ts == nullptr || xs_floats > root->band_xs_floats) return SGNN_OK;
-    }
-    if (ts == nullptr) {
-        bool sorted = false;
-        int rc = band_rows_sorted(p, st, &sorted);
-        if (rc != SGNN_OK) return rc;
-        if (!sorted) return SGNN_OK;
-        if (p->tiles.size() >= (size_t)kMaxTileSchedules) {
-            SGNN_HIP_CHECK(hipDeviceSynchronize());   // queued launches may still read it
-            const size_t victim = p->tiles[0]->captured || (p->tiles[1]->last_use < p->tiles[0]->last_use && !p->tiles[1]->captured) ? 1 : 0;
-            if (p->tiles[victim]->captured) return SGNN_OK;
-            delete p->tiles[victim];
-            p->tiles.erase(p->tiles.begin() + (long)victim);
-        }
-        rc = tile_build(p, rows, st, &ts);
-        if (rc == SGNN_ERR_HIP && band_build_out_of_memory()) return SGNN_OK;   // no room: the other schedules run
-        if (rc != SGNN_OK) return rc;
-        if (ts == nullptr) return SGNN_OK;
-        p->tiles.push_back(ts);
-    }
+    rc = tile_streams(p, p->tiles, F, rows, st, may_build, &ts);
+    if (rc != SGNN_OK || ts == nullptr) return rc;
     if (xs_floats > root->band_xs_floats) {
+        if (!may_build) return SGNN_OK;
         bool ok = false;
-        const int rc = grow_xs(root, xs_floats, &ok);
+        rc = grow_xs(root, xs_floats, &ok);
         if (rc != SGNN_OK || !ok) return rc;
     }
     if (capturing) ts->captured = root->band_xs_captured = true;
@@ -2518,7 +2529,6 @@ static int spmm_run_tile(sgnn_spmm_plan *p, int rows, const float *val, const De
                            ts->stream, slots);
     }
     if (p->whole == nullptr) ++root->call_serial;
-    ts->last_use = ++root->band_use_clock;
     // the restaged operand of this layout is told from a band schedule's by its slice count's sign
     if (!(root->xs_serial == root->call_serial && root->xs_F == (int)F && root->xs_slices == -n_slices)) {
         ProfScope prof(K_SPMM_BAND_RESTAGE, st, may_build);

@@ -132,3 +132,24 @@ def test_captured_products_keep_their_buffers(kind, monkeypatch):
         torch.cuda.synchronize()
         assert torch.equal(c.out, first), F
         del fresh
+
+
+def test_widths_in_turn_settle_on_the_streams_there_are(monkeypatch):
+    """Four widths that each want another number of rows per wave: three get streams of their own, and from then on nothing
+    is built (streams are never given up, so their number says so); a product captured on the first width goes on."""
+    monkeypatch.setenv("SGNN_SPMM_BAND", "2")
+    widths = (64, 256, 602, 1024)
+    c = _Case(40000, 2500, 30, widths[0])
+    assert len({c.plan.tiles(F)[0] for F in widths}) == 4
+    c.product(c.value)
+    graph = _captured(c, c.value)
+    for turn in range(3):
+        for F in widths:
+            x, out = c.operand(F), torch.empty(c.M, F, device=DEV)
+            c.product(c.value, x, out)
+            c.check(c.value, x, out, what=(turn, F))
+        assert c.plan.tiles(widths[0])[1] == 3, turn
+        c.out.fill_(7.0)
+        graph.replay()
+        c.check(c.value, what=("replay", turn))
+        torch.cuda.synchronize()
