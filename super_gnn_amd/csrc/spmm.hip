@@ -1435,7 +1435,8 @@ struct sgnn_spmm_plan {
     uint64_t bind_gen = 1;          // bumped by every sgnn_spmm_plan_bind_values
     std::vector<BandSchedule *> bands;
     std::vector<TileSchedule *> tiles;
-    double tile_spread = 0.0;       // batches of the row blocks' longest streams over their average (0: not known)
+    std::vector<float> tile_spread; // per number of rows a wave (tile_candidate): see tile_measure
+    bool tile_too_many = false;     // more batches than the streams can number
     float *band_xs = nullptr;       // the dense operand restaged slice by slice (see band_restage_kernel), grown on demand
     size_t band_xs_floats = 0;
     bool band_xs_captured = false, partial_captured = false;   // a captured product names the buffer
@@ -1529,6 +1530,32 @@ static int upload(T **dst, const std::vector<T> &src, hipStream_t st) {
     SGNN_HIP_CHECK(hipMalloc(dst, sizeof(T) * src.size()));
     SGNN_HIP_CHECK(hipMemcpyAsync(*dst, src.data(), sizeof(T) * src.size(), hipMemcpyHostToDevice, st));
     return SGNN_OK;
+}
+
+// Numbers of rows a wave that the tile schedule chooses from: 103, 100, ... 16.
+constexpr int kTileCandidates = 30;
+static int tile_candidate(int i) { return kTileRows - 3 * i; }
+
+// A workgroup of the tile schedule takes as long as its longest stream.  For every number of rows, the batches of the row
+// blocks' longest streams over their average, so that it is known before anything is built which numbers are not for this
+// matrix (rows of very different lengths: none).
+static void tile_measure(sgnn_spmm_plan *p) {
+    if (p->K > (int64_t)kTileMax * kTileCols || (double)p->nnz * 2000.0 < (double)p->M * (double)p->K) return;   // (see tile_rows)
+    for (int i = 0; i < kTileCandidates; ++i) {
+        const int64_t rows = tile_candidate(i);
+        int64_t longest = 0, all = 0;
+        for (int64_t b = 0; b < p->M; b += rows * kTileConsumers) {
+            int64_t most = 1;
+            for (int w = 0; w < kTileConsumers; ++w) {
+                const int64_t r0 = std::min(p->M, b + w * rows), r1 = std::min(p->M, r0 + rows);
+                const int64_t n = (p->h_rowptr[(size_t)r1] - p->h_rowptr[(size_t)r0] + kTileBatch - 1) / kTileBatch + 1;
+                most = std::max(most, n);
+                all += n;
+            }
+            longest += most;
+        }
+        p->tile_spread.push_back(all > 0 ? (float)((double)longest * kTileConsumers / (double)all) : 1.0f);
+    }
 }
 
 static int plan_create_impl(sgnn_spmm_plan *p, const int64_t *rowptr, const void *col, int col_is_i64,
@@ -1685,6 +1712,7 @@ static int plan_create_impl(sgnn_spmm_plan *p, const int64_t *rowptr, const void
         if ((rc = upload(&p->cls_work, cls_work, st)) != SGNN_OK) return rc;
     }
     SGNN_HIP_CHECK(hipStreamSynchronize(st));  // the host vectors die at return
+    tile_measure(p);
     // The short-row chunk lists of all three lane-group shapes (a few MB in total): no later call has
     // to build, and therefore allocate, one.
     for (int which = 0; which < 3; ++which)
@@ -2393,7 +2421,7 @@ static int spmm_run_band(sgnn_spmm_plan *p, const BandWindows &bw, const float *
 // ------------------------------------------------------------------------------------------------
 // Tile schedule, host side.
 // ------------------------------------------------------------------------------------------------
-constexpr double kTileSpread = 1.25;   // see tile_build
+constexpr double kTileSpread = 1.25;   // see tile_measure
 constexpr int kMaxTileSchedules = 3;   // row counts a plan keeps streams for (12 bytes per slot each)
 constexpr double kTileBuildGain = 0.9; // share of the held streams' estimate below which another row count gets its own
 
@@ -2419,16 +2447,19 @@ static int tile_rows(const sgnn_spmm_plan *p, int64_t F) {
     const int mode = env_int("SGNN_SPMM_BAND", -1);
     if (mode == 0 || mode == 1) return 0;
     // (below a density of 1 / 2000 the stream of the operand alone takes longer than the other schedules)
-    if (mode < 2 && (p->tile_spread > kTileSpread || (double)p->nnz * 2000.0 < (double)p->M * (double)p->K)) return 0;
+    if (p->tile_too_many || (mode < 2 && (double)p->nnz * 2000.0 < (double)p->M * (double)p->K)) return 0;
     // One chain of fmas per row: where the row classes would take the product, which add up long rows in parts, only if there
     // are none (a chain of 370 edges is off by 3.0e-7, the parts by 1.3e-7).
     if (mode < 2 && p->long_edges > 0 && !band_wanted(p, F, band_windows(p, F, true).w[0])) return 0;
     const double others = tile_others(p, F);
     if ((double)((p->K + kTileCols - 1) / kTileCols) * 1200.0 > others) return 0;
-    int best = kTileRows;
-    for (int r = kTileRows; r >= 16; r -= 3)
-        if (tile_clocks(p, F, r) < 0.97 * tile_clocks(p, F, best)) best = r;
-    return tile_clocks(p, F, best) < others ? best : 0;
+    int best = 0;
+    for (int i = 0; i < kTileCandidates; ++i) {
+        const int r = tile_candidate(i);
+        if (mode < 2 && p->tile_spread[(size_t)i] > kTileSpread) continue;
+        if (best == 0 || tile_clocks(p, F, r) < 0.97 * tile_clocks(p, F, best)) best = r;
+    }
+    return best > 0 && tile_clocks(p, F, best) < others ? best : 0;
 }
 
 static int tile_build(sgnn_spmm_plan *p, int rows, hipStream_t st, TileSchedule **out) {
@@ -2445,21 +2476,12 @@ static int tile_build(sgnn_spmm_plan *p, int rows, hipStream_t st, TileSchedule 
     std::vector<int32_t> h, first((size_t)waves);
     const int rc = download(h, counts.p, (size_t)waves, st);
     if (rc != SGNN_OK) return rc;
-    int64_t longest = 0;
-    for (int64_t b = 0; b < ts->n_rb; ++b) {
-        int32_t most = 0;
-        for (int w = 0; w < kTileConsumers; ++w) {
-            const size_t i = (size_t)(b * kTileConsumers + w);
-            first[i] = (int32_t)ts->batches;
-            ts->batches += h[i];
-            most = std::max(most, h[i]);
-        }
-        longest += most;
+    for (size_t i = 0; i < (size_t)waves; ++i) {
+        first[i] = (int32_t)ts->batches;
+        ts->batches += h[i];
     }
-    p->tile_spread = (double)longest * kTileConsumers / (double)ts->batches;
-    // a workgroup takes as long as its longest stream: rows of very different lengths are not for this schedule
-    if (ts->batches > (INT32_MAX >> 5) || (p->tile_spread > kTileSpread && env_int("SGNN_SPMM_BAND", -1) < 2)) {
-        p->tile_spread = 1e9;
+    if (ts->batches > (INT32_MAX >> 5)) {
+        p->tile_too_many = true;
         return SGNN_OK;
     }
     SGNN_BAND_ALLOC(&ts->stream, (size_t)ts->batches * (8 * kTileBatch) + kTileSlack);

@@ -153,3 +153,48 @@ def test_widths_in_turn_settle_on_the_streams_there_are(monkeypatch):
         graph.replay()
         c.check(c.value, what=("replay", turn))
         torch.cuda.synchronize()
+
+
+def test_a_width_that_tiles_do_not_suit_leaves_the_others_theirs():
+    """Rows of 300 and 120 edges in turns of 32: 103 rows a wave are even enough, a few are not.  A width that wants few must not
+    turn off the streams of one that wants many, for calls that may build nothing either (the row classes they would fall
+    back to add long rows up in parts: other bits)."""
+    from super_gnn_amd import supergnn_ops as ops
+    from super_gnn_amd._lib import check, lib
+    M, K, many, few = 24000, 40000, 1024, 320
+    rng = np.random.default_rng(5)
+    deg = np.where(np.arange(M) // 32 % 2 == 0, 300, 120)
+    rowptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int64)
+    col = rng.integers(0, K, size=rowptr[-1])
+    col = col[np.lexsort((col, np.repeat(np.arange(M), deg)))]
+    plan = ops.SpmmPlan(torch.from_numpy(rowptr).to(DEV), torch.from_numpy(col).to(DEV), K)
+    x = {F: torch.randn(K, F, generator=torch.Generator().manual_seed(F)).to(DEV) for F in (many, few)}
+    out = torch.empty(M, many, device=DEV)
+    assert plan.tiles(many)[0] == 103
+
+    def noalloc(F, out):
+        check(lib.sgnn_spmm_csr_f32_noalloc(plan._h, None, x[F].data_ptr(), out.data_ptr(), F, F, F, 0, None, torch.cuda.current_stream().cuda_stream))
+
+    plan.run(None, x[many], out, accumulate=False)
+    first = out.clone()
+    lo, hi = rowptr[1000], rowptr[1100]
+    want = np.zeros((100, many), np.float32)
+    orc.spmm_accumulate(rowptr[1000:1101] - lo, col[lo:hi], np.ones(hi - lo, np.float32), x[many].cpu().numpy(), want)
+    equal = np.array_equal(first[1000:1100].cpu().numpy(), want)
+    assert equal
+    for _ in range(2):
+        narrow = torch.empty(M, few, device=DEV)
+        plan.run(None, x[few], narrow, accumulate=False)
+    assert plan.tiles(many)[0] == 103
+    out.fill_(7.0)
+    noalloc(many, out)
+    assert torch.equal(out, first)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        plan.run(None, x[many], out, accumulate=False)
+    for _ in range(3):
+        out.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, first)
