@@ -22,6 +22,7 @@
 //     each XCD gathers only its own class of dense rows, so the eight L2 caches hold disjoint sets
 //     of popular rows.
 #include <algorithm>
+#include <atomic>
 #include <cstdlib>
 #include <functional>
 #include <list>
@@ -1403,6 +1404,24 @@ struct TileSchedule {
     }
 };
 
+// The tile schedule's state for products that the row classes would take otherwise, which keep none: of a matrix without long
+// rows products on several streams, from several threads and in captured graphs do not know of each other.  So this state
+// belongs to one product in flight at a time, and any other one runs the row classes, with the same bits.
+struct TileAlone {
+    std::mutex mu;
+    std::vector<TileSchedule *> tiles;
+    float *xs = nullptr;               // the restaged operand
+    size_t xs_floats = 0;
+    hipEvent_t done = nullptr;         // behind the last product, on `stream`
+    hipStream_t stream = nullptr;
+    bool used = false;
+    ~TileAlone() {
+        for (TileSchedule *t : tiles) delete t;
+        (void)hipFree(xs);
+        if (done) (void)hipEventDestroy(done);
+    }
+};
+
 struct sgnn_spmm_plan {
     int device = 0;
     int64_t M = 0, K = 0, nnz = 0;
@@ -1431,12 +1450,13 @@ struct sgnn_spmm_plan {
     int32_t *empty_rows = nullptr;
     int64_t n_empty = 0;
     // Band schedules (dense-degree matrices), built on first use for a band width.
-    int cols_sorted = -1;           // -1 unknown, 0 some row's columns are out of order, 1 every row is column-sorted
+    std::atomic<int> cols_sorted{-1};   // -1 unknown, 0 some row's columns are out of order, 1 every row is column-sorted
     uint64_t bind_gen = 1;          // bumped by every sgnn_spmm_plan_bind_values
     std::vector<BandSchedule *> bands;
     std::vector<TileSchedule *> tiles;
+    TileAlone tile_alone;
     std::vector<float> tile_spread; // per number of rows a wave (tile_candidate): see tile_measure
-    bool tile_too_many = false;     // more batches than the streams can number
+    std::atomic<bool> tile_too_many{false};   // more batches than the streams can number
     float *band_xs = nullptr;       // the dense operand restaged slice by slice (see band_restage_kernel), grown on demand
     size_t band_xs_floats = 0;
     bool band_xs_captured = false, partial_captured = false;   // a captured product names the buffer
@@ -2450,7 +2470,8 @@ static int tile_rows(const sgnn_spmm_plan *p, int64_t F) {
     if (p->tile_too_many || (mode < 2 && (double)p->nnz * 2000.0 < (double)p->M * (double)p->K)) return 0;
     // One chain of fmas per row: where the row classes would take the product, which add up long rows in parts, only if there
     // are none (a chain of 370 edges is off by 3.0e-7, the parts by 1.3e-7).
-    if (mode < 2 && p->long_edges > 0 && !band_wanted(p, F, band_windows(p, F, true).w[0])) return 0;
+    // (Row blocks keep their state in the whole plan, so those that the row classes would take stay there too.)
+    if (mode < 2 && (p->long_edges > 0 || p->whole != nullptr) && !band_wanted(p, F, band_windows(p, F, true).w[0])) return 0;
     const double others = tile_others(p, F);
     if ((double)((p->K + kTileCols - 1) / kTileCols) * 1200.0 > others) return 0;
     int best = 0;
@@ -2522,44 +2543,14 @@ static int tile_streams(sgnn_spmm_plan *p, std::vector<TileSchedule *> &held, in
     return SGNN_OK;
 }
 
-// The product through the tile schedule; as spmm_run_band.
-static int spmm_run_tile(sgnn_spmm_plan *p, int rows, const float *val, const DenseSrc &dense, float *out, int64_t F, int64_t ldo,
-                         int accumulate, const float *row_div, hipStream_t st, bool may_build, bool *done) {
-    *done = false;
-    sgnn_spmm_plan *root = p->whole ? p->whole : p;
+static size_t tile_xs_floats(const sgnn_spmm_plan *p, int64_t F) {
+    return (size_t)((F + 63) / 64) * (size_t)p->K * 64 + kTileCols * 64;   // the last tile may reach beyond the last row
+}
+
+// What a product launches: the values into the streams and the operand into xs, where asked for, and the product itself.
+static int tile_launch(const sgnn_spmm_plan *p, const TileSchedule *ts, float *xs, bool restage, const float *val, bool fill, const DenseSrc &dense,
+                       float *out, int64_t F, int64_t ldo, int accumulate, const float *row_div, hipStream_t st, bool may_prof) {
     const int n_slices = (int)((F + 63) / 64);
-    const size_t xs_floats = (size_t)n_slices * (size_t)p->K * 64 + kTileCols * 64;   // the last tile may reach beyond the last row
-    bool capturing = false;
-    int rc = is_capturing(st, &capturing);
-    if (rc != SGNN_OK) return rc;
-    may_build = may_build && !capturing;
-    TileSchedule *ts = nullptr;
-    rc = tile_streams(p, p->tiles, F, rows, st, may_build, &ts);
-    if (rc != SGNN_OK || ts == nullptr) return rc;
-    if (xs_floats > root->band_xs_floats) {
-        if (!may_build) return SGNN_OK;
-        bool ok = false;
-        rc = grow_xs(root, xs_floats, &ok);
-        if (rc != SGNN_OK || !ok) return rc;
-    }
-    if (capturing) ts->captured = root->band_xs_captured = true;
-    // Without long rows the row classes read the caller's array in every product, so edits of it count here as well.
-    // (20 k rows of 65 edges, F = 602: the fill is 10 of 145 us; 114 M edges: 0.6 of 11.0 ms, saved where the values are bound)
-    if (val != nullptr && values_due(p, ts, val, p->long_edges > 0)) {
-        const int64_t slots = ts->batches * kTileBatch;
-        hipLaunchKernelGGL(tile_values_kernel, dim3((uint32_t)((slots + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, val, ts->slot_edge,
-                           ts->stream, slots);
-    }
-    if (p->whole == nullptr) ++root->call_serial;
-    // the restaged operand of this layout is told from a band schedule's by its slice count's sign
-    if (!(root->xs_serial == root->call_serial && root->xs_F == (int)F && root->xs_slices == -n_slices)) {
-        ProfScope prof(K_SPMM_BAND_RESTAGE, st, may_build);
-        const int64_t n = (int64_t)n_slices * p->K * 16;
-        hipLaunchKernelGGL(band_restage_kernel, dim3((uint32_t)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, dense.x, dense.ldx,
-                           root->band_xs, p->K, (int)F, 64, 64, n_slices);
-        root->xs_serial = root->call_serial;
-        root->xs_F = (int)F; root->xs_slice_pad = 64; root->xs_slices = -n_slices;
-    }
     auto kernel = val ? spmm_tile_kernel<true> : spmm_tile_kernel<false>;
     {
         static std::mutex mu;
@@ -2571,16 +2562,118 @@ static int spmm_run_tile(sgnn_spmm_plan *p, int rows, const float *val, const De
             allowed = true;
         }
     }
+    if (fill) {
+        const int64_t slots = ts->batches * kTileBatch;
+        hipLaunchKernelGGL(tile_values_kernel, dim3((uint32_t)((slots + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, val, ts->slot_edge,
+                           ts->stream, slots);
+    }
+    if (restage) {
+        ProfScope prof(K_SPMM_BAND_RESTAGE, st, may_prof);
+        const int64_t n = (int64_t)n_slices * p->K * 16;
+        hipLaunchKernelGGL(band_restage_kernel, dim3((uint32_t)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, dense.x, dense.ldx, xs, p->K,
+                           (int)F, 64, 64, n_slices);
+    }
     {
-        ProfScope prof(K_SPMM_BAND, st, may_build);
+        ProfScope prof(K_SPMM_BAND, st, may_prof);
         const int64_t total = ts->n_rb * n_slices;
-        const TileArgs a{root->band_xs, p->K, ts->stream, ts->batch0, out, row_div, p->M, ldo, ts->tiles, ts->rows_per_wave,
-                         (int)ts->n_rb, n_slices, (int)F, accumulate};
+        const TileArgs a{xs, p->K, ts->stream, ts->batch0, out, row_div, p->M, ldo, ts->tiles, ts->rows_per_wave, (int)ts->n_rb, n_slices, (int)F,
+                         accumulate};
         hipLaunchKernelGGL(kernel, dim3((uint32_t)((total + kNumXCD - 1) / kNumXCD * kNumXCD)), dim3(1024), kTileLds, st, a);
     }
     SGNN_HIP_CHECK(hipGetLastError());
+    return SGNN_OK;
+}
+
+// The product through the tile schedule in place of the band schedule; as spmm_run_band.
+static int spmm_run_tile(sgnn_spmm_plan *p, int rows, const float *val, const DenseSrc &dense, float *out, int64_t F, int64_t ldo,
+                         int accumulate, const float *row_div, hipStream_t st, bool may_build, bool *done) {
+    *done = false;
+    const bool prof = may_build;
+    sgnn_spmm_plan *root = p->whole ? p->whole : p;
+    const int n_slices = (int)((F + 63) / 64);
+    bool capturing = false;
+    int rc = is_capturing(st, &capturing);
+    if (rc != SGNN_OK) return rc;
+    may_build = may_build && !capturing;
+    TileSchedule *ts = nullptr;
+    rc = tile_streams(p, p->tiles, F, rows, st, may_build, &ts);
+    if (rc != SGNN_OK || ts == nullptr) return rc;
+    const size_t xs_floats = tile_xs_floats(p, F);
+    if (xs_floats > root->band_xs_floats) {
+        if (!may_build) return SGNN_OK;
+        bool ok = false;
+        rc = grow_xs(root, xs_floats, &ok);
+        if (rc != SGNN_OK || !ok) return rc;
+    }
+    if (capturing) ts->captured = root->band_xs_captured = true;
+    // Without long rows every product fills its values: the row classes read the caller's array there, so edits of it count here as
+    // well.  With them a bound array's stay (114 M edges: the fill is 0.6 of 11.0 ms).
+    if (p->whole == nullptr) ++root->call_serial;
+    // the restaged operand of this layout is told from a band schedule's by its slice count's sign
+    const bool restaged = root->xs_serial == root->call_serial && root->xs_F == (int)F && root->xs_slices == -n_slices;
+    rc = tile_launch(p, ts, root->band_xs, !restaged, val, val != nullptr && values_due(p, ts, val, p->long_edges > 0), dense, out, F, ldo,
+                     accumulate, row_div, st, prof);
+    if (rc != SGNN_OK) return rc;
+    root->xs_serial = root->call_serial;
+    root->xs_F = (int)F; root->xs_slice_pad = 64; root->xs_slices = -n_slices;
     *done = true;
     return SGNN_OK;
+}
+
+// Calls that another thread's capture in the runtime's global mode would refuse (allocations, event queries) are this thread's
+// own business for the life of this.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// The state of TileAlone made ready for a product of width F on stream st, false where something is in the way: another product
+// in flight on another stream, a capture, no memory.
+static bool tile_alone_ready(sgnn_spmm_plan *p, int rows, int64_t F, hipStream_t st, TileSchedule **ts) {
+    TileAlone &own = p->tile_alone;
+    bool capturing = true;
+    if (is_capturing(st, &capturing) != SGNN_OK || capturing) return false;
+    if (own.done == nullptr && hipEventCreateWithFlags(&own.done, hipEventDisableTiming) != hipSuccess) return false;
+    if (own.used && own.stream != st && hipEventQuery(own.done) != hipSuccess) return false;
+    try {
+        own.tiles.reserve(kMaxTileSchedules);
+        if (tile_streams(p, own.tiles, F, rows, st, true, ts) != SGNN_OK || *ts == nullptr) return false;
+    } catch (const std::bad_alloc &) {
+        return false;
+    }
+    const size_t floats = tile_xs_floats(p, F);
+    if (floats <= own.xs_floats) return true;
+    if (own.used && hipEventSynchronize(own.done) != hipSuccess) return false;
+    (void)hipFree(own.xs);
+    own.xs = nullptr;
+    own.xs_floats = 0;
+    if (hipMalloc(&own.xs, floats * sizeof(float)) != hipSuccess) return false;
+    own.xs_floats = floats;
+    return true;
+}
+
+// The product through the tile schedule in place of the row classes, which it is left to where the state is not to be had.
+static int spmm_run_tile_alone(sgnn_spmm_plan *p, int rows, const float *val, const DenseSrc &dense, float *out, int64_t F, int64_t ldo,
+                               int accumulate, const float *row_div, hipStream_t st, bool *done) {
+    *done = false;
+    if (st == hipStreamPerThread) return SGNN_OK;   // one handle, a stream of its own in every thread
+    TileAlone &own = p->tile_alone;
+    std::unique_lock<std::mutex> lock(own.mu, std::try_to_lock);
+    if (!lock.owns_lock()) return SGNN_OK;
+    RelaxedCapture relaxed;
+    TileSchedule *ts = nullptr;
+    if (!tile_alone_ready(p, rows, F, st, &ts)) {
+        (void)hipGetLastError();
+        return SGNN_OK;
+    }
+    // the caller's values, read by every product as the row classes read them (20 k rows of 65 edges, F = 602: 10 of 145 us)
+    const int rc = tile_launch(p, ts, own.xs, true, val, val != nullptr, dense, out, F, ldo, accumulate, row_div, st, true);
+    own.stream = st;
+    own.used = hipEventRecord(own.done, st) == hipSuccess;
+    if (!own.used) SGNN_HIP_CHECK(hipStreamSynchronize(st));
+    *done = rc == SGNN_OK;
+    return rc;
 }
 
 extern "C" int sgnn_spmm_plan_schedule(const sgnn_spmm_plan *p, int64_t F, int64_t info[4]) {
@@ -2598,7 +2691,7 @@ extern "C" int sgnn_spmm_plan_tiles(const sgnn_spmm_plan *p, int64_t F, int64_t 
     SGNN_REQUIRE(F > 0 && F < (1 << 24), "feature width F=%lld out of range", (long long)F);
     if (!p->parts.empty()) p = p->parts[0];
     info[0] = tile_rows(p, F);
-    info[1] = (int64_t)p->tiles.size();
+    info[1] = (int64_t)(p->tiles.size() + p->tile_alone.tiles.size());
     return SGNN_OK;
 }
 
@@ -2683,7 +2776,11 @@ static int spmm_run(sgnn_spmm_plan *p, const float *val, const DenseSrc &dense, 
         const int tr = tile_rows(p, F);
         if (tr > 0) {
             bool done = false;
-            const int rc = spmm_run_tile(p, tr, val, dense, out, F, ldo, accumulate, row_div, st, scratch == nullptr, &done);
+            int rc = SGNN_OK;
+            if (band_wanted(p, F, band_windows(p, F, true).w[0]))
+                rc = spmm_run_tile(p, tr, val, dense, out, F, ldo, accumulate, row_div, st, scratch == nullptr, &done);
+            else if (scratch == nullptr)
+                rc = spmm_run_tile_alone(p, tr, val, dense, out, F, ldo, accumulate, row_div, st, &done);
             if (rc != SGNN_OK || done) return rc;
         }
         const BandWindows bw = band_windows(p, F, ldo % 2 == 0 && aligned(out, 8));

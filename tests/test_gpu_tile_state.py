@@ -198,3 +198,68 @@ def test_a_width_that_tiles_do_not_suit_leaves_the_others_theirs():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, first)
+
+
+def test_products_of_one_matrix_on_several_streams():
+    """Without long rows a plan keeps no state between products that are in flight: operands, values and outputs of two streams
+    stay apart, with nothing that orders them, and one stream after the other gets its turn."""
+    c = _Case(*SHORT)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    sets = []
+    for i in range(2):
+        x, v = torch.randn(c.K, c.F, device=DEV), torch.rand(c.value.numel(), device=DEV)
+        sets.append((x, v, torch.empty_like(c.out)))
+    torch.cuda.synchronize()
+    for turn in range(20):
+        for st, (x, v, out) in zip(streams, sets):
+            with torch.cuda.stream(st):
+                c.product(v, x, out)
+        if turn % 5 == 4:
+            torch.cuda.synchronize()
+            for x, v, out in sets:
+                c.check(v, x, out, what=turn)
+                out.zero_()
+            streams.reverse()
+    assert c.plan.tiles(c.F)[1] == 1
+
+
+def test_threads_and_captures_beside_each_other():
+    """Another thread's products, the first of a width among them, neither disturb a capture nor wait for one; a captured
+    product that is the plan's first builds nothing."""
+    import threading
+    c = _Case(*SHORT)
+    graph = _captured(c, c.value)
+    assert c.plan.tiles(c.F)[1] == 0
+    errors, widths = [], (602, 700, 1024)
+    sets = {F: (c.operand(F), torch.empty(c.M, F, device=DEV)) for F in widths}
+    torch.cuda.synchronize()
+
+    def work(n):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(n):
+                    for x, out in sets.values():
+                        c.plan.run(c.value, x, out, accumulate=False, bind=False)
+        except Exception as e:   # noqa: BLE001 (shown below)
+            errors.append(e)
+
+    second = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(second):
+        c.plan.run(c.value, c.x, c.out, accumulate=False, bind=False)
+        t = threading.Thread(target=work, args=(2,))
+        t.start()
+        t.join()
+    assert not errors and c.plan.tiles(c.F)[1] > 0
+    threads = [threading.Thread(target=work, args=(30,)) for _ in range(3)]
+    for t in threads:
+        t.start()
+    for i in range(30):
+        c.out.fill_(7.0)
+        (graph, second)[i % 2].replay()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors
+    c.check(c.value)
+    for x, out in sets.values():
+        c.check(c.value, x, out)
