@@ -172,11 +172,11 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4))) vo
                     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
                                  "global_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024\n\t"
                                  "global_load_lds_dwordx4 %0, %1 offset:2048\n\tglobal_load_lds_dwordx4 %0, %1 offset:3072"
-                                 ::"v"(off), "s"(src + q * 1024), "s"(slot + q * 1024) : "memory");
+                                 ::"v"(off), "s"(src + q * 1024), "s"(slot + q * 1024) : "m0", "memory");
                 else
                     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
                                  "global_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024"
-                                 ::"v"(off), "s"(src + q * 1024), "s"(slot + q * 1024) : "memory");
+                                 ::"v"(off), "s"(src + q * 1024), "s"(slot + q * 1024) : "m0", "memory");
             }
             // 52 loads may be out: those of this tile and of the one before
             landed = t - 1 > landed ? t - 1 : landed;
@@ -220,8 +220,8 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4))) vo
         const int32_t *wp = a.stream + (int64_t)a.batch0[w] * (2 * kTileBatch);
 #define TL_NONE(vl, voff) ""
 #define TL_OPERANDS \
-            : "+{v[24:55]}"(r0), "+{v[56:87]}"(r1), "+{v[88:119]}"(r2), "+{v[120:127]}"(r3), "+{v0}"(lane4), "+{v2}"(post) \
-            : "{s[0:1]}"(wp), "{v1}"(0x3ff00), \
+            : "+{v[24:55]}"(r0), "+{v[56:87]}"(r1), "+{v[88:119]}"(r2), "+{v[120:127]}"(r3), "+{v0}"(lane4), "+{v2}"(post), "+{s[0:1]}"(wp) \
+            : "{v1}"(0x3ff00), \
               "{v3}"(kTileTouch + (lane4 & 4) * 16), "{v7}"(kTileFilled) \
             : "v4", "v5", "v6", "v8", "v9", "v10", "v11", "v12", "v13", "v14", "v15", "v16", "v17", "v18", "v19", "v20", "v21", "v22", \
               "v23", "s6", "s7", "s10", "s11", "s12", "s20", "s21", "s22", "s23", "s24", "s25", "s26", "s27", "s28", "s29", "s30", \
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4))) vo
               "s48", "s49", "s50", "s51", "s52", "s53", "s54", "s55", "s56", "s57", "s58", "s59", "s60", "s61", "s62", "s63", "s64", \
               "s65", "s66", "s67", "s68", "s69", "s70", "s71", "s72", "s73", "s74", "s75", "s76", "s77", "s78", "s79", "s80", "s81", \
               "s82", "s83", "s84", "s85", "s86", "s87", "s88", "s89", "s90", "s91", "s92", "s93", "s94", "s95", "s96", "s97", "s98", \
-              "s99", "scc", "memory"
+              "s99", "m0", "scc", "memory"
         if constexpr (WEIGHTED) asm volatile(TL_LOOP(TL_V0, TL_V1, TL_VL) TL_OPERANDS);
         else asm volatile(TL_LOOP(TL_ONES, TL_ONES, TL_NONE) TL_OPERANDS);
     }
