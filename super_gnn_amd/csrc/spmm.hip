@@ -28,6 +28,7 @@
 #include <list>
 #include <memory>
 #include <mutex>
+#include <new>
 #include <vector>
 
 #include "common.hpp"
@@ -2860,6 +2861,16 @@ static int spmm_run(sgnn_spmm_plan *p, const float *val, const DenseSrc &dense, 
     return SGNN_OK;
 }
 
+// A product may build a schedule on the host: running out of memory there is a status like any other, not an exception for C.
+static int spmm_entry(sgnn_spmm_plan *p, const float *val, const DenseSrc &dense, int bits, float *out, int64_t F, int64_t ldo, int accumulate,
+                      const float *row_div, hipStream_t st, float *scratch, size_t scratch_floats) {
+    try {
+        return spmm_run(p, val, dense, bits, out, F, ldo, accumulate, row_div, st, scratch, scratch_floats);
+    } catch (const std::bad_alloc &) {
+        return fail(SGNN_ERR_HIP, "out of host memory");
+    }
+}
+
 extern "C" int sgnn_spmm_plan_bind_values(sgnn_spmm_plan *p, const float *val, sgnn_stream_t stream) {
     SGNN_REQUIRE(p != nullptr, "plan is null");
     for (size_t i = 0; i < p->parts.size(); ++i) {
@@ -2916,7 +2927,7 @@ extern "C" int sgnn_spmm_csr_f32(sgnn_spmm_plan *p, const float *val, const floa
     SGNN_REQUIRE(ldx >= F, "leading dimension smaller than F (ldx=%lld F=%lld)", (long long)ldx, (long long)F);
     SGNN_REQUIRE(x != nullptr || p->nnz == 0 || p->M == 0, "x is null");
     DenseSrc d{x, ldx, nullptr, ParamBuf{nullptr, 0}, nullptr, nullptr, 0};
-    return spmm_run(p, val, d, 0, out, F, ldo, accumulate, row_div, (hipStream_t)stream);
+    return spmm_entry(p, val, d, 0, out, F, ldo, accumulate, row_div, (hipStream_t)stream, nullptr, 0);
 }
 
 extern "C" int sgnn_spmm_csr_f32_noalloc(sgnn_spmm_plan *p, const float *val, const float *x, float *out, int64_t F,
@@ -2929,7 +2940,7 @@ extern "C" int sgnn_spmm_csr_f32_noalloc(sgnn_spmm_plan *p, const float *val, co
     const int rc = scratch_for_current_device(&scratch);
     if (rc != SGNN_OK) return rc;
     DenseSrc d{x, ldx, nullptr, ParamBuf{nullptr, 0}, nullptr, nullptr, 0};
-    return spmm_run(p, val, d, 0, out, F, ldo, accumulate, row_div, (hipStream_t)stream, scratch, kScratchFloats);
+    return spmm_entry(p, val, d, 0, out, F, ldo, accumulate, row_div, (hipStream_t)stream, scratch, kScratchFloats);
 }
 
 static int spmm_dq_impl(sgnn_spmm_plan *p, const float *val, const uint8_t *q, const void *params, int params_bf16,
@@ -2960,7 +2971,7 @@ static int spmm_dq_impl(sgnn_spmm_plan *p, const float *val, const uint8_t *q, c
             d.eslot_long = p->eslot_long ? p->eslot_long : p->eslot_csr;  // unregrouped long rows index the CSR arrays
         }
     }
-    return spmm_run(p, val, d, bits, out, F, ldo, accumulate, row_div, (hipStream_t)stream);
+    return spmm_entry(p, val, d, bits, out, F, ldo, accumulate, row_div, (hipStream_t)stream, nullptr, 0);
 }
 
 extern "C" int sgnn_spmm_csr_dq_f32(sgnn_spmm_plan *p, const float *val, const uint8_t *q, const float *params,
