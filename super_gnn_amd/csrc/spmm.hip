@@ -1460,7 +1460,7 @@ struct sgnn_spmm_plan {
     std::atomic<bool> tile_too_many{false};   // more batches than the streams can number
     float *band_xs = nullptr;       // the dense operand restaged slice by slice (see band_restage_kernel), grown on demand
     size_t band_xs_floats = 0;
-    bool band_xs_captured = false, partial_captured = false;   // a captured product names the buffer
+    bool band_xs_captured = false, partial_captured = false, val_long_captured = false;   // a captured product names the buffer
     std::vector<void *> kept;       // buffers grown out of that captured products may still name
     // A matrix with 2^31 edges or more is held as consecutive row blocks, each a plan of its own with fewer
     // edges than that (the kernels' edge offsets are 32-bit); every call on the whole runs the blocks in turn.
@@ -2808,6 +2808,11 @@ static int spmm_run(sgnn_spmm_plan *p, const float *val, const DenseSrc &dense, 
         }
     }
     float *partial = p->partial;
+    bool capturing = false;
+    if (p->n_items > 0) {
+        const int rc = is_capturing(st, &capturing);
+        if (rc != SGNN_OK) return rc;
+    }
     if (scratch != nullptr) {
         const size_t need = (size_t)p->n_items * (size_t)F;
         SGNN_REQUIRE(need <= scratch_floats,
@@ -2817,11 +2822,9 @@ static int spmm_run(sgnn_spmm_plan *p, const float *val, const DenseSrc &dense, 
         partial = scratch;
     } else if (p->n_items > 0) {
         const size_t need = (size_t)p->n_items * (size_t)F;
-        bool capturing = false;
-        int rc = is_capturing(st, &capturing);
-        if (rc != SGNN_OK) return rc;
         if (need > p->partial_floats) {
-            if ((rc = give_up(p, &p->partial, &p->partial_captured)) != SGNN_OK) return rc;
+            const int rc = give_up(p, &p->partial, &p->partial_captured);
+            if (rc != SGNN_OK) return rc;
             p->partial_floats = 0;
             SGNN_HIP_CHECK(hipMalloc(&p->partial, need * sizeof(float)));
             p->partial_floats = need;
@@ -2840,6 +2843,7 @@ static int spmm_run(sgnn_spmm_plan *p, const float *val, const DenseSrc &dense, 
     if (val != nullptr && val == p->bound_val && p->val_long != nullptr) {
         s.eperm = nullptr;   // values already sit in regrouped order: contiguous reads, no indirection
         s.val = p->val_long;
+        if (capturing) p->val_long_captured = true;
     }
     FinalArgs f{p->long_rows, p->long_pbeg, partial, out, (int)p->n_long, (int)F, ldo, accumulate, row_div};
     if (bits != 0) {
@@ -2884,6 +2888,17 @@ extern "C" int sgnn_spmm_plan_bind_values(sgnn_spmm_plan *p, const float *val, s
     if (!p->partitioned || p->regrouped == 0) {  // nothing to regroup for the piece path
         p->bound_val = val;
         return SGNN_OK;
+    }
+    if (p->val_long_captured) {
+        // A captured product goes on reading the values it was captured with, so others get a copy of their own (a binding that
+        // is captured itself belongs to its graph).
+        bool capturing = false;
+        const int rc = is_capturing((hipStream_t)stream, &capturing);
+        if (rc != SGNN_OK) return rc;
+        if (!capturing) {
+            const int kept = give_up(p, &p->val_long, &p->val_long_captured);
+            if (kept != SGNN_OK) return kept;
+        }
     }
     if (p->val_long == nullptr) SGNN_HIP_CHECK(hipMalloc(&p->val_long, sizeof(float) * (size_t)p->regrouped));
     const int64_t nb = (p->regrouped + kBlock - 1) / kBlock;

@@ -110,6 +110,29 @@ def test_replays_and_eager_products_do_not_see_each_others_values(kind, bound, m
         torch.cuda.synchronize()
 
 
+def test_captured_products_keep_the_bound_values_of_long_rows():
+    """The row classes read a bound array's long rows from the plan's copy; binding another array gives that one its own."""
+    c = _Case(700, 900, 40, 130, hubs=5, hub_deg=600)
+    assert c.plan.tiles(c.F) == (0, 0) and c.plan.info()["partitioned"] == 1
+    for _ in range(3):
+        c.product(c.value)
+    first, other = c.out.clone(), c.value * 3 + 1
+    c.plan.unbind_values()
+    second = c.product(other).clone()
+    for _ in range(3):
+        c.product(c.value)
+    graph = _captured(c, c.value)
+    for i in range(3):
+        for value, want in ((other, second), (c.value, first)):
+            for j in range(3):
+                c.product(value)
+                assert torch.equal(c.out, want), (i, j)
+            c.out.fill_(7.0)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(c.out, first), i
+
+
 @pytest.mark.parametrize("kind", ["tiles", "bands", "row classes"])
 def test_captured_products_keep_their_buffers(kind, monkeypatch):
     """Wider products later on need a larger workspace, other schedules of the same matrix and larger partial sums; what a
