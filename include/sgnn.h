@@ -294,18 +294,20 @@ int sgnn_dequant_v1_f32(const uint8_t *q, float *x, const int64_t *range, const 
  * ------------------------------------------------------------------------------------------- */
 
 /* y = relu((x - mean) * rstd * weight + bias) per row of C floats (a multiple of 4 up to 1024; all pointers 16-byte
- * aligned), stats[n, 2] = (mean, rstd = 1 / sqrt(variance + eps)).  NaN stays NaN. */
-int sgnn_norm_relu_f32(const float *x, const float *weight, const float *bias, float eps, float *y, float *stats, int64_t n, int64_t C,
-                       sgnn_stream_t stream);
+ * aligned), stats[n, 2] = (mean, rstd = 1 / sqrt(variance + eps)).  NaN stays NaN.  signs (or null): [n, ceil(C / 8)] bytes, bit c % 8
+ * of byte c / 8 set where the rectifier passed column c. */
+int sgnn_norm_relu_f32(const float *x, const float *weight, const float *bias, float eps, float *y, float *stats, uint8_t *signs, int64_t n,
+                       int64_t C, sgnn_stream_t stream);
 
 /* Floats of workspace the gradient needs. */
 int64_t sgnn_norm_relu_workspace(int64_t n, int64_t C);
 
 /* Its gradient for rows that came out of a dropout: the norm's operand was mask * scale * x (mask[n, C] bytes of 0 or 1; null:
- * x itself, scale 1).  gx: gradient w.r.t. x; gw, gb: w.r.t. weight and bias, summed over the rows in a fixed order. */
+ * x itself, scale 1).  signs: the forward pass's; null: the rectifier's side is computed anew from x, which a scale that is rounded
+ * otherwise than the dropout's own moves for elements next to 0.  gx: gradient w.r.t. x; gw, gb: w.r.t. weight and bias, summed over the rows in a fixed order. */
 int sgnn_norm_relu_backward_f32(const float *g, const float *x, const uint8_t *mask, float scale, const float *stats,
-                                const float *weight, const float *bias, float *gx, float *workspace, float *gw, float *gb, int64_t n, int64_t C,
-                                sgnn_stream_t stream);
+                                const uint8_t *signs, const float *weight, const float *bias, float *gx, float *workspace, float *gw, float *gb,
+                                int64_t n, int64_t C, sgnn_stream_t stream);
 
 /* out[c] = sum over n > 0 rows of x[n, C], in a fixed order (C and alignment as above; workspace: as many floats as
  * sgnn_norm_relu_workspace(n, C)). */

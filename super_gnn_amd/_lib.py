@@ -39,9 +39,9 @@ SIGNATURES = {
     "sgnn_spmm_csr_dq_wire_f32": (_int, [_vp, _vp, _vp, _vp, _int, _vp, _int, _vp, _i64, _i64, _int, _vp, _vp]),
     "sgnn_quant_v1_f32": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _vp]),
     "sgnn_dequant_v1_f32": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _vp]),
-    "sgnn_norm_relu_f32": (_int, [_vp, _vp, _vp, ctypes.c_float, _vp, _vp, _i64, _i64, _vp]),
+    "sgnn_norm_relu_f32": (_int, [_vp, _vp, _vp, ctypes.c_float, _vp, _vp, _vp, _i64, _i64, _vp]),
     "sgnn_norm_relu_workspace": (_i64, [_i64, _i64]),
-    "sgnn_norm_relu_backward_f32": (_int, [_vp, _vp, _vp, ctypes.c_float, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _vp]),
+    "sgnn_norm_relu_backward_f32": (_int, [_vp, _vp, _vp, ctypes.c_float, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _vp]),
     "sgnn_column_sum_f32": (_int, [_vp, _vp, _vp, _i64, _i64, _vp]),
     "sgnn_rest_product_f32": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _vp]),
     "sgnn_profile_enable": (_int, [_int]),

@@ -26,7 +26,8 @@ __device__ __forceinline__ float group_sum(float v) {
 template <int G, int NV>
 __global__ __launch_bounds__(kNormBlock) void norm_relu_kernel(const float *__restrict__ x, const float *__restrict__ weight,
                                                                const float *__restrict__ bias, float eps, float *__restrict__ y,
-                                                               float2 *__restrict__ stats, int64_t n, int C) {
+                                                               float2 *__restrict__ stats, uint8_t *__restrict__ signs, int64_t n,
+                                                               int C) {
     const int lig = threadIdx.x % G;
     const int64_t row0 = ((int64_t)blockIdx.x * (kNormBlock / G) + threadIdx.x / G) * kNormRows;
     float v[kNormRows][NV][4];
@@ -64,27 +65,33 @@ __global__ __launch_bounds__(kNormBlock) void norm_relu_kernel(const float *__re
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
             const int c = 4 * (lig + G * k);
-            if (c >= C) continue;
-            float w[4], b[4], o[4];
-            vec_load<4>(w, weight + c);
-            vec_load<4>(b, bias + c);
+            uint32_t passed = 0;   // bit e: the rectifier passes element e (NaN passes)
+            if (c < C) {
+                float w[4], b[4], o[4];
+                vec_load<4>(w, weight + c);
+                vec_load<4>(b, bias + c);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float p = fmaf((v[r][k][e] - mean) * rstd, w[e], b[e]);
-                o[e] = p < 0.0f ? 0.0f : p;   // (NaN stays)
+                for (int e = 0; e < 4; ++e) {
+                    const float p = fmaf((v[r][k][e] - mean) * rstd, w[e], b[e]);
+                    o[e] = p < 0.0f ? 0.0f : p;   // (NaN stays)
+                    passed |= (p <= 0.0f ? 0u : 1u) << e;
+                }
+                vec_store<4>(y + (row0 + r) * C + c, o);
             }
-            vec_store<4>(y + (row0 + r) * C + c, o);
+            const uint32_t right = __shfl_xor(passed, 1, 64);   // two lanes share a byte
+            if (signs && c < C && (lig & 1) == 0) signs[(row0 + r) * ((C + 7) / 8) + c / 8] = (uint8_t)(passed | right << 4);
         }
     }
 }
 
 // Gradient w.r.t. the rows x before a dropout that kept the elements of `mask` times `scale` (mask null: no dropout), and each
-// workgroup's sums of the gradients w.r.t. weight and bias: partial[block][2][C].
+// workgroup's sums of the gradients w.r.t. weight and bias: partial[block][2][C].  The elements that the rectifier passed are those
+// of `signs`; null: where the norm of mask * scale * x, computed anew, is above 0.
 template <int G, int NV>
 __global__ __launch_bounds__(kNormBlock) void norm_relu_backward_kernel(
     const float *__restrict__ g, const float *__restrict__ x, const uint8_t *__restrict__ mask, float scale,
-    const float2 *__restrict__ stats, const float *__restrict__ weight, const float *__restrict__ bias, float *__restrict__ gx,
-    float *__restrict__ partial, int64_t n, int C) {
+    const float2 *__restrict__ stats, const uint8_t *__restrict__ signs, const float *__restrict__ weight, const float *__restrict__ bias,
+    float *__restrict__ gx, float *__restrict__ partial, int64_t n, int C) {
     constexpr int kGroups = kNormBlock / G;
     __shared__ float sums[kGroups][2][G * NV * 4];
     const int lig = threadIdx.x % G, group = threadIdx.x / G;
@@ -103,7 +110,7 @@ __global__ __launch_bounds__(kNormBlock) void norm_relu_backward_kernel(
     const int64_t step = (int64_t)gridDim.x * kGroups * kNormRows;
     for (int64_t row0 = ((int64_t)blockIdx.x * kGroups + group) * kNormRows; row0 < n; row0 += step) {
         float gv[kNormRows][NV][4], xv[kNormRows][NV][4];
-        uint32_t keep[kNormRows][NV];
+        uint32_t keep[kNormRows][NV], passed[kNormRows][NV];
         float2 st[kNormRows];
 #pragma unroll
         for (int r = 0; r < kNormRows; ++r) {
@@ -113,7 +120,9 @@ __global__ __launch_bounds__(kNormBlock) void norm_relu_backward_kernel(
                 const int c = 4 * (lig + G * k);
                 const int64_t i = (row0 + r) * C + c;
                 keep[r][k] = 0x01010101u;
+                passed[r][k] = 0;
                 if (row0 + r < n && c < C) {
+                    if (signs) passed[r][k] = (uint32_t)signs[(row0 + r) * ((C + 7) / 8) + c / 8] >> (c & 4);
                     vec_load_nt<4>(gv[r][k], g + i);
                     vec_load_nt<4>(xv[r][k], x + i);
                     if (mask) keep[r][k] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(mask + i));
@@ -134,8 +143,8 @@ __global__ __launch_bounds__(kNormBlock) void norm_relu_backward_kernel(
                 for (int e = 0; e < 4; ++e) {
                     const float xd = keep[r][k] >> (8 * e) & 0xffu ? xv[r][k][e] * scale : 0.0f;
                     const float h = in ? (xd - mean) * rstd : 0.0f;
-                    const float p = fmaf(h, w[k][e], b[k][e]);
-                    const float gr = p <= 0.0f ? 0.0f : gv[r][k][e];
+                    const bool pass = signs ? passed[r][k] >> e & 1u : !(fmaf(h, w[k][e], b[k][e]) <= 0.0f);
+                    const float gr = pass ? gv[r][k][e] : 0.0f;
                     gw[k][e] = fmaf(gr, h, gw[k][e]);
                     gb[k][e] += gr;
                     const float gh = gr * w[k][e];
@@ -314,15 +323,15 @@ static int check_norm(const void *a, const void *b, const void *w, const void *b
     return SGNN_OK;
 }
 
-extern "C" int sgnn_norm_relu_f32(const float *x, const float *weight, const float *bias, float eps, float *y, float *stats, int64_t n,
-                                  int64_t C, sgnn_stream_t stream) {
+extern "C" int sgnn_norm_relu_f32(const float *x, const float *weight, const float *bias, float eps, float *y, float *stats,
+                                  uint8_t *signs, int64_t n, int64_t C, sgnn_stream_t stream) {
     const int rc = check_norm(x, y, weight, bias, n, C);
     if (rc != SGNN_OK || n == 0) return rc;
     SGNN_REQUIRE(stats != nullptr && aligned(stats, 8), "stats must be non-null and 8-byte aligned");
     with_norm_shape(C, [&](auto g, auto nv) {
         const int64_t per = (kNormBlock / g) * kNormRows;
         hipLaunchKernelGGL((norm_relu_kernel<g, nv>), dim3((uint32_t)((n + per - 1) / per)), dim3(kNormBlock), 0, (hipStream_t)stream, x, weight,
-                           bias, eps, y, reinterpret_cast<float2 *>(stats), n, (int)C);
+                           bias, eps, y, reinterpret_cast<float2 *>(stats), signs, n, (int)C);
     });
     SGNN_HIP_CHECK(hipGetLastError());
     return SGNN_OK;
@@ -331,15 +340,15 @@ extern "C" int sgnn_norm_relu_f32(const float *x, const float *weight, const flo
 extern "C" int64_t sgnn_norm_relu_workspace(int64_t n, int64_t C) { return n <= 0 || C <= 0 ? 0 : (int64_t)norm_blocks(n, C) * 2 * C; }
 
 extern "C" int sgnn_norm_relu_backward_f32(const float *g, const float *x, const uint8_t *mask, float scale, const float *stats,
-                                           const float *weight, const float *bias, float *gx, float *workspace, float *gw, float *gb, int64_t n,
-                                           int64_t C, sgnn_stream_t stream) {
+                                           const uint8_t *signs, const float *weight, const float *bias, float *gx, float *workspace, float *gw,
+                                           float *gb, int64_t n, int64_t C, sgnn_stream_t stream) {
     int rc = check_norm(g, x, weight, bias, n, C);
     if (rc != SGNN_OK || n == 0) return rc;
     SGNN_REQUIRE(gx && workspace && gw && gb && stats && aligned(gx, 16) && aligned(stats, 8) && aligned(mask, 4), "null or misaligned argument");
     const int blocks = norm_blocks(n, C);
     with_norm_shape(C, [&](auto gl, auto nv) {
         hipLaunchKernelGGL((norm_relu_backward_kernel<gl, nv>), dim3((uint32_t)blocks), dim3(kNormBlock), 0, (hipStream_t)stream, g, x, mask, scale,
-                           reinterpret_cast<const float2 *>(stats), weight, bias, gx, workspace, n, (int)C);
+                           reinterpret_cast<const float2 *>(stats), signs, weight, bias, gx, workspace, n, (int)C);
     });
     hipLaunchKernelGGL(partial_sum_kernel, dim3((uint32_t)((2 * C + 15) / 16)), dim3(256), 0, (hipStream_t)stream, workspace, gw, gb, blocks,
                        (int)C, (int)(2 * C));

@@ -98,14 +98,15 @@ class _DropoutNormRelu(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias, eps, p):
         dropped, mask = torch.native_dropout(x, p, True) if p > 0 else (x, None)
-        y, stats = norm_relu(dropped, weight, bias, eps)
-        ctx.save_for_backward(x, mask, stats, weight, bias)
+        signs = torch.empty((x.shape[0], (x.shape[1] + 7) // 8), dtype=torch.uint8, device=x.device)
+        y, stats = norm_relu(dropped, weight, bias, eps, signs)
+        ctx.save_for_backward(x, mask, stats, signs, weight, bias)
         ctx.eps, ctx.scale = eps, 1.0 / (1.0 - p)
         return y
 
     @staticmethod
     def backward(ctx, g):
-        x, mask, stats, weight, bias = ctx.saved_tensors
+        x, mask, stats, signs, weight, bias = ctx.saved_tensors
         if torch.is_grad_enabled():   # a gradient that is differentiated itself
             with torch.enable_grad():
                 dropped = x if mask is None else x * mask * ctx.scale
@@ -113,7 +114,7 @@ class _DropoutNormRelu(torch.autograd.Function):
                 wanted = [t for t, need in zip((x, weight, bias), ctx.needs_input_grad) if need]
                 found = iter(torch.autograd.grad(y, wanted, g, create_graph=True))
             return tuple(next(found) if need else None for need in ctx.needs_input_grad[:3]) + (None, None)
-        return norm_relu_backward(g.contiguous(), x, mask, ctx.scale, stats, weight, bias) + (None, None)
+        return norm_relu_backward(g.contiguous(), x, mask, ctx.scale, stats, weight, bias, signs) + (None, None)
 
 
 _global_hooks = getattr(torch.nn.modules.module, "_has_any_global_hook", lambda: False)

@@ -671,21 +671,24 @@ def dequantize_tensor_v1(input, output, quantized_nodes_feat_range, quantized_pa
 # -------------------------------------------------------------------------------------------------
 # Layer passes
 # -------------------------------------------------------------------------------------------------
-def norm_relu(x, weight, bias, eps):
-    """relu(layer_norm(x)) of contiguous fp32 rows on the GPU, and each row's (mean, 1 / standard deviation)."""
+def norm_relu(x, weight, bias, eps, signs=None):
+    """relu(layer_norm(x)) of contiguous fp32 rows on the GPU, and each row's (mean, 1 / standard deviation).  ``signs`` (uint8
+    [rows, ceil(columns / 8)], optional) receives a bit for every element that the rectifier passed."""
     n, C = x.shape
     y, stats = torch.empty_like(x), torch.empty((n, 2), dtype=torch.float32, device=x.device)
-    check(lib.sgnn_norm_relu_f32(x.data_ptr(), weight.data_ptr(), bias.data_ptr(), eps, y.data_ptr(), stats.data_ptr(), n, C, _stream()))
+    check(lib.sgnn_norm_relu_f32(x.data_ptr(), weight.data_ptr(), bias.data_ptr(), eps, y.data_ptr(), stats.data_ptr(), _ptr(signs), n, C,
+                                 _stream()))
     return y, stats
 
 
-def norm_relu_backward(g, x, mask, scale, stats, weight, bias):
-    """Gradients of relu(layer_norm(mask * scale * x)) w.r.t. x, weight and bias; mask None: no dropout."""
+def norm_relu_backward(g, x, mask, scale, stats, weight, bias, signs=None):
+    """Gradients of relu(layer_norm(mask * scale * x)) w.r.t. x, weight and bias; mask None: no dropout.  ``signs``: those of norm_relu;
+    None: the rectifier's side is computed anew."""
     n, C = x.shape
     gx, gw, gb = torch.empty_like(x), torch.empty_like(weight), torch.empty_like(bias)
     work = torch.empty(lib.sgnn_norm_relu_workspace(n, C), dtype=torch.float32, device=x.device)
-    check(lib.sgnn_norm_relu_backward_f32(g.data_ptr(), x.data_ptr(), _ptr(mask), scale, stats.data_ptr(), weight.data_ptr(), bias.data_ptr(),
-                                          gx.data_ptr(), work.data_ptr(), gw.data_ptr(), gb.data_ptr(), n, C, _stream()))
+    check(lib.sgnn_norm_relu_backward_f32(g.data_ptr(), x.data_ptr(), _ptr(mask), scale, stats.data_ptr(), _ptr(signs), weight.data_ptr(),
+                                          bias.data_ptr(), gx.data_ptr(), work.data_ptr(), gw.data_ptr(), gb.data_ptr(), n, C, _stream()))
     return gx, gw, gb
 
 

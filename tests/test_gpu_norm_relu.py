@@ -109,3 +109,26 @@ def test_weight_gradient_of_rows_that_slabs_leave_over():
         with torch.no_grad():
             assert bool(((_weight_grad(g, a).double() - want).abs() <= bound).all())
         assert bool(((_weight_grad(g, a).double() - want).abs() <= bound).all())   # as in a gradient that is differentiated
+
+
+@pytest.mark.parametrize("C", [4, 12, 64, 100, 256, 260, 516, 1024])
+def test_rectifier_side_is_the_forward_passs(C):
+    """Gradients pass where the output is above 0 and nowhere else, also for elements a rounding away from 0 behind a dropout whose
+    factor 1 / (1 - p) may be rounded in more ways than one."""
+    from super_gnn_amd import layers
+    from super_gnn_amd.supergnn_ops import norm_relu
+    norm = torch.nn.LayerNorm(C).cuda()
+    g = torch.Generator().manual_seed(C)
+    for p in (0.04, 0.09, 0.128, 0.5):
+        for seed in range(20):
+            x = (torch.randn(1, C, generator=g) * 3 + 1).cuda().requires_grad_()
+            torch.manual_seed(seed)
+            dropped = F.dropout(x.detach(), p)
+            stats = norm_relu(dropped, torch.ones_like(norm.weight), torch.zeros_like(norm.bias), norm.eps)[1]
+            with torch.no_grad():   # the norm's output is 0 or one rounding of it
+                norm.bias.copy_(torch.nextafter(-(dropped[0] - stats[0, 0]) * stats[0, 1], torch.randn(C, generator=g).sign().cuda() * 1e3))
+            norm.zero_grad()
+            torch.manual_seed(seed)
+            y = layers._dropout_norm_relu(x, norm, p, True)
+            y.backward(torch.ones_like(y))
+            assert torch.equal(norm.bias.grad != 0, y[0] > 0), (p, seed)
