@@ -165,7 +165,7 @@ __global__ __launch_bounds__(kNormBlock) void norm_relu_backward_kernel(
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const float v = (gv[r][k][e] - s1 - xv[r][k][e] * s2) * rstd;
-                        o[e] = keep[r][k] >> (8 * e) & 0xffu ? v * scale : 0.0f;
+                        o[e] = v * (keep[r][k] >> (8 * e) & 0xffu ? scale : 0.0f);   // (NaN and infinities times 0, as the mask's product)
                     }
                     vec_store<4>(gx + (row0 + r) * C + c, o);
                 }

@@ -132,3 +132,25 @@ def test_rectifier_side_is_the_forward_passs(C):
             y = layers._dropout_norm_relu(x, norm, p, True)
             y.backward(torch.ones_like(y))
             assert torch.equal(norm.bias.grad != 0, y[0] > 0), (p, seed)
+
+
+def test_dropped_elements_of_rows_that_are_not_finite():
+    """A NaN row and an infinite row behind a dropout: every gradient NaN where the separate modules' is, dropped elements included."""
+    from super_gnn_amd import layers
+    x = torch.randn(6, 64, generator=torch.Generator().manual_seed(1)).cuda()
+    x[0, 3], x[1, 5] = float("nan"), float("inf")
+    go = torch.randn(6, 64, generator=torch.Generator().manual_seed(2)).cuda()
+    go[4, 7], go[5, 9] = float("inf"), float("nan")
+    found = []
+    for fused in (True, False):
+        norm = torch.nn.LayerNorm(64).cuda()
+        if not fused:
+            norm.register_forward_hook(lambda *a: None)
+        xs = x.clone().requires_grad_()
+        torch.manual_seed(4)
+        assert layers._fusable(norm, xs) == fused
+        y = layers._dropout_norm_relu(xs, norm, 0.5, True)
+        y.backward(go)
+        found.append((y.detach(), xs.grad, norm.weight.grad, norm.bias.grad))
+    for a, b in zip(*found):
+        assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.isinf(a), torch.isinf(b))
