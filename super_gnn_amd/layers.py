@@ -114,7 +114,10 @@ class _DropoutNormRelu(torch.autograd.Function):
                 wanted = [t for t, need in zip((x, weight, bias), ctx.needs_input_grad) if need]
                 found = iter(torch.autograd.grad(y, wanted, g, create_graph=True))
             return tuple(next(found) if need else None for need in ctx.needs_input_grad[:3]) + (None, None)
-        return norm_relu_backward(g.contiguous(), x, mask, ctx.scale, stats, weight, bias, signs) + (None, None)
+        g = g.contiguous()
+        if g.data_ptr() % 16:   # contiguous, yet somewhere inside another tensor, as torch.cat hands gradients back
+            g = g.clone()
+        return norm_relu_backward(g, x, mask, ctx.scale, stats, weight, bias, signs) + (None, None)
 
 
 _global_hooks = getattr(torch.nn.modules.module, "_has_any_global_hook", lambda: False)

@@ -154,3 +154,18 @@ def test_dropped_elements_of_rows_that_are_not_finite():
         found.append((y.detach(), xs.grad, norm.weight.grad, norm.bias.grad))
     for a, b in zip(*found):
         assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.isinf(a), torch.isinf(b))
+
+
+def test_gradients_that_begin_inside_another_tensor():
+    from super_gnn_amd import layers
+    norm = torch.nn.LayerNorm(64).cuda()
+    x = torch.randn(30, 64, generator=torch.Generator().manual_seed(1)).cuda().requires_grad_()
+    go = torch.randn(30 * 64 + 1, generator=torch.Generator().manual_seed(2)).cuda()
+    y = layers._dropout_norm_relu(x, norm, 0.0, True)
+    torch.cat([x.new_zeros(1), y.reshape(-1)]).backward(go)      # y's part starts at element 1
+    got = x.grad.clone(), norm.weight.grad.clone(), norm.bias.grad.clone()
+    x.grad = None
+    norm.zero_grad()
+    y = layers._dropout_norm_relu(x, norm, 0.0, True)
+    y.backward(go[1:].clone().view(30, 64))
+    assert all(torch.equal(a, b) for a, b in zip(got, (x.grad, norm.weight.grad, norm.bias.grad)))
