@@ -107,17 +107,32 @@ class _DropoutNormRelu(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         x, mask, stats, signs, weight, bias = ctx.saved_tensors
-        if torch.is_grad_enabled():   # a gradient that is differentiated itself
-            with torch.enable_grad():
-                dropped = x if mask is None else x * mask * ctx.scale
-                y = F.relu(F.layer_norm(dropped, weight.shape, weight, bias, ctx.eps))
-                wanted = [t for t, need in zip((x, weight, bias), ctx.needs_input_grad) if need]
-                found = iter(torch.autograd.grad(y, wanted, g, create_graph=True))
-            return tuple(next(found) if need else None for need in ctx.needs_input_grad[:3]) + (None, None)
+        if torch.is_grad_enabled():
+            return _norm_relu_gradients(g, x, mask, ctx.scale, ctx.eps, stats, signs, weight) + (None, None)
         g = g.contiguous()
         if g.data_ptr() % 16:   # contiguous, yet somewhere inside another tensor, as torch.cat hands gradients back
             g = g.clone()
         return norm_relu_backward(g, x, mask, ctx.scale, stats, weight, bias, signs) + (None, None)
+
+
+def _norm_relu_gradients(g, x, mask, scale, eps, stats, signs, weight):
+    """norm_relu_backward in torch's operations: for gradients that are differentiated themselves, which go through the rows' mean
+    and deviation too, for batches of gradients, and for tensors that hooks on saved tensors hand back as something else."""
+    C = weight.numel()
+    passed = (signs.unsqueeze(-1) >> torch.arange(8, dtype=torch.uint8, device=signs.device) & 1).flatten(1)[:, :C].bool()
+    if mask is not None:
+        x = x * mask * scale
+    if torch.is_grad_enabled():
+        mean, rstd = x.mean(1, keepdim=True), (x.var(1, unbiased=False, keepdim=True) + eps).rsqrt()
+    else:
+        mean, rstd = stats[:, :1], stats[:, 1:]
+    hat = (x - mean) * rstd
+    g = torch.where(passed, g, 0.0)
+    gh = g * weight
+    gx = (gh - gh.mean(1, keepdim=True) - hat * (gh * hat).mean(1, keepdim=True)) * rstd
+    if mask is not None:
+        gx = gx * mask * scale
+    return gx, (g * hat).sum(0), g.sum(0)
 
 
 _global_hooks = getattr(torch.nn.modules.module, "_has_any_global_hook", lambda: False)

@@ -169,3 +169,32 @@ def test_gradients_that_begin_inside_another_tensor():
     y = layers._dropout_norm_relu(x, norm, 0.0, True)
     y.backward(go[1:].clone().view(30, 64))
     assert all(torch.equal(a, b) for a, b in zip(got, (x.grad, norm.weight.grad, norm.bias.grad)))
+
+
+def _stretch(x, norm, p, fused):
+    """The stretch through the one-pass kernels, or as the separate modules with the same masks."""
+    from super_gnn_amd import layers
+    torch.manual_seed(4)
+    if fused:
+        assert layers._fusable(norm, x)
+        return layers._dropout_norm_relu(x, norm, p, True)
+    return F.relu(norm(F.dropout(x, p)))
+
+
+def _close(a, b):
+    return torch.allclose(a, b, rtol=1e-4, atol=1e-5 * float(b.abs().max()))   # a few roundings, and sums over 30 rows
+
+
+@pytest.mark.parametrize("p", [0.0, 0.5])
+def test_rows_that_come_from_the_norms_own_weight(p):
+    """A gradient that is differentiated itself, of rows that depend on the weight by another way as well: each way counts once."""
+    norm = torch.nn.LayerNorm(64).cuda()
+    base, w = torch.randn(30, 64, generator=torch.Generator().manual_seed(1)).cuda(), norm.weight
+    with torch.no_grad():
+        norm.bias.normal_(generator=torch.Generator("cuda").manual_seed(1))
+    found = []
+    for fused in (True, False):
+        first, = torch.autograd.grad((_stretch(base * w, norm, p, fused) ** 2).sum(), w, create_graph=True)
+        second, = torch.autograd.grad((first ** 2).sum(), w)
+        found.append((first.detach(), second))
+    assert _close(found[0][0], found[1][0]) and torch.allclose(found[0][1], found[1][1], rtol=1e-3, atol=1e-4 * float(found[1][1].abs().max()))
