@@ -31,9 +31,15 @@ def _column_sum(g: Tensor) -> Tensor:
 _SPLIT_K = 64
 
 
+def _addressable(t):
+    """Whether a kernel may read the tensor by address: a plain one on the current device with memory of its own, which the
+    members of a batch of gradients do not have."""
+    return type(t) in (Tensor, Parameter) and t.is_cuda and torch._C._has_storage(t) and t.get_device() == torch.cuda.current_device()
+
+
 def _plain(*tensors):
     """Tensors a kernel may read by address, in a gradient that is not differentiated itself."""
-    return not torch.is_grad_enabled() and all(type(t) is Tensor and t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() for t in tensors)
+    return not torch.is_grad_enabled() and all(_addressable(t) and t.dtype == torch.float32 and t.is_contiguous() for t in tensors)
 
 
 def _weight_grad(g: Tensor, a: Tensor) -> Tensor:
@@ -107,11 +113,14 @@ class _DropoutNormRelu(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         x, mask, stats, signs, weight, bias = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        (n, C), real = g.shape, torch.float32
+        expected = ((g, real, (n, C)), (x, real, (n, C)), (mask, torch.bool, (n, C)), (stats, real, (n, 2)),
+                    (signs, torch.uint8, (n, (C + 7) // 8)), (weight, real, (C,)), (bias, real, (C,)))
+        if torch.is_grad_enabled() or not all(t is None or _addressable(t) and t.dtype == kind and t.shape == shape for t, kind, shape in expected):
             return _norm_relu_gradients(g, x, mask, ctx.scale, ctx.eps, stats, signs, weight) + (None, None)
-        g = g.contiguous()
-        if g.data_ptr() % 16:   # contiguous, yet somewhere inside another tensor, as torch.cat hands gradients back
-            g = g.clone()
+        # contiguous, yet somewhere inside another tensor, as torch.cat hands gradients back, will not do either
+        g, x, mask, stats, signs, weight, bias = (t if t is None or t.is_contiguous() and t.data_ptr() % 16 == 0
+                                                  else t.clone(memory_format=torch.contiguous_format) for t, _, _ in expected)
         return norm_relu_backward(g, x, mask, ctx.scale, stats, weight, bias, signs) + (None, None)
 
 

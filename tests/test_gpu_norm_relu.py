@@ -198,3 +198,37 @@ def test_rows_that_come_from_the_norms_own_weight(p):
         second, = torch.autograd.grad((first ** 2).sum(), w)
         found.append((first.detach(), second))
     assert _close(found[0][0], found[1][0]) and torch.allclose(found[0][1], found[1][1], rtol=1e-3, atol=1e-4 * float(found[1][1].abs().max()))
+
+
+@pytest.mark.parametrize("p", [0.0, 0.5])
+def test_hooks_on_saved_tensors_and_batches_of_gradients(p):
+    """Hooks may hand saved tensors back in another memory order, on other storage or as another type; a batch of gradients has no
+    memory that a kernel could read."""
+    norm = torch.nn.LayerNorm(64).cuda()
+    x = torch.randn(30, 64, generator=torch.Generator().manual_seed(1)).cuda().requires_grad_()
+    go = torch.randn(3, 30, 64, generator=torch.Generator().manual_seed(2)).cuda()
+    inputs = (x, norm.weight, norm.bias)
+    want = [torch.autograd.grad(_stretch(x, norm, p, False), inputs, g) for g in go]
+
+    def turned(t):
+        return t.t().contiguous().t() if t.dim() == 2 else t.clone()
+
+    for pack, unpack in ((lambda t: t, turned), (lambda t: t.cpu(), lambda t: t.cuda()),
+                         (lambda t: t.double() if t.is_floating_point() else t, lambda t: t)):
+        with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+            y = _stretch(x, norm, p, True)
+        got = torch.autograd.grad(y, inputs, go[0])
+        assert all(_close(a.to(b.dtype), b) for a, b in zip(got, want[0]))
+    got = torch.autograd.grad(_stretch(x, norm, p, True), inputs, go, is_grads_batched=True)
+    for i in range(3):
+        assert all(_close(a[i], b) for a, b in zip(got, want[i]))
+
+
+def test_bias_gradients_of_a_batch():
+    from super_gnn_amd.layers import _SageCombine
+    gen = torch.Generator().manual_seed(1)
+    agg, x, wn, ws, b = (torch.randn(*s, generator=gen).cuda() for s in ((50, 12), (50, 12), (8, 12), (8, 12), (8,)))
+    b.requires_grad_()
+    go = torch.randn(3, 50, 8, generator=gen).cuda()
+    got, = torch.autograd.grad(_SageCombine.apply(agg, x, None, wn, ws, b), b, go, is_grads_batched=True)
+    assert _close(got, go.sum(1))
