@@ -145,12 +145,21 @@ def _norm_relu_gradients(g, x, mask, scale, eps, stats, signs, weight):
 
 
 _global_hooks = getattr(torch.nn.modules.module, "_has_any_global_hook", lambda: False)
+_layer_norm_forward = LayerNorm.forward
+
+
+def _watched():
+    """Whether something sees or transforms the operations that run: autocast, tracing, function and dispatch modes, torch.func,
+    forward-mode differentiation."""
+    return (torch.is_autocast_enabled() or torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_function_stack() > 0
+            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._are_functorch_transforms_active()
+            or torch.autograd.forward_ad._current_level >= 0)
 
 
 def _fusable(norm, x):
     """Whether the one-pass kernels stand for dropout, ``norm`` and the rectifier: a plain LayerNorm over fp32 rows on the GPU,
     with nothing attached that would see the modules' own calls."""
-    if type(norm) is not LayerNorm or type(x) is not torch.Tensor or not x.is_cuda or x.dtype != torch.float32 or x.dim() != 2:
+    if type(norm) is not LayerNorm or type(x) is not Tensor or not _addressable(x) or x.dtype != torch.float32 or x.dim() != 2:
         return False
     n, C = x.shape
     if n == 0 or n >= 1 << 31 or C % 4 or C > 1024 or tuple(norm.normalized_shape) != (C,) or not x.is_contiguous() or x.data_ptr() % 16:
@@ -160,7 +169,9 @@ def _fusable(norm, x):
             return False
     if norm._forward_hooks or norm._forward_pre_hooks or norm._backward_hooks or norm._backward_pre_hooks or _global_hooks():
         return False
-    return not (torch.is_autocast_enabled() or torch.jit.is_tracing() or torch.compiler.is_compiling())
+    if "forward" in norm.__dict__ or LayerNorm.forward is not _layer_norm_forward:   # another forward put in its place
+        return False
+    return not _watched()
 
 
 def _dropout_norm_relu(x, norm, p, training):

@@ -182,7 +182,7 @@ def _stretch(x, norm, p, fused):
 
 
 def _close(a, b):
-    return torch.allclose(a, b, rtol=1e-4, atol=1e-5 * float(b.abs().max()))   # a few roundings, and sums over 30 rows
+    return torch.allclose(a, b, rtol=1e-4, atol=1e-5 * float(b.detach().abs().max()))   # a few roundings, and sums over 30 rows
 
 
 @pytest.mark.parametrize("p", [0.0, 0.5])
@@ -232,3 +232,57 @@ def test_bias_gradients_of_a_batch():
     go = torch.randn(3, 50, 8, generator=gen).cuda()
     got, = torch.autograd.grad(_SageCombine.apply(agg, x, None, wn, ws, b), b, go, is_grads_batched=True)
     assert _close(got, go.sum(1))
+
+
+def test_another_forward_is_called(monkeypatch):
+    from super_gnn_amd import layers
+    norm = torch.nn.LayerNorm(64).cuda()
+    x = torch.randn(8, 64, generator=torch.Generator().manual_seed(1)).cuda()
+    norm.forward = lambda t: t + 1
+    assert torch.equal(layers._dropout_norm_relu(x, norm, 0.5, False), F.relu(x + 1))
+    del norm.forward
+    monkeypatch.setattr(torch.nn.LayerNorm, "forward", lambda self, t: t + 2)
+    assert torch.equal(layers._dropout_norm_relu(x, norm, 0.5, False), F.relu(x + 2))
+
+
+def test_modes_and_transforms_see_the_operations(monkeypatch):
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from super_gnn_amd import layers
+    norm = torch.nn.LayerNorm(64).cuda()
+    x = torch.randn(3, 8, 64, generator=torch.Generator().manual_seed(1)).cuda()
+    plain = [F.relu(norm(t)) for t in x]
+    seen = []
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func.__name__)
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func.__name__)
+            return func(*args, **(kwargs or {}))
+
+    for mode in (Functions, Dispatch):
+        seen.clear()
+        with mode():
+            y = layers._dropout_norm_relu(x[0], norm, 0.5, False)
+        assert any("layer_norm" in name for name in seen) and torch.equal(y, plain[0])
+
+    def f(t):
+        return layers._dropout_norm_relu(t, norm, 0.5, False)
+
+    def ref(t):
+        return F.relu(norm(t))
+
+    assert _close(torch.func.vmap(f)(x), torch.stack(plain))
+    assert _close(torch.func.grad(lambda t: f(t).sum())(x[0]), torch.func.grad(lambda t: ref(t).sum())(x[0]))
+    for a, b in zip(torch.func.jvp(f, (x[0],), (x[1],)), torch.func.jvp(ref, (x[0],), (x[1],))):
+        assert _close(a, b)
+    with torch.autograd.forward_ad.dual_level():
+        tangents = [torch.autograd.forward_ad.unpack_dual(h(torch.autograd.forward_ad.make_dual(x[0], x[1]))).tangent for h in (f, ref)]
+    assert _close(*tangents)
+    assert layers._fusable(norm, x[0])
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)      # the kernels go to the current device's stream
+    assert not layers._fusable(norm, x[0])
