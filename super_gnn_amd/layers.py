@@ -18,7 +18,7 @@ from .supergnn_ops import add_rest_product, column_sum, norm_relu, norm_relu_bac
 
 def _column_sum(g: Tensor) -> Tensor:
     n, c = g.shape
-    if n and c % 4 == 0 and c <= 1024 and _plain(g) and g.data_ptr() % 16 == 0:
+    if 0 < n < 1 << 31 and c % 4 == 0 and c <= 1024 and _plain(g) and g.data_ptr() % 16 == 0:
         return column_sum(g)
     k = 4 // math.gcd(c, 4)
     if k == 1 or n < k or not g.is_contiguous():

@@ -286,3 +286,12 @@ def test_modes_and_transforms_see_the_operations(monkeypatch):
     assert layers._fusable(norm, x[0])
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)      # the kernels go to the current device's stream
     assert not layers._fusable(norm, x[0])
+
+
+def test_column_sums_of_more_rows_than_the_kernel_counts():
+    from super_gnn_amd.layers import _column_sum
+    n = (1 << 31) + 5
+    g = torch.ones(n, 4, device="cuda")
+    with torch.no_grad():
+        got = _column_sum(g)
+    assert bool(((got.double() - n).abs() <= 1e-4 * n).all())
