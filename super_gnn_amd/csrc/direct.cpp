@@ -18,6 +18,13 @@ decltype(&sgnn_quant_pack_rows_wire_f32) quant_wire;
 decltype(&sgnn_unpack_dequant_rows_f32) dequant_f32;
 decltype(&sgnn_unpack_dequant_rows_wire_f32) dequant_wire;
 
+// Other Python threads run while this lives.  (Taken back on every way out: the library reports errors through strings, which
+// may throw.)
+struct WithoutGil {
+    PyThreadState *state = PyEval_SaveThread();
+    ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+
 const at::Tensor *plain(PyObject *o, int device) {
     if (!THPVariable_CheckExact(o)) return nullptr;
     const at::Tensor &t = THPVariable_Unpack(o);
@@ -51,18 +58,16 @@ PyObject *rows(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
             const float *xp = x->const_data_ptr<float>();
             uint8_t *qp = q->mutable_data_ptr<uint8_t>();
             void *pp = p->mutable_data_ptr();
-            Py_BEGIN_ALLOW_THREADS
+            const WithoutGil unlocked;
             rc = bf16 ? quant_wire(xp, F, nullptr, n_rows, qp, pp, 1, sp, psp, P, n_rows, n_packed, F, (int)bits, st)
                       : quant_f32(xp, qp, static_cast<float *>(pp), sp, psp, P, n_rows, n_packed, F, (int)bits, st);
-            Py_END_ALLOW_THREADS
         } else {
             const uint8_t *qp = q->const_data_ptr<uint8_t>();
             float *xp = x->mutable_data_ptr<float>();
             const void *pp = p->const_data_ptr();
-            Py_BEGIN_ALLOW_THREADS
+            const WithoutGil unlocked;
             rc = bf16 ? dequant_wire(qp, xp, pp, 1, sp, psp, P, n_rows, n_packed, F, (int)bits, st)
                       : dequant_f32(qp, xp, static_cast<const float *>(pp), sp, psp, P, n_rows, n_packed, F, (int)bits, st);
-            Py_END_ALLOW_THREADS
         }
         return PyLong_FromLong(rc < 0 ? rc : 1);
     } catch (...) {
