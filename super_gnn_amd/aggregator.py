@@ -296,7 +296,7 @@ class _Product(object):
         self.value = None       # the edge values: this product's piece of the direction's space (_Stacked.ready)
         self._refused = False
         self._bound = self._seen = None   # [(values, version, hand binds of the part's plan)] as in SpmmPlan._maybe_bind
-        self._bands = {}
+        self._no_bands = set()
 
     def stack(self):
         """Makes the stacked plan on the first call.  False where there is none: stacking may be refused (long-row thresholds
@@ -314,13 +314,17 @@ class _Product(object):
         return self.plan is not None
 
     def takes_bands(self, F):
-        """Whether one of the partitions' own fp32 products would take the band schedule."""
+        """Whether one of the partitions' own fp32 products would take the band schedule (or tiles).  Only a no is kept: a yes ends
+        when a first product finds the columns out of order."""
         key = (F,) + tuple(os.environ.get(k) for k in _BAND_SWITCHES)
-        if key not in self._bands:
-            if len(self._bands) > 16:
-                self._bands.clear()
-            self._bands[key] = any(p.schedule(F)["band"] for p in self.plans)
-        return self._bands[key]
+        if key in self._no_bands:
+            return False
+        if any(p.schedule(F)["band"] for p in self.plans):
+            return True
+        if len(self._no_bands) > 16:
+            self._no_bands.clear()
+        self._no_bands.add(key)
+        return False
 
     def move(self, value):
         """Another place for the edge values."""
