@@ -111,8 +111,8 @@ def test_unsorted_rows_keep_the_other_schedules(monkeypatch):
 
 
 def test_strided_rows_replay_and_calls_that_may_not_allocate(monkeypatch):
-    """A captured product replays with the program's own work between; rows may lie at a pitch; a width that needs other
-    streams falls back to the ones there are when nothing may be built."""
+    """A captured product replays with the program's own work between; rows may lie at a pitch; a call that may not allocate takes
+    the streams once they are there."""
     from super_gnn_amd._lib import check, lib
     monkeypatch.setenv("SGNN_SPMM_BAND", "2")
     M, K, F = 900, 1300, 130

@@ -286,3 +286,112 @@ def test_threads_and_captures_beside_each_other():
     c.check(c.value)
     for x, out in sets.values():
         c.check(c.value, x, out)
+
+
+@pytest.mark.parametrize("weighted", [True, False])
+def test_other_widths_take_the_streams_there_are_where_nothing_may_be_built(weighted, monkeypatch):
+    """Widths that want other numbers of rows, through the non-allocating entry point and captured.  Long rows tell the tile schedule
+    from the row classes, which add them up in parts."""
+    from super_gnn_amd._lib import check, lib
+    monkeypatch.setenv("SGNN_SPMM_BAND", "2")
+    c = _Case(20000, 2500, 30, 1024, hubs=400, hub_deg=1500)
+    value = c.value if weighted else None
+    hub = int(np.argmax(np.diff(c.rowptr) > 1000))
+    c.product(value)
+    c.check(value)
+    assert c.plan.tiles(c.F)[1] == 1
+
+    def hubs_in_one_chain(x, out):
+        lo, hi = c.rowptr[hub], c.rowptr[hub + 1]
+        want = np.zeros((1, x.shape[1]), np.float32)
+        orc.spmm_accumulate(np.array([0, hi - lo]), c.col[lo:hi], np.ones(hi - lo, np.float32) if value is None else value[lo:hi].cpu().numpy(),
+                            x.cpu().numpy(), want)
+        return np.array_equal(out[hub].cpu().numpy(), want[0])
+
+    for F in (64, 256, 602):
+        x, out = c.operand(F), torch.full((c.M, F), 7.0, device=DEV)
+        assert c.plan.tiles(F)[0] != c.plan.tiles(c.F)[0]
+        args = (c.plan._h, None if value is None else value.data_ptr(), x.data_ptr(), out.data_ptr(), F, F, F, 0, None)
+        check(lib.sgnn_spmm_csr_f32_noalloc(*args, torch.cuda.current_stream().cuda_stream))
+        c.check(value, x, out, what=F)
+        assert hubs_in_one_chain(x, out), F
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            check(lib.sgnn_spmm_csr_f32(*args, torch.cuda.current_stream().cuda_stream))
+        for _ in range(3):
+            x.mul_(1.5)
+            out.fill_(7.0)
+            graph.replay()
+            torch.cuda.synchronize()
+            c.check(value, x, out, what=F)
+            assert hubs_in_one_chain(x, out), F
+    assert c.plan.tiles(c.F)[1] == 1
+
+
+@pytest.mark.parametrize("kind", ["short", "long"])
+def test_a_product_captured_behind_a_rebinding(kind, monkeypatch):
+    """An edit that the version counter sees, between the products that bound the values and the captured one."""
+    monkeypatch.setenv("SGNN_SPMM_BAND", "2")
+    c = _Case(700, 900, 40, 130, **({"hubs": 5, "hub_deg": 600} if kind == "long" else {}))
+    for _ in range(3):
+        c.product(c.value)
+    c.value.add_(1)
+    graph = _captured(c, c.value)
+    for i in range(3):
+        c.out.fill_(7.0)
+        graph.replay()
+        c.check(c.value, what=("replay", i))
+        c.product(c.value)
+        c.check(c.value, what=("eager", i))
+        torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("weighted", [True, False])
+def test_row_blocks_under_the_tile_schedule(weighted, monkeypatch):
+    """Blocks share one restaged operand, and each has its own streams and its own part of the values."""
+    monkeypatch.setenv("SGNN_SPMM_BAND", "2")
+    whole = _Case(3000, 2600, 35, 130, hubs=3, hub_deg=800)
+    monkeypatch.setenv("SGNN_SPMM_PART_EDGES", str(int(whole.rowptr[-1]) // 5))
+    blocks = _Case(3000, 2600, 35, 130, hubs=3, hub_deg=800)
+    monkeypatch.delenv("SGNN_SPMM_PART_EDGES")
+    value = whole.value if weighted else None
+    for F in (130, 64, 200, 130):
+        x, a, b = whole.operand(F), torch.empty(3000, F, device=DEV), torch.empty(3000, F, device=DEV)
+        for _ in range(3):
+            whole.product(value, x, a)
+            blocks.product(value, x, b)
+            whole.check(value, x, a, what=F)
+            assert torch.equal(a, b), F
+    assert blocks.plan.tiles(130)[1] > 0
+
+
+def test_row_blocks_of_which_one_takes_tiles_and_one_bands():
+    """By the default rule: a block of even rows streams tiles, one whose rows of 400 and 20 edges lie in runs of 300 does not.  The
+    two layouts of the restaged operand are told apart within one product."""
+    from super_gnn_amd import supergnn_ops as ops
+    M, K, F = 24000, 40000, 602
+    rng = np.random.default_rng(6)
+    deg = np.full(M, 210)
+    deg[M // 2:] = np.where(np.arange(M // 2) // 300 % 2 == 0, 400, 20)
+    rowptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int64)
+    col = rng.integers(0, K, size=rowptr[-1])
+    col = col[np.lexsort((col, np.repeat(np.arange(M), deg)))]
+    rp, cl, x = torch.from_numpy(rowptr).to(DEV), torch.from_numpy(col).to(DEV), torch.randn(K, F, generator=torch.Generator().manual_seed(1))
+    with pytest.MonkeyPatch.context() as m:
+        m.setenv("SGNN_SPMM_PART_EDGES", str(int(rowptr[M // 2])))
+        plan = ops.SpmmPlan(rp, cl, K)
+    halves = [ops.SpmmPlan(rp[a:a + M // 2 + 1] - rp[a], cl[rp[a]:rp[a + M // 2]].clone(), K) for a in (0, M // 2)]
+    assert [h.tiles(F)[0] > 0 for h in halves] == [True, False] and all(h.schedule(F)["band"] == 1 for h in halves)
+    xd, out = x.to(DEV), torch.empty(M, F, device=DEV)
+    for value in (None, torch.rand(col.size, generator=torch.Generator().manual_seed(2))):
+        for _ in range(3):
+            out.fill_(7.0)
+            plan.run(None if value is None else value.to(DEV), xd, out, accumulate=False)
+            for r0 in (5000, 17900):
+                lo, hi = rowptr[r0], rowptr[r0 + 100]
+                want = np.zeros((100, F), np.float32)
+                orc.spmm_accumulate(rowptr[r0:r0 + 101] - lo, col[lo:hi], np.ones(hi - lo, np.float32) if value is None else value[lo:hi].numpy(),
+                                    x.numpy(), want)
+                equal = np.array_equal(out[r0:r0 + 100].cpu().numpy(), want)
+                assert equal, r0
