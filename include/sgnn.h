@@ -89,7 +89,7 @@ int sgnn_spmm_plan_stack(sgnn_spmm_plan *const *parts, int n_parts, sgnn_stream_
 int sgnn_spmm_plan_info(const sgnn_spmm_plan *plan, int64_t info[10]);
 
 /* Which schedule sgnn_spmm_csr_f32 takes for a dense operand of F contiguous, 16-byte aligned fp32 columns:
- * info[0] = 1 for the band schedule, 0 for the row-class schedule above.  The band schedule is for
+ * info[0] = 1 for the band schedule or the tile schedule (sgnn_spmm_plan_tiles), 0 for the row-class schedule above.  The band schedule is for
  * dense-degree matrices whose dense operand does not fit the L2 caches (e.g. 233 k nodes with ~490 edges
  * per row at F = 602): the column space is cut into bands of info[1] columns (info[2] bands), the product
  * is one launch per band accumulating onto out, and inside a launch the eight XCDs split the feature axis
@@ -168,7 +168,9 @@ int sgnn_spmm_csr_f32(sgnn_spmm_plan *plan, const float *val, const float *x, fl
  *     bands into different chunks).  The simple way to guarantee that is one sgnn_spmm_csr_f32 call with the same
  *     F and the same kind of weights beforehand.  Otherwise the row-class kernels run: same result on rows of up
  *     to 128 edges, bit for bit; longer rows are summed per piece instead of in one chain (within the fp32
- *     tolerance, not the same bits).  The tile schedule in the same way: streams for any number of rows will do;
+ *     tolerance, not the same bits).  The tile schedule in the same way: streams for any number of rows will do.
+ *     A product that takes tiles where the row classes would run otherwise (a matrix without long rows) runs the row classes here,
+ *     under stream capture, and while another product of the same plan is in flight on another stream: the same bits;
  *   - the scratch address is looked up when a plan is created, so the call itself performs no lazy symbol
  *     lookup, and it records no profiling events (sgnn_profile_enable does not see its kernels). */
 int sgnn_spmm_csr_f32_noalloc(sgnn_spmm_plan *plan, const float *val, const float *x, float *out,

@@ -926,8 +926,9 @@ __global__ __launch_bounds__(kBlock) void spmm_long_final_kernel(
 
 // The short rows, and with them what else may run beside them: the long rows' final sum where its partials are kept
 // (keep_partials) and the rows without edges.  Both are short and wait for memory, and a launch of their own costs the
-// ramp-up and the tail of one (200 k power-law nodes, F = 100, transposed 192 -> 173 us; fused 1 M rows 580 -> 564).  Workgroups in this order: final sum (the longest chains), short rows, empty rows; the final
-// sum's number is a multiple of eight, so that the short rows' workgroups stay on their XCDs.
+// ramp-up and the tail of one (200 k power-law nodes, F = 100, transposed 192 -> 173 us; fused 1 M rows 580 -> 564).  Workgroups in
+// this order: final sum (the longest chains), short rows, empty rows; the final sum's number is a multiple of eight, so that
+// the short rows' workgroups stay on their XCDs.
 struct RowTails {
     const int32_t *long_rows, *long_pbeg;
     const float *partial;
@@ -1455,7 +1456,7 @@ struct sgnn_spmm_plan {
     uint64_t bind_gen = 1;          // bumped by every sgnn_spmm_plan_bind_values
     std::vector<BandSchedule *> bands;
     std::vector<TileSchedule *> tiles;
-    TileAlone tile_alone;
+    mutable TileAlone tile_alone;
     std::vector<float> tile_spread; // per number of rows a wave (tile_candidate): see tile_measure
     std::atomic<bool> tile_too_many{false};   // more batches than the streams can number
     float *band_xs = nullptr;       // the dense operand restaged slice by slice (see band_restage_kernel), grown on demand
@@ -2446,6 +2447,11 @@ constexpr double kTileSpread = 1.25;   // see tile_measure
 constexpr int kMaxTileSchedules = 3;   // row counts a plan keeps streams for (12 bytes per slot each)
 constexpr double kTileBuildGain = 0.9; // share of the held streams' estimate below which another row count gets its own
 
+// The constants below are cautious.  Over 80 products (4 k ... 100 k nodes, 40 ... 400 edges a row, F = 128 ... 1024) the rule takes tiles
+// in 34, at 0.43 ... 0.87 of the time of the fastest other schedule.  Of the rest tiles would have been faster in 11 of 14 with
+// long rows (down to 0.52), which stay with the row classes for their rounding, and in 9 of 32 without (down to 0.66), whose
+// estimates lie at 1.0 ... 1.5 of the other schedules'.
+//
 // Estimated time of a product, in clocks of the chip: the rounds of workgroups times the tiles of a sweep times the clocks
 // of a tile, which go with its edges (240 edges of 104 columns 1480 clocks, 640 2950, 4800 20800) down to what the stream
 // of tiles takes.
@@ -2692,6 +2698,7 @@ extern "C" int sgnn_spmm_plan_tiles(const sgnn_spmm_plan *p, int64_t F, int64_t 
     SGNN_REQUIRE(F > 0 && F < (1 << 24), "feature width F=%lld out of range", (long long)F);
     if (!p->parts.empty()) p = p->parts[0];
     info[0] = tile_rows(p, F);
+    std::lock_guard<std::mutex> lock(p->tile_alone.mu);
     info[1] = (int64_t)(p->tiles.size() + p->tile_alone.tiles.size());
     return SGNN_OK;
 }

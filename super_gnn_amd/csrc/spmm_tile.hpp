@@ -7,19 +7,21 @@
 //   * waves 0 .. 14 (the consumers) walk their edges in (tile, row, column) order: per edge one ds_read of the 256-byte
 //     operand row and one fma into the row's register, chosen by VGPR-index mode, so there is no branch per row.
 // The edges are a stream of batches of 16: 16 words (bits 0..7 row register, 8..17 ring column, in the first word 18..30
-// tiles entered before the batch, 31 end) and 16 values, read through the scalar cache two batches ahead; a vector load
-// touches the line 4 KB ahead so that the scalar loads hit the L2.  A batch holds edges of two neighbouring tiles at most.
+// tiles entered before the batch, 31 end) and 16 values, read through the scalar cache: the words of batch i + 2 and the values of
+// i + 1 are on their way during the fmas of batch i and waited for behind them, with the operand rows of batch i + 1.  A vector
+// load touches the line 4 KB ahead so that the scalar loads hit the L2.  A batch holds edges of two neighbouring tiles at most.
 // Two waits, both on LDS words: a consumer enters tile m once the producer has filled it, the producer overwrites the slot
 // of tile t - 6 once every consumer has entered t - 4 (then all are done with t - 6).  The slowest consumer never waits for
 // another consumer and the producer publishes what has landed before it waits, so every wait ends.
 // Rows are summed in CSR order with one fma per edge from the old out value: bit-identical to the band schedule and to the
 // reference on column-sorted rows.
 //
-// Bound: instruction issue (per edge an address, a ds_read, an index and an fma: 4.3 clocks per edge and CU where a tile
-// holds 640 edges and more; 16 x 64-lane v_fma with a scalar operand take 4.3 clocks each on a SIMD, ds_read_b32 2.1 per CU).
-// With fewer edges per tile the stream of 26 KB tiles takes over: 1480 clocks per tile at 240 edges, 1240 at 80.  A gather of
-// the band schedule takes 7.5 clocks per edge of 64 floats.  Two floats per lane would need a third less issue per float but
-// half the rows per workgroup, that is twice the stream.
+// Bound: waiting.  Per edge an address, a ds_read, an index and an fma: two vector instructions with a scalar operand (4.3 clocks
+// each on one of four SIMDs) and 2.1 clocks of the CU's LDS, so about 2.2 clocks per edge and CU of issue, and it takes 4.3 where
+// a tile holds 640 edges and more: every batch of 16 ends in one wait for all its loads, and four waves per SIMD do not cover it
+// (114 M edges, F = 602: waves wait 0.50 of their cycles and 0.20 more for issue).  With fewer edges per tile the stream of 26 KB
+// tiles takes over: 1480 clocks per tile at 240 edges, 1240 at 80.  A gather of the band schedule takes 7.5 clocks per edge of 64
+// floats.  Two floats per lane would need a third less issue per float but half the rows per workgroup, that is twice the stream.
 #pragma once
 
 namespace sgnn {

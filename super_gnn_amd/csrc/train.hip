@@ -3,8 +3,8 @@
 //
 // Bound by memory: each direction reads its row operands once and writes once.  A group of G lanes owns a row of up to
 // 4 * G * NV floats and holds it in registers between the reductions over the row; two rows per group are in flight.
-// 150 k rows of 256 floats: forward 0.21 ms as torch's layer_norm and relu (0.17 of it the norm) -> 0.06 ms; backward 0.44 ms as
-// threshold, two layer_norm gradients and the mask's product -> 0.10 ms (5.2 TB/s).
+// 150 k rows of 256 floats: forward 215 us as torch's layer_norm and relu -> 52; backward 440 us as threshold, two layer_norm
+// gradients and the mask's product -> 85 (5.9 TB/s).
 #include <algorithm>
 #include <type_traits>
 
@@ -190,8 +190,8 @@ __global__ __launch_bounds__(kNormBlock) void norm_relu_backward_kernel(
     }
 }
 
-// Sums over the rows of each column, per workgroup: partial[block][C].  Bound by memory (150 k x 256: 55 us as torch's sum,
-// whose 64 workgroups leave most of the chip idle -> 27 us with the sum of the partials).
+// Sums over the rows of each column, per workgroup: partial[block][C].  Bound by memory (150 k x 256: 65 us as torch's sum,
+// whose 64 workgroups leave most of the chip idle -> 30 us with the sum of the partials).
 template <int G, int NV>
 __global__ __launch_bounds__(kNormBlock) void column_sum_kernel(const float *__restrict__ x, float *__restrict__ partial, int64_t n, int C) {
     constexpr int kGroups = kNormBlock / G, kRows = 4;
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(256) void partial_sum_kernel(const float *__restric
 }
 
 // w[i, j] += sum over rows r of g[r, i] * a[r, j], for the few rows a batched product over equal slabs leaves over: the library gives
-// the whole product to one workgroup (12 ... 25 us for 48 rows of 47 ... 256 columns, six times a training step of three layers).
+// the whole product to one workgroup (18 ... 21 us for 48 rows of 47 ... 256 columns, here 9 ... 11; six times a training step of three layers).
 // 64 x 64 outputs per workgroup, 4 x 4 per thread, 64 rows of both operands in LDS at a time: the latency of one round of loads.
 constexpr int kRestRows = 64;
 __global__ __launch_bounds__(256) void rest_product_kernel(const float *__restrict__ g, const float *__restrict__ a, float *__restrict__ w,

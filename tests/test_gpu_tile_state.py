@@ -246,7 +246,8 @@ def test_products_of_one_matrix_on_several_streams():
     assert c.plan.tiles(c.F)[1] == 1
 
 
-def test_threads_and_captures_beside_each_other():
+@pytest.mark.parametrize("default_stream", [False, True])
+def test_threads_and_captures_beside_each_other(default_stream):
     """Another thread's products, the first of a width among them, neither disturb a capture nor wait for one; a captured
     product that is the plan's first builds nothing."""
     import threading
@@ -259,7 +260,7 @@ def test_threads_and_captures_beside_each_other():
 
     def work(n):
         try:
-            with torch.cuda.stream(torch.cuda.Stream()):
+            with torch.cuda.stream(torch.cuda.default_stream() if default_stream else torch.cuda.Stream()):
                 for _ in range(n):
                     for x, out in sets.values():
                         c.plan.run(c.value, x, out, accumulate=False, bind=False)
