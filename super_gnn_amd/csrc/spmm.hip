@@ -1458,7 +1458,7 @@ struct sgnn_spmm_plan {
     std::vector<TileSchedule *> tiles;
     mutable TileAlone tile_alone;
     std::vector<float> tile_spread; // per number of rows a wave (tile_candidate): see tile_measure
-    std::atomic<bool> tile_too_many{false};   // more batches than the streams can number
+    std::atomic<uint32_t> tile_refused{0};   // bit i: candidate i has more batches than the streams can number
     float *band_xs = nullptr;       // the dense operand restaged slice by slice (see band_restage_kernel), grown on demand
     size_t band_xs_floats = 0;
     bool band_xs_captured = false, partial_captured = false, val_long_captured = false;   // a captured product names the buffer
@@ -2291,7 +2291,11 @@ static int is_capturing(hipStream_t st, bool *yes) {
 // its graph is replayed, so the plan then keeps it to its own end.
 static int give_up(sgnn_spmm_plan *p, float **buf, bool *captured) {
     if (*captured) {
-        p->kept.push_back(*buf);
+        try {
+            p->kept.push_back(*buf);
+        } catch (const std::bad_alloc &) {
+            return fail(SGNN_ERR_HIP, "out of host memory");
+        }
     } else if (*buf != nullptr) {
         SGNN_HIP_CHECK(hipDeviceSynchronize());
         (void)hipFree(*buf);
@@ -2474,7 +2478,7 @@ static int tile_rows(const sgnn_spmm_plan *p, int64_t F) {
     const int mode = env_int("SGNN_SPMM_BAND", -1);
     if (mode == 0 || mode == 1) return 0;
     // (below a density of 1 / 2000 the stream of the operand alone takes longer than the other schedules)
-    if (p->tile_too_many || (mode < 2 && (double)p->nnz * 2000.0 < (double)p->M * (double)p->K)) return 0;
+    if (mode < 2 && (double)p->nnz * 2000.0 < (double)p->M * (double)p->K) return 0;
     // One chain of fmas per row: where the row classes would take the product, which add up long rows in parts, only if there
     // are none (a chain of 370 edges is off by 3.0e-7, the parts by 1.3e-7).
     // (Row blocks keep their state in the whole plan, so those that the row classes would take stay there too.)
@@ -2484,7 +2488,7 @@ static int tile_rows(const sgnn_spmm_plan *p, int64_t F) {
     int best = 0;
     for (int i = 0; i < kTileCandidates; ++i) {
         const int r = tile_candidate(i);
-        if (mode < 2 && p->tile_spread[(size_t)i] > kTileSpread) continue;
+        if ((p->tile_refused >> i & 1u) != 0 || (mode < 2 && p->tile_spread[(size_t)i] > kTileSpread)) continue;
         if (best == 0 || tile_clocks(p, F, r) < 0.97 * tile_clocks(p, F, best)) best = r;
     }
     return best > 0 && tile_clocks(p, F, best) < others ? best : 0;
@@ -2509,7 +2513,7 @@ static int tile_build(sgnn_spmm_plan *p, int rows, hipStream_t st, TileSchedule 
         ts->batches += h[i];
     }
     if (ts->batches > (INT32_MAX >> 5)) {
-        p->tile_too_many = true;
+        p->tile_refused |= 1u << ((kTileRows - rows) / 3);
         return SGNN_OK;
     }
     SGNN_BAND_ALLOC(&ts->stream, (size_t)ts->batches * (8 * kTileBatch) + kTileSlack);
@@ -2620,7 +2624,10 @@ static int spmm_run_tile(sgnn_spmm_plan *p, int rows, const float *val, const De
     const bool restaged = root->xs_serial == root->call_serial && root->xs_F == (int)F && root->xs_slices == -n_slices;
     rc = tile_launch(p, ts, root->band_xs, !restaged, val, val != nullptr && values_due(p, ts, val, p->long_edges > 0), dense, out, F, ldo,
                      accumulate, row_div, st, prof);
-    if (rc != SGNN_OK) return rc;
+    if (rc != SGNN_OK) {
+        ts->val_gen = 0;   // (the fill may not have been launched)
+        return rc;
+    }
     root->xs_serial = root->call_serial;
     root->xs_F = (int)F; root->xs_slice_pad = 64; root->xs_slices = -n_slices;
     *done = true;
